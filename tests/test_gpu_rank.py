@@ -91,3 +91,18 @@ def test_isdf_check_rank_deficient(ctx):
     out = ctx.isdf(a, idx, n, cg, check_rank=True)
     assert out["cct_rank"] == IO.rank(c) <= 21
     assert out["status"] in (L.THC_ERR_NOT_POSDEF, L.THC_WARN_RANK_DEFICIENT)
+
+
+@pytest.mark.parametrize("k", [2, 127, 128, 129, 255, 257, 512, 513, 1025, 2049])
+def test_rank_chunk_edges(ctx, k):
+    """Sizes either side of the reduction's 128-column chunks, its 256 workgroups and its row-width variants
+    (512, 1024, 2048 columns): the exact rank of B B^T, and the largest singular value to k eps (a Householder
+    reduction's backward error is below k eps of it)."""
+    r = max(1, k - k // 5)
+    b = np.random.default_rng(k).standard_normal((k, r))
+    c = b @ b.T
+    rank, smax, _ = ctx.cct_rank(c)
+    if k >= 40:
+        assert rank == r
+    want = np.linalg.eigvalsh(c)[-1]
+    assert abs(smax - want) <= k * 2.3e-16 * want + 4e-16 * want

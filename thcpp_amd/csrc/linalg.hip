@@ -413,80 +413,143 @@ inline int grid_for(long count) { return (int)std::min<long>(4096, std::max<long
 // launch), takes reflection j from it (v = x - alpha e1, beta = 1/(alpha
 // (alpha - x0)), alpha = -sign(x0) |x|), and multiplies its updated rows by v
 // (p = beta A22 v).  The diagonal d and off-diagonal e of T go to d, e.
+//
+// A launch moves the trailing matrix once through the CUs (33 MB read and
+// written at k = 2048) and is otherwise a chain of two block sums.  Each wave
+// takes a whole row in registers, and its loads are issued before the chain,
+// so the chain's latency hides the matrix read; row i belongs to workgroup
+// i mod TD_WG in every launch, so it stays in the L2 of one XCD.  Measured at
+// k = 2048: 15.9 ms for the whole rank, 7.7 us per column; with one workgroup
+// of four waves per row at a time on 128 CUs, loading after the chain, it was
+// 54.2 ms (45-51 us per column at full width, 1.4 TB/s).
 constexpr int TD_MAXK = 4096;
+constexpr int TD_WG = 256, TD_W = 8;  // workgroups (one per CU), waves of each
 
 __device__ inline double td_block_sum(double v, double* red) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __syncthreads();
   if (lane == 0) red[w] = v;
   __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
+  double s = 0.0;
+#pragma unroll
+  for (int q = 0; q < TD_W; ++q) s += red[q];
+  return s;
 }
 
-__global__ __launch_bounds__(256) void tridiag_step(double* __restrict__ W, int k, int j,
-                                                    const double* __restrict__ vp, const double* __restrict__ pp,
-                                                    const double* __restrict__ bp, double* __restrict__ vn,
-                                                    double* __restrict__ pn, double* __restrict__ bn,
-                                                    double* __restrict__ d, double* __restrict__ e) {
-  __shared__ double sv[TD_MAXK], sw[TD_MAXK], sx[TD_MAXK];
-  __shared__ double red[4];
-  const int t = threadIdx.x;
+// CH: 128-column chunks of the widest row (k <= 128 CH); the rows of W are ld
+// doubles apart (a multiple of 128, zero beyond k), vp .. pn hold ld entries.
+template <int CH>
+__global__ __launch_bounds__(64 * TD_W) void tridiag_step(double* __restrict__ W, int ld, int k, int j,
+                                                          const double* __restrict__ vp,
+                                                          const double* __restrict__ pp,
+                                                          const double* __restrict__ bp, double* __restrict__ vn,
+                                                          double* __restrict__ pn, double* __restrict__ bn,
+                                                          double* __restrict__ d, double* __restrict__ e) {
+  constexpr int NT = 64 * TD_W, PT = CH * 128 / NT > 0 ? CH * 128 / NT : 1;
+  __shared__ __attribute__((aligned(16))) double sv[CH * 128], sw[CH * 128], sx[CH * 128];
+  __shared__ double red[2][TD_W];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const bool upd = j > 0;
-  if (upd) {
-    double g = 0.0;
-    for (int c = j + t; c < k; c += 256) g += pp[c] * vp[c];
-    g = td_block_sum(g, red);
-    const double hb = 0.5 * bp[0] * g;
-    for (int c = j + t; c < k; c += 256) {
-      sv[c] = vp[c];
-      sw[c] = pp[c] - hb * vp[c];
-    }
-    __syncthreads();
+  const int cb = j & ~127;  // the chunks from column j on
+  const int nch = (ld - cb) >> 7, ncol = ld - cb;
+  // first row > j of this wave: rows i = blockIdx + TD_WG (wave + TD_W q)
+  int i = blockIdx.x + TD_WG * wave;
+  if (i <= j) i += (j - i + TD_WG * TD_W) / (TD_WG * TD_W) * (TD_WG * TD_W);
+  if (blockIdx.x != 0 && (int)blockIdx.x + (k - 1 - (int)blockIdx.x) / TD_WG * TD_WG <= j) return;  // no row left
+  double2 x[CH];
+  double2* row = reinterpret_cast<double2*>(W + (long)i * ld + cb) + lane;
+  if (i < k) {
+#pragma unroll
+    for (int q = 0; q < CH; ++q)
+      if (q < nch) x[q] = row[64 * q];
   }
-  for (int c = j + t; c < k; c += 256) {
-    double x = W[(long)j * k + c];
-    if (upd) x -= sv[j] * sw[c] + sw[j] * sv[c];
-    sx[c] = x;
+  // w of reflection j - 1 and row j, columns c = cb + t + NT q
+  double v[PT], w[PT], r[PT];
+  double g = 0.0;
+#pragma unroll
+  for (int q = 0; q < PT; ++q) {
+    const int c = t + NT * q;
+    const bool ok = c < ncol && cb + c >= j;
+    r[q] = ok ? W[(long)j * ld + cb + c] : 0.0;
+    v[q] = ok && upd ? vp[cb + c] : 0.0;
+    w[q] = ok && upd ? pp[cb + c] : 0.0;
+    g += w[q] * v[q];
   }
-  __syncthreads();
+  const double vj = upd ? vp[j] : 0.0, pj = upd ? pp[j] : 0.0, hb = upd ? 0.5 * bp[0] : 0.0;
+  g = td_block_sum(g, red[0]) * hb;
+  const double wj = pj - g * vj;
   double nrm2 = 0.0;
-  for (int c = j + 1 + t; c < k; c += 256) nrm2 += sx[c] * sx[c];
-  nrm2 = td_block_sum(nrm2, red);
+#pragma unroll
+  for (int q = 0; q < PT; ++q) {
+    w[q] -= g * v[q];
+    r[q] -= vj * w[q] + wj * v[q];
+    if (cb + t + NT * q > j) nrm2 += r[q] * r[q];
+  }
+  // columns up to j keep v = w = x = 0: they are done
+#pragma unroll
+  for (int q = 0; q < PT; ++q) {
+    const int c = t + NT * q;
+    if (c < ncol) {
+      const bool live = cb + c > j;
+      sv[c] = live ? v[q] : 0.0;
+      sw[c] = live ? w[q] : 0.0;
+      sx[c] = live ? r[q] : 0.0;
+      if (blockIdx.x == 0 && cb + c == j) d[j] = r[q];
+    }
+  }
+  nrm2 = td_block_sum(nrm2, red[1]);
   double alpha = 0.0, beta = 0.0;
   if (j + 1 < k && nrm2 > 0.0) {
-    const double x0 = sx[j + 1];
+    const double x0 = sx[j + 1 - cb];
     alpha = x0 >= 0.0 ? -sqrt(nrm2) : sqrt(nrm2);
     beta = 1.0 / (alpha * (alpha - x0));
   }
   __syncthreads();
-  if (t == 0 && j + 1 < k) sx[j + 1] -= alpha;  // v = x - alpha e1
+  if (t == 0 && j + 1 < k) sx[j + 1 - cb] -= alpha;  // v = x - alpha e1
   __syncthreads();
   if (blockIdx.x == 0) {
     if (t == 0) {
-      d[j] = sx[j];
       if (j + 1 < k) e[j] = alpha;
       bn[0] = beta;
     }
-    for (int c = j + 1 + t; c < k; c += 256) vn[c] = sx[c];
+    for (int c = t; c < ncol; c += NT) vn[cb + c] = sx[c];
   }
-  for (int i = j + 1 + blockIdx.x; i < k; i += gridDim.x) {
+  const double2* v2 = reinterpret_cast<const double2*>(sv) + lane;
+  const double2* w2 = reinterpret_cast<const double2*>(sw) + lane;
+  const double2* x2 = reinterpret_cast<const double2*>(sx) + lane;
+  while (i < k) {
+    const double vi = sv[i - cb], wi = sw[i - cb];
     double acc = 0.0;
-    double* row = W + (long)i * k;
-    for (int c = j + 1 + t; c < k; c += 256) {
-      double x = row[c];
-      if (upd) x -= sv[i] * sw[c] + sw[i] * sv[c];
-      row[c] = x;
-      acc += x * sx[c];
+#pragma unroll
+    for (int q = 0; q < CH; ++q)
+      if (q < nch) {
+        const double2 a = w2[64 * q], b = v2[64 * q], c = x2[64 * q];
+        x[q].x -= vi * a.x + wi * b.x;
+        x[q].y -= vi * a.y + wi * b.y;
+        if (upd) row[64 * q] = x[q];
+        acc += x[q].x * c.x + x[q].y * c.y;
+      }
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+    if (lane == 0) pn[i] = beta * acc;
+    i += TD_WG * TD_W;
+    if (i < k) {
+      row = reinterpret_cast<double2*>(W + (long)i * ld + cb) + lane;
+#pragma unroll
+      for (int q = 0; q < CH; ++q)
+        if (q < nch) x[q] = row[64 * q];
     }
-    acc = td_block_sum(acc, red);
-    if (t == 0) pn[i] = beta * acc;
   }
 }
 
-__global__ __launch_bounds__(256) void copy_square(const double* a, long lda, int k, double* w) {
-  const long total = (long)k * k;
-  for (long q = blockIdx.x * 256L + threadIdx.x; q < total; q += 256L * gridDim.x) w[q] = a[(q / k) * lda + q % k];
+// a (k x k) into rows of ld doubles, zero beyond column k; the step vectors zeroed
+__global__ __launch_bounds__(256) void copy_square(const double* a, long lda, int k, double* w, int ld, double* vec,
+                                                   int nvec) {
+  const long total = (long)k * ld;
+  for (long q = blockIdx.x * 256L + threadIdx.x; q < total; q += 256L * gridDim.x) {
+    const long r = q / ld, c = q - r * ld;
+    w[q] = c < k ? a[r * lda + c] : 0.0;
+  }
+  for (long q = blockIdx.x * 256L + threadIdx.x; q < nvec; q += 256L * gridDim.x) vec[q] = 0.0;
 }
 
 // number of eigenvalues of the tridiagonal (d, e) below x (Sturm count of the
@@ -604,8 +667,10 @@ int spd_inverse_from_chol(const double* l, int k, long lda, double* ainv, void* 
   return THC_OK;
 }
 
+inline int td_ld(int k) { return (k + 127) / 128 * 128; }
+
 size_t tridiag_work_bytes(int k) {
-  return align_up(sizeof(double) * (size_t)k * k, 256) + 6 * align_up(sizeof(double) * (size_t)k, 256) +
+  return align_up(sizeof(double) * (size_t)k * td_ld(k), 256) + 6 * align_up(sizeof(double) * (size_t)td_ld(k), 256) +
          2 * align_up(sizeof(double) * 4, 256) + 256;
 }
 
@@ -618,19 +683,27 @@ int sym_tridiag(const double* a, int k, long lda, double* d_host, double* e_host
     w += align_up(sizeof(double) * count, 256);
     return p;
   };
-  double* W = take((size_t)k * k);
-  double* vb[2] = {take(k), take(k)};
-  double* pb[2] = {take(k), take(k)};
+  const int ld = td_ld(k);
+  double* W = take((size_t)k * ld);
+  double* vec = take((size_t)4 * ld);  // v and p of the two latest reflections
+  double* vb[2] = {vec, vec + ld};
+  double* pb[2] = {vec + 2 * ld, vec + 3 * ld};
   double* bb[2] = {take(4), take(4)};
-  double* dd = take(k);
-  double* ee = take(k);
-  hipLaunchKernelGGL(copy_square, dim3(grid_for((long)k * k)), dim3(256), 0, s, a, lda, k, W);
+  double* dd = take(ld);
+  double* ee = take(ld);
+  hipLaunchKernelGGL(copy_square, dim3(grid_for((long)k * ld)), dim3(256), 0, s, a, lda, k, W, ld, vec, 4 * ld);
   THC_HIP(hipGetLastError());
   for (int j = 0; j < k; ++j) {
     const int cur = j & 1, prev = cur ^ 1;
-    const int rows = std::max(1, std::min(128, k - j - 1));
-    hipLaunchKernelGGL(tridiag_step, dim3(rows), dim3(256), 0, s, W, k, j, vb[prev], pb[prev], bb[prev], vb[cur],
-                       pb[cur], bb[cur], dd, ee);
+    const int left = (ld - (j & ~127)) >> 7;  // chunks this step touches: the registers and LDS of the step follow
+    auto step = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(std::min(TD_WG, k)), dim3(64 * TD_W), 0, s, W, ld, k, j, vb[prev], pb[prev],
+                         bb[prev], vb[cur], pb[cur], bb[cur], dd, ee);
+    };
+    if (left <= 4) step(tridiag_step<4>);
+    else if (left <= 8) step(tridiag_step<8>);
+    else if (left <= 16) step(tridiag_step<16>);
+    else step(tridiag_step<32>);
     THC_HIP(hipGetLastError());
   }
   THC_HIP(hipMemcpyAsync(d_host, dd, sizeof(double) * k, hipMemcpyDeviceToHost, s));
