@@ -84,3 +84,39 @@ def test_qrcp_complex_real_orbitals_match_real_path(ctx):
         assert st_r == L.THC_OK and st_c == L.THC_OK
         np.testing.assert_array_equal(idx_c.cpu().numpy(), idx_r.cpu().numpy())
         np.testing.assert_allclose(rd_c, rd_r, rtol=1e-12)
+
+
+@pytest.mark.parametrize("n,m,mo,k", [(40, 6, 0, 21), (255, 9, 0, 40), (257, 5, 3, 12), (1030, 11, 0, 66),
+                                      (5000, 30, 0, 300), (9001, 13, 7, 70)])
+def test_qrcp_rounds_edges(ctx, n, m, mo, k):
+    """Rounds of shared pivots at the edges: fewer points than candidates, k up to the rank M (M + 1) / 2, point
+    counts either side of a workgroup's 256, orbital counts that are no multiple of 4, runs beyond one 16-pivot
+    tile.  Residuals as separated as those of test_qrcp_vs_oracle, hence its tolerance."""
+    print("qrcp rounds n=%d m=%d m_occ=%d k=%d" % (n, m, mo, k), flush=True)
+    rng = np.random.default_rng(n + k)
+    a = _orbitals(n, m, n + k) * rng.uniform(0.2, 1.0, (n, 1))
+    occ = np.ascontiguousarray(a[:, :mo]) if mo else None
+    st, idx, rd = ctx.qrcp_points(a, k, occ)
+    assert st == L.THC_OK
+    ref_idx, ref_rd, _ = QO.qrcp_points(a, k, occ)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ref_idx)
+    np.testing.assert_allclose(rd, ref_rd, rtol=1e-7)
+
+
+@pytest.mark.parametrize("repeat", [2, 300])
+def test_qrcp_equal_points(ctx, repeat):
+    """Points with the same orbital values have bit-equal residuals: the first one is the pivot (more of them than
+    candidates fit in a round, with 300), and its copies never are."""
+    a = _orbitals(40, 10, 11) * np.random.default_rng(4).uniform(0.3, 1.0, (40, 1))
+    ref_idx, ref_rd, _ = QO.qrcp_points(a, 30)
+    st, idx, rd = ctx.qrcp_points(np.repeat(a, repeat, axis=0), 30)
+    assert st == L.THC_OK
+    np.testing.assert_array_equal(idx.cpu().numpy(), repeat * ref_idx)
+    np.testing.assert_allclose(rd, ref_rd, rtol=1e-7)
+
+
+def test_qrcp_no_finite_residual(ctx):
+    """All-zero and NaN orbitals have no pivot."""
+    for fill in (0.0, np.nan):
+        st, _, _ = ctx.qrcp_points(np.full((700, 4), fill), 3)
+        assert st == L.THC_ERR_NOT_POSDEF

@@ -10,15 +10,27 @@
 // i.e. the Gram matrix G = P o Pocc (P o P without half rotation).  Pivoted
 // Cholesky of G picks, step by step, the column of largest residual norm and
 // projects it out -- the same pivots as QR with column pivoting of ZT in exact
-// arithmetic, with the pivot's residual norm equal to |R_jj|.  Each step is
-// one kernel over the N grid points:
-//   p      = argmax residual d (first index on ties), from the previous step's
-//            per-block maxima;
+// arithmetic, with the pivot's residual norm equal to |R_jj|.  A step is
+//   p      = argmax residual d (first index on ties);
 //   g_a    = G[a][p] from two M-length dot products with the pivot's row;
 //   l_a    = (g_a - sum_{q<j} L[q][a] L[q][p]) / sqrt(d_p);
-//   d_a   -= l_a^2  (the pivot itself is retired);
-//   new per-block maxima of d.
-// Cost per step: one read of phi (N M) and of the j previous columns of L.
+//   d_a   -= l_a^2  (the pivot itself is retired),
+// and reads all j earlier columns of L, N j doubles, for one column.  Residuals
+// only ever fall, so several steps can share that read: take as candidates all
+// points with residual above some bound (at most QC of them).  As long as the
+// largest candidate residual stays above the bound, no other point can be the
+// next pivot, and the steps run on the candidates' own QC x QC block of the
+// Schur complement.  A round (real G) is
+//   qr_pick    candidates: all points in the top bins of a histogram of d;
+//   qr_gather  their columns of L, qr_gram their block G - L L^T (MFMA);
+//   qr_run     the pivot steps on that block, up to QR_MAX of them;
+//   qr_apply   the chosen columns for all N points at once: one pass over L
+//              (MFMA), a triangular solve, the new d, its histogram and maxima.
+// On a 40^3 grid, M = 64, K = 512: 27 rounds of 19 pivots on average, 2.8 ms
+// (qr_apply 44 us, qr_run 28 us a round); one kernel per pivot, each reading
+// all earlier columns, took 17.7 ms (8 us + 0.085 us per earlier column).
+// QC = 256 candidates: 128 give 37 rounds, 512 give 21 with a four times
+// larger block.
 //
 // Complex orbitals (ZT[(i k), a] = conj(phi_i(r_a)) phi_k(r_a), src/qrcp.cpp:
 // 33-48): with Q[a][b] = sum_k conj(phi_k(a)) phi_k(b) the Gram matrix is
@@ -29,6 +41,7 @@
 // those of QR with column pivoting of the complex ZT.
 #include <algorithm>
 #include <cfloat>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -108,17 +121,545 @@ __global__ __launch_bounds__(QB) void qr_init(const double* __restrict__ phi, co
   block_argmax(v, vi, pv, pi);
 }
 
+// ---- rounds of pivots for a real G --------------------------------------------
+
+constexpr int QC = 256;       // candidates of a round (threads of qr_run)
+constexpr int QR_MAX = 32;    // pivots of a round: two MFMA tiles of columns
+constexpr int QBINS = 1536;   // bins of the residual histogram: 128 an octave, 12 octaves below the reference
+constexpr int QBIN_SHIFT = 13;  // a residual's bin: the exponent and 7 mantissa bits of its high word
+
+enum { G_SQUARE = 0, G_PRODUCT = 1, G_MODULUS = 2 };  // G = P^2, P Pocc, |P|^2 (complex)
+
+struct QrState {
+  int j, fail, done;  // pivots chosen, step that found none (1-based), run ended: read back together
+  int base, r;      // pivots chosen before this round, chosen in it
+  int ncand, cut;   // candidates, the lowest bin (counted downwards) that is among them
+  int refkey;       // bin key no residual is above
+  int slot[QR_MAX];  // candidate slots of the round's pivots
+  int piv[QR_MAX];
+  double rs[QR_MAX];            // 1 / sqrt(residual) of the pivots
+  double tri[QR_MAX][QR_MAX];   // tri[s][t] = l_s at pivot t > s
+};
+
+__device__ inline int qr_key(double v) { return (int)(__double_as_longlong(v) >> 32) >> QBIN_SHIFT; }
+// bin of a positive residual, counted downwards from the reference; QBINS and
+// above are out of range
+__device__ inline int qr_bin(double v, int refkey) { return max(0, refkey - qr_key(v)); }
+
+// first maximum over nparts per-block maxima, to all threads of the block
+__device__ inline void qr_top(const double* pv, const int* pi, int nparts, double& v, int& vi, double* sv, int* si) {
+  v = -DBL_MAX;
+  vi = INT_MAX;
+  for (int q = threadIdx.x; q < nparts; q += blockDim.x)
+    if (wins(pv[q], pi[q], v, vi)) { v = pv[q]; vi = pi[q]; }
+  for (int o = 32; o > 0; o >>= 1) {
+    const double ov = __shfl_xor(v, o);
+    const int oi = __shfl_xor(vi, o);
+    if (wins(ov, oi, v, vi)) { v = ov; vi = oi; }
+  }
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __syncthreads();
+  if (lane == 0) { sv[w] = v; si[w] = vi; }
+  __syncthreads();
+  v = sv[0];
+  vi = si[0];
+  for (int q = 1; q < (int)(blockDim.x >> 6); ++q)
+    if (wins(sv[q], si[q], v, vi)) { v = sv[q]; vi = si[q]; }
+}
+
+// Start: the reference residual, an empty histogram.
+__global__ __launch_bounds__(QB) void qr_begin(const double* pv, const int* pi, int nparts, QrState* st, int* hist) {
+  __shared__ double sv[QB / 64];
+  __shared__ int si[QB / 64];
+  double v;
+  int vi;
+  qr_top(pv, pi, nparts, v, vi, sv, si);
+  if (threadIdx.x == 0) {
+    st->j = st->base = st->r = st->ncand = st->fail = st->done = 0;
+    st->cut = -1;
+    st->refkey = v > 0.0 ? qr_key(v) : 0;
+  }
+  for (int b = threadIdx.x; b < QBINS; b += QB) hist[b] = 0;
+}
+
+// The block's residuals (one a thread) into the histogram, through LDS.
+__device__ inline void qr_count(double v, int refkey, int* h, int* hist) {
+  for (int b = threadIdx.x; b < QBINS; b += blockDim.x) h[b] = 0;
+  __syncthreads();
+  if (v > 0.0) {
+    const int b = qr_bin(v, refkey);
+    if (b < QBINS) atomicAdd(&h[b], 1);
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < QBINS; b += blockDim.x)
+    if (h[b]) atomicAdd(&hist[b], h[b]);
+}
+
+__global__ __launch_bounds__(QB) void qr_hist(const double* __restrict__ d, long n, const QrState* st, int* hist) {
+  __shared__ int h[QBINS];
+  const long a = (long)blockIdx.x * QB + threadIdx.x;
+  qr_count(a < n ? d[a] : 0.0, st->refkey, h, hist);
+}
+
+// Candidates: the points of the most bins from the top that hold at most QC
+// of them.  If the top bin alone holds more (or nothing is in range), the
+// first maximum is the only candidate.
+__global__ __launch_bounds__(QB) void qr_pick(const double* __restrict__ d, long n, int nparts, const double* pv,
+                                              const int* pi, const int* __restrict__ hist, QrState* st, int* cand) {
+  if (st->done) return;
+  constexpr int PER = QBINS / QB;
+  static_assert(PER * QB == QBINS, "bins split evenly over the threads");
+  __shared__ int part[QB];
+  __shared__ int cut;
+  __shared__ double sv[QB / 64];
+  __shared__ int si[QB / 64];
+  const int t = threadIdx.x;
+  const int refkey = st->refkey;
+  int c[PER], sum = 0;
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    c[q] = hist[t * PER + q];
+    sum += c[q];
+  }
+  part[t] = sum;
+  if (t == 0) cut = -1;
+  __syncthreads();
+  for (int o = 1; o < QB; o <<= 1) {
+    const int v = t >= o ? part[t - o] : 0;
+    __syncthreads();
+    part[t] += v;
+    __syncthreads();
+  }
+  int run = part[t] - sum;
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    run += c[q];
+    if (run > 0 && run <= QC) atomicMax(&cut, t * PER + q);
+  }
+  __syncthreads();
+  if (cut < 0) {
+    if (blockIdx.x == 0) {
+      double v;
+      int vi;
+      qr_top(pv, pi, nparts, v, vi, sv, si);
+      if (t == 0) {
+        st->cut = -1;
+        st->ncand = vi >= 0 && vi < n ? 1 : 0;
+        cand[0] = vi;
+      }
+    }
+    return;
+  }
+  if (blockIdx.x == 0 && t == 0) st->cut = cut;
+  const long a = (long)blockIdx.x * QB + t;
+  const double v = a < n ? d[a] : 0.0;
+  if (v > 0.0 && qr_bin(v, refkey) <= cut) cand[atomicAdd(&st->ncand, 1)] = (int)a;
+}
+
+// LT[q][t] = L[q][cand[t]], q < j, zero for rows up to the next multiple of 4
+// and slots without a candidate.
+__global__ __launch_bounds__(QC) void qr_gather(const double* __restrict__ L, long ln, const QrState* st,
+                                                const int* __restrict__ cand, double* __restrict__ LT) {
+  if (st->done) return;
+  const int t = threadIdx.x, j = st->j, j4 = (j + 3) & ~3;
+  const bool ok = t < st->ncand;
+  const double* src = L + (ok ? cand[t] : 0);
+  for (int q = blockIdx.x; q < j4; q += gridDim.x) LT[(long)q * QC + t] = ok && q < j ? src[q * ln] : 0.0;
+}
+
+typedef double qd4 __attribute__((ext_vector_type(4)));
+__device__ inline qd4 qr_mfma(double a, double b, qd4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+
+// entry k of i phi at point p (interleaved): against phi it gives the imaginary part of P
+__device__ inline double qr_times_i(const double* __restrict__ phi, long p, int m, int k) {
+  const double v = phi[p * m + (k ^ 1)];
+  return k & 1 ? -v : v;
+}
+template <int G>
+__device__ inline double qr_combine(double p, double q) {
+  return G == G_SQUARE ? p * p : (G == G_PRODUCT ? p * q : p * p + q * q);
+}
+
+// S = G - L L^T over the candidates: one 16 x 16 tile per workgroup, the inner
+// dimensions split over its four waves.
+template <int G>
+__global__ __launch_bounds__(256) void qr_gram(const double* __restrict__ phi, const double* __restrict__ occ, int m,
+                                               int mo, const QrState* st, const int* __restrict__ cand,
+                                               const double* __restrict__ LT, double* __restrict__ S) {
+  const int nc = st->ncand;
+  const int I = (blockIdx.x & 15) * 16, J = (blockIdx.x >> 4) * 16;
+  if (st->done || I >= nc || J >= nc) return;
+  __shared__ double red[3][4][256];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l16 = lane & 15, l4 = lane >> 4;
+  const int j4 = (st->j + 3) >> 2;
+  qd4 acc = {}, p1 = {}, p2 = {};
+  {
+    const int per = (j4 + 3) / 4, q0 = w * per, q1 = min(j4, q0 + per);
+    const double* base = LT + (long)l4 * QC + l16;
+    for (int q = q0; q < q1; q += 8) {  // eight steps' loads in flight
+      double x[8], y[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const double* row = base + (long)min(q + u, q1 - 1) * 4 * QC;
+        x[u] = row[I];
+        y[u] = row[J];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (q + u < q1) acc = qr_mfma(x[u], y[u], acc);
+    }
+  }
+  const long pi = I + l16 < nc ? cand[I + l16] : cand[0], pj = J + l16 < nc ? cand[J + l16] : cand[0];
+  for (int k0 = 4 * w; k0 < m; k0 += 64) {
+    double x[4], y[4], z[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = k0 + 16 * u + l4;
+      const bool ok = k < m;
+      x[u] = ok ? phi[pi * m + k] : 0.0;
+      y[u] = ok ? phi[pj * m + k] : 0.0;
+      z[u] = G == G_MODULUS && ok ? qr_times_i(phi, pj, m, k) : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      p1 = qr_mfma(x[u], y[u], p1);
+      if (G == G_MODULUS) p2 = qr_mfma(x[u], z[u], p2);
+    }
+  }
+  if (G == G_PRODUCT)
+    for (int k0 = 4 * w; k0 < mo; k0 += 64) {
+      double x[4], y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = k0 + 16 * u + l4;
+        x[u] = k < mo ? occ[pi * mo + k] : 0.0;
+        y[u] = k < mo ? occ[pj * mo + k] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) p2 = qr_mfma(x[u], y[u], p2);
+    }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int o = (l4 + 4 * v) * 16 + l16;
+    red[0][w][o] = acc[v];
+    red[1][w][o] = p1[v];
+    if (G != G_SQUARE) red[2][w][o] = p2[v];
+  }
+  __syncthreads();
+  const int t = threadIdx.x;
+  double sum[3] = {};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    sum[0] += red[0][q][t];
+    sum[1] += red[1][q][t];
+    if (G != G_SQUARE) sum[2] += red[2][q][t];
+  }
+  S[(long)(I + (t >> 4)) * QC + J + (t & 15)] = qr_combine<G>(sum[1], sum[2]) - sum[0];
+}
+
+// v, or where the DPP control moves a lane's value there, the larger of the two
+template <int CTRL, int ROWS>
+__device__ inline double qr_dpp_max(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return fmax(v, __longlong_as_double(((long long)hi << 32) | (unsigned)lo));
+}
+// maximum over the wave: within rows of 16 by shifts, then lane 15 of a row to
+// the next and lane 31 to the upper half; lane 63 holds it
+__device__ inline double qr_wave_max(double v) {
+  v = qr_dpp_max<0x111, 0xf>(v);
+  v = qr_dpp_max<0x112, 0xf>(v);
+  v = qr_dpp_max<0x114, 0xf>(v);
+  v = qr_dpp_max<0x118, 0xf>(v);
+  v = qr_dpp_max<0x142, 0xa>(v);
+  v = qr_dpp_max<0x143, 0xc>(v);
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// Pivot steps on the candidates, until the largest residual falls out of
+// their bins.  The first pivot of a round is the first maximum over all points
+// in any case: the candidates hold every point of the top bin.  One wave, four
+// candidates a lane (lane l owns l, l + 64, ...), so a step is a chain without
+// barriers: the maximum over the lanes, one row of S, r multiply-adds.  The
+// other waves read S once, so that its rows are in this XCD's L2 by then.
+__global__ __launch_bounds__(1024) void qr_run(const double* __restrict__ S, const double* __restrict__ d,
+                                             const int* __restrict__ cand, int k, QrState* st, int* __restrict__ hist,
+                                             int* __restrict__ piv, double* __restrict__ rdiag) {
+  if (st->done) return;
+  constexpr int PL = QC / 64;
+  __shared__ double lh[QR_MAX][QC];
+  const int lane = threadIdx.x & 63;
+  const int j = st->j, nc = st->ncand, cut = st->cut, refkey = st->refkey;
+  if (threadIdx.x >= 64) {
+    double sum = 0.0;
+    const int lines = (nc + 15) / 16;  // 128-byte lines of a row's first nc entries
+    for (int q = threadIdx.x - 64; q < nc * lines; q += 1024 - 64) sum += S[(long)(q / lines) * QC + q % lines * 16];
+    asm volatile("" ::"v"(sum));
+    return;
+  }
+  int me[PL];
+  double dt[PL];
+#pragma unroll
+  for (int u = 0; u < PL; ++u) {
+    const int t = lane + 64 * u;
+    me[u] = t < nc ? cand[t] : INT_MAX;
+    dt[u] = t < nc ? d[me[u]] : -DBL_MAX;
+  }
+  double d0 = j > 0 ? rdiag[0] * rdiag[0] : 0.0;
+  int newkey = refkey, fail = 0, r = 0;
+  for (; r < QR_MAX && j + r < k; ++r) {
+    double v = dt[0];
+    int vi = me[0], vs = lane;
+#pragma unroll
+    for (int u = 1; u < PL; ++u)
+      if (wins(dt[u], me[u], v, vi)) { v = dt[u]; vi = me[u]; vs = lane + 64 * u; }
+    const double top = qr_wave_max(v);
+    unsigned long long at = __ballot(v == top);
+    if (__popcll(at) > 1) {  // equal residuals: the first point
+      int low = v == top ? vi : INT_MAX;
+      for (int o = 32; o > 0; o >>= 1) low = min(low, __shfl_xor(low, o));
+      at = __ballot(v == top && vi == low);
+    }
+    const int win = at ? __ffsll((long long)at) - 1 : 0;
+    v = top;
+    vi = __builtin_amdgcn_readlane(vi, win);
+    vs = __builtin_amdgcn_readlane(vs, win);
+    if (r > 0 && (cut < 0 || !(v > 0.0) || qr_bin(v, refkey) > cut)) break;
+    if (j + r == 0) d0 = v;
+    // residual exhausted (K beyond the numerical rank): below 1e-13 of the first
+    // pivot the squared residuals are rounding noise of the Gram downdate
+    if (nc == 0 || !(v > 1e-13 * d0)) { fail = j + r + 1; break; }
+    if (r == 0) newkey = qr_key(v);
+    double c[PL];
+#pragma unroll
+    for (int u = 0; u < PL; ++u) c[u] = lane + 64 * u < nc ? S[(long)vs * QC + lane + 64 * u] : 0.0;
+    const double rt = sqrt(v), rs = 1.0 / rt;
+    const double mine = lane < r ? lh[lane & (QR_MAX - 1)][vs] : 0.0;
+#pragma unroll 4
+    for (int q = 0; q < r; ++q) {
+      const double f = lh[q][vs];
+#pragma unroll
+      for (int u = 0; u < PL; ++u) c[u] -= lh[q][lane + 64 * u] * f;
+    }
+#pragma unroll
+    for (int u = 0; u < PL; ++u) {
+      const double l = c[u] * rs;
+      lh[r][lane + 64 * u] = l;
+      if (lane + 64 * u == vs) dt[u] = RETIRED;
+      else if (dt[u] != RETIRED) dt[u] -= l * l;
+    }
+    if (lane == 0) {
+      st->slot[r] = vs;
+      st->piv[r] = vi;
+      st->rs[r] = rs;
+      piv[j + r] = vi;
+      rdiag[j + r] = rt;
+    }
+    if (lane < r) st->tri[lane][r] = mine;
+    // the next step's reads of lh follow these writes in the wave's own order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  }
+  for (int b = lane; b < QBINS; b += 64) hist[b] = 0;
+  if (lane == 0) {
+    st->base = j;
+    st->r = r;
+    st->j = j + r;
+    st->ncand = 0;
+    st->refkey = newkey;
+    st->fail = fail;
+    st->done = fail || j + r >= k;
+  }
+}
+
+// The pivots' columns of LT side by side, LP[q][s] (zero for s >= r), so that
+// qr_apply reads them in whole lines: with every wave gathering them from LT
+// the 40^3, K = 512 run took 3.05 ms, with this kernel 2.80.
+__global__ __launch_bounds__(256) void qr_compact(const QrState* st, const double* __restrict__ LT,
+                                                  double* __restrict__ LP) {
+  if (st->done) return;
+  const int s = threadIdx.x & (QR_MAX - 1), j4 = (st->base + 3) & ~3;
+  const bool ok = s < st->r;
+  const double* src = LT + (ok ? st->slot[s] : 0);
+  constexpr int ROWS = 256 / QR_MAX;
+  for (int q = blockIdx.x * ROWS + threadIdx.x / QR_MAX; q < j4; q += gridDim.x * ROWS)
+    LP[q * QR_MAX + s] = ok ? src[(long)q * QC] : 0.0;
+}
+
+// The round's r columns of L for all points, one pass over the earlier ones:
+// acc[s][a] = sum_q L[q][p_s] L[q][a] by MFMA (A: the pivots' entries from LP,
+// B: 32 points a wave, two interleaved 16-point fragments from one 16-byte
+// load), G the same way from the orbitals, then the triangular solve with one
+// lane a point.  Loads of QU steps are in flight while the previous QU are
+// multiplied.  Bound by the read of L, 8 j N bytes a round, and by latency: two
+// waves a SIMD at N = 64000, 3.4 TB/s.
+constexpr int QU = 8;
+constexpr int QW = QB / 32;  // waves of a workgroup: 32 points each, QB together
+
+template <int G>
+__global__ __launch_bounds__(64 * QW) void qr_apply(const double* __restrict__ phi, const double* __restrict__ occ,
+                                                    long n, int m, int mo, double* __restrict__ d,
+                                                    double* __restrict__ L, long ln, const double* __restrict__ LP,
+                                                    const QrState* __restrict__ st, double* pv, int* pi, int* hist) {
+  if (st->done) return;
+  __shared__ double tile[QW][32][QR_MAX + 1];
+  __shared__ int h[QBINS];
+  __shared__ double sv[QW];
+  __shared__ int si[QW];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l16 = lane & 15, l4 = lane >> 4;
+  const int r = st->r, j = st->base;
+  const bool two = r > 16;
+  const long a0 = (long)blockIdx.x * QB + 32 * w;
+  qd4 acc[2][2] = {}, p1[2][2] = {}, p2[2][2] = {};
+  {
+    // rows are ln >= the workgroups' points apart, so every load is inside L
+    const double2* lb = reinterpret_cast<const double2*>(L + (long)l4 * ln + a0 + 2 * l16);
+    const double* t0 = LP + l4 * QR_MAX + l16;
+    const long lstep = 2 * ln;  // four rows, in double2
+    const int n4 = j >> 2;      // whole steps of four columns
+    auto columns = [&](auto both) {
+      double2 b[2][QU];
+      double u0[2][QU], u1[2][QU];
+      auto load = [&](int buf, int q0) {
+#pragma unroll
+        for (int u = 0; u < QU; ++u) {
+          const int q = min(q0 + u, n4 - 1);
+          b[buf][u] = lb[q * lstep];
+          u0[buf][u] = t0[q * 4 * QR_MAX];
+          if (both.value) u1[buf][u] = t0[q * 4 * QR_MAX + 16];
+        }
+      };
+      auto mul = [&](int buf, int u) {
+        acc[0][0] = qr_mfma(u0[buf][u], b[buf][u].x, acc[0][0]);
+        acc[0][1] = qr_mfma(u0[buf][u], b[buf][u].y, acc[0][1]);
+        if (both.value) {
+          acc[1][0] = qr_mfma(u1[buf][u], b[buf][u].x, acc[1][0]);
+          acc[1][1] = qr_mfma(u1[buf][u], b[buf][u].y, acc[1][1]);
+        }
+      };
+      load(0, 0);
+      int q = 0;
+      for (; q + 2 * QU <= n4; q += 2 * QU) {
+        load(1, q + QU);
+#pragma unroll
+        for (int u = 0; u < QU; ++u) mul(0, u);
+        load(0, q + 2 * QU);  // past the end: the last step again, not multiplied
+#pragma unroll
+        for (int u = 0; u < QU; ++u) mul(1, u);
+      }
+      if (q + QU < n4) load(1, q + QU);
+#pragma unroll
+      for (int u = 0; u < 2 * QU; ++u)
+        if (q + u < n4) mul(u / QU, u % QU);
+    };
+    if (n4 > 0) {
+      if (two) columns(std::true_type{});
+      else columns(std::false_type{});
+    }
+    if (j & 3) {  // the last one to three columns; LP is zero beyond them, L is not
+      const bool ok = 4 * n4 + l4 < j;
+      const double2 x = ok ? lb[n4 * lstep] : double2{0.0, 0.0};
+      const double v0 = t0[n4 * 4 * QR_MAX], v1 = t0[n4 * 4 * QR_MAX + 16];
+      acc[0][0] = qr_mfma(v0, x.x, acc[0][0]);
+      acc[0][1] = qr_mfma(v0, x.y, acc[0][1]);
+      acc[1][0] = qr_mfma(v1, x.x, acc[1][0]);
+      acc[1][1] = qr_mfma(v1, x.y, acc[1][1]);
+    }
+  }
+  {
+    const long ra = min(a0 + 2 * l16, n - 1), rb = min(a0 + 2 * l16 + 1, n - 1);
+    const long q0 = st->piv[min(l16, r - 1)], q1 = st->piv[min(16 + l16, r - 1)];
+    for (int k0 = 0; k0 < m; k0 += 4) {
+      const int k = k0 + l4;
+      const bool ok = k < m;
+      const double x = ok ? phi[ra * m + k] : 0.0, y = ok ? phi[rb * m + k] : 0.0;
+      const double u = ok ? phi[q0 * m + k] : 0.0, v = ok ? phi[q1 * m + k] : 0.0;
+      p1[0][0] = qr_mfma(u, x, p1[0][0]);
+      p1[0][1] = qr_mfma(u, y, p1[0][1]);
+      if (two) {
+        p1[1][0] = qr_mfma(v, x, p1[1][0]);
+        p1[1][1] = qr_mfma(v, y, p1[1][1]);
+      }
+      if (G == G_MODULUS) {
+        const double u2 = ok ? qr_times_i(phi, q0, m, k) : 0.0;
+        const double v2 = ok ? qr_times_i(phi, q1, m, k) : 0.0;
+        p2[0][0] = qr_mfma(u2, x, p2[0][0]);
+        p2[0][1] = qr_mfma(u2, y, p2[0][1]);
+        p2[1][0] = qr_mfma(v2, x, p2[1][0]);
+        p2[1][1] = qr_mfma(v2, y, p2[1][1]);
+      }
+    }
+    if (G == G_PRODUCT)
+      for (int k0 = 0; k0 < mo; k0 += 4) {
+        const int k = k0 + l4;
+        const bool ok = k < mo;
+        const double x = ok ? occ[ra * mo + k] : 0.0, y = ok ? occ[rb * mo + k] : 0.0;
+        const double u = ok ? occ[q0 * mo + k] : 0.0, v = ok ? occ[q1 * mo + k] : 0.0;
+        p2[0][0] = qr_mfma(u, x, p2[0][0]);
+        p2[0][1] = qr_mfma(u, y, p2[0][1]);
+        p2[1][0] = qr_mfma(v, x, p2[1][0]);
+        p2[1][1] = qr_mfma(v, y, p2[1][1]);
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        tile[w][2 * l16 + f][16 * i + l4 + 4 * v] = qr_combine<G>(p1[i][f][v], p2[i][f][v]) - acc[i][f][v];
+  __syncthreads();
+  const long a = a0 + lane;
+  double v = -DBL_MAX;
+  int vi = INT_MAX;
+  if (lane < 32 && a < n) {
+    double x[QR_MAX];
+#pragma unroll
+    for (int s = 0; s < QR_MAX; ++s) x[s] = tile[w][lane][s];
+    double da = d[a];
+#pragma unroll
+    for (int s = 0; s < QR_MAX; ++s)
+      if (s < r) {
+        const double l = x[s] * st->rs[s];
+        L[(j + s) * ln + a] = l;
+#pragma unroll
+        for (int q = s + 1; q < QR_MAX; ++q) x[q] -= l * st->tri[s][q];
+        if (a == st->piv[s] || da == RETIRED) da = RETIRED;
+        else da -= l * l;
+      }
+    d[a] = da;
+    v = da;
+    vi = (int)a;
+  }
+  qr_count(v, st->refkey, h, hist);
+  for (int o = 32; o > 0; o >>= 1) {
+    const double ov = __shfl_xor(v, o);
+    const int oi = __shfl_xor(vi, o);
+    if (wins(ov, oi, v, vi)) { v = ov; vi = oi; }
+  }
+  if (lane == 0) { sv[w] = v; si[w] = vi; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < QW; ++q)
+      if (wins(sv[q], si[q], v, vi)) { v = sv[q]; vi = si[q]; }
+    pv[blockIdx.x] = v;
+    pi[blockIdx.x] = vi;
+  }
+}
+
+// ---- one pivot a step, for complex half-rotated orbitals -----------------------
 // Pivot step j; partial maxima are read from (pv_in, pi_in) and written to
-// (pv_out, pi_out), which the host alternates between steps.
-// MODE 0: real orbitals; 1: complex orbitals, all on both sides (real G);
-// 2: complex half-rotated (complex G and L: L[2q] real, L[2q + 1] imaginary
-// parts of column q).
-template <int MODE>
+// (pv_out, pi_out), which the host alternates between steps.  G and L are
+// complex: L[2q] holds the real, L[2q + 1] the imaginary parts of column q.
 __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, const double* __restrict__ occ, long n,
                                               int m, int mo, int j, int nparts, double* __restrict__ d,
                                               double* __restrict__ L, const double* pv_in, const int* pi_in,
                                               double* pv_out, int* pi_out, int* piv, double* rdiag, int* fail) {
-  extern __shared__ double sh[];  // pivot rows: phi (m), occ (mo), then L[q][p] for q < j (2j values in MODE 2)
+  extern __shared__ double sh[];  // pivot rows: phi (m), occ (mo), then L[q][p], 2j values
   __shared__ double gv;
   __shared__ int gi;
   // global argmax of the previous residuals (every block, redundantly)
@@ -160,12 +701,10 @@ __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, co
   }
   double* prow = sh;
   double* orow = sh + m;
-  double* lp = orow + (occ ? mo : 0);
+  double* lp = orow + mo;
   for (int q = threadIdx.x; q < m; q += QB) prow[q] = phi[p * m + q];
-  if (occ)
-    for (int q = threadIdx.x; q < mo; q += QB) orow[q] = occ[p * mo + q];
-  constexpr int LW = MODE == 2 ? 2 : 1;  // doubles per entry of L
-  for (int q = threadIdx.x; q < LW * j; q += QB) lp[q] = L[(long)q * n + p];
+  for (int q = threadIdx.x; q < mo; q += QB) orow[q] = occ[p * mo + q];
+  for (int q = threadIdx.x; q < 2 * j; q += QB) lp[q] = L[(long)q * n + p];
   __syncthreads();
   const double rs = 1.0 / sqrt(pval);
   const long a = (long)blockIdx.x * QB + threadIdx.x;
@@ -173,45 +712,22 @@ __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, co
   int vi = INT_MAX;
   if (a < n) {
     double da = d[a];
-    if (MODE == 2) {
-      double qr, qi, o_r, o_i;
-      cdot_row(phi + a * m, prow, m, qr, qi);
-      cdot_row(occ + a * mo, orow, mo, o_r, o_i);
-      const double gr = o_r * qr + o_i * qi, gi = o_r * qi - o_i * qr;  // conj(Qocc) Q
-      double ar = 0.0, ai = 0.0;
-      for (int q = 0; q < j; ++q) {
-        const double xr = L[(long)(2 * q) * n + a], xi = L[(long)(2 * q + 1) * n + a];
-        const double yr = lp[2 * q], yi = lp[2 * q + 1];
-        ar = fma(xr, yr, fma(xi, yi, ar));
-        ai = fma(xi, yr, fma(-xr, yi, ai));
-      }
-      const double lr = (gr - ar) * rs, li = (gi - ai) * rs;
-      L[(long)(2 * j) * n + a] = lr;
-      L[(long)(2 * j + 1) * n + a] = li;
-      if (a == p || da == RETIRED) da = RETIRED;
-      else da -= lr * lr + li * li;
-    } else {
-      double g;
-      if (MODE == 1) {
-        double qr, qi;
-        cdot_row(phi + a * m, prow, m, qr, qi);
-        g = qr * qr + qi * qi;  // |Q[a][p]|^2
-      } else {
-        const double s = dot_row(phi + a * m, prow, m);
-        g = occ ? s * dot_row(occ + a * mo, orow, mo) : s * s;
-      }
-      double acc0 = 0.0, acc1 = 0.0;
-      int q = 0;
-      for (; q + 2 <= j; q += 2) {
-        acc0 = fma(L[(long)q * n + a], lp[q], acc0);
-        acc1 = fma(L[(long)(q + 1) * n + a], lp[q + 1], acc1);
-      }
-      if (q < j) acc0 = fma(L[(long)q * n + a], lp[q], acc0);
-      const double l = (g - (acc0 + acc1)) * rs;
-      L[(long)j * n + a] = l;
-      if (a == p || da == RETIRED) da = RETIRED;
-      else da -= l * l;
+    double qr, qi, o_r, o_i;
+    cdot_row(phi + a * m, prow, m, qr, qi);
+    cdot_row(occ + a * mo, orow, mo, o_r, o_i);
+    const double gr = o_r * qr + o_i * qi, gi = o_r * qi - o_i * qr;  // conj(Qocc) Q
+    double ar = 0.0, ai = 0.0;
+    for (int q = 0; q < j; ++q) {
+      const double xr = L[(long)(2 * q) * n + a], xi = L[(long)(2 * q + 1) * n + a];
+      const double yr = lp[2 * q], yi = lp[2 * q + 1];
+      ar = fma(xr, yr, fma(xi, yi, ar));
+      ai = fma(xi, yr, fma(-xr, yi, ai));
     }
+    const double lr = (gr - ar) * rs, li = (gi - ai) * rs;
+    L[(long)(2 * j) * n + a] = lr;
+    L[(long)(2 * j + 1) * n + a] = li;
+    if (a == p || da == RETIRED) da = RETIRED;
+    else da -= lr * lr + li * li;
     d[a] = da;
     v = da;
     vi = (int)a;
@@ -221,12 +737,61 @@ __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, co
 
 }  // namespace
 
+// L of the rounds: rows of whole workgroups' points
+inline long qr_ln(long n) { return (n + QB - 1) / QB * QB; }
+
 size_t qrcp_work_bytes(long n, int k, bool cplx) {
   const long nparts = (n + QB - 1) / QB;
-  return carve_bytes<double>((size_t)n) + carve_bytes<double>((size_t)n * k * (cplx ? 2 : 1)) +
+  return carve_bytes<double>((size_t)n) + carve_bytes<double>((size_t)qr_ln(n) * k * (cplx ? 2 : 1)) +
          2 * carve_bytes<double>(nparts) + 2 * carve_bytes<int>(nparts) + carve_bytes<int>(k) +
-         carve_bytes<double>(k) + carve_bytes<int>(1);
+         carve_bytes<double>(k) + carve_bytes<int>(1) + carve_bytes<double>((size_t)(k + 4) * QC) +
+         carve_bytes<double>((size_t)(k + 4) * QR_MAX) + carve_bytes<double>((size_t)QC * QC) + carve_bytes<int>(QC) + carve_bytes<int>(QBINS) +
+         carve_bytes<QrState>(1);
 }
+
+namespace {
+
+// Rounds of pivots (real G) until k are chosen; pv, pi hold the first maxima.
+template <int G>
+int qr_rounds(const double* phi, const double* occ, long n, int m, int mo, int k, double* d, double* L, double* pv,
+              int* pi, int* piv, double* rd, int* fail, Arena& ws, hipStream_t s) {
+  const int nparts = (int)((n + QB - 1) / QB);
+  const long ln = qr_ln(n);
+  double* LT = ws.take<double>((size_t)(k + 4) * QC);
+  double* LP = ws.take<double>((size_t)(k + 4) * QR_MAX);
+  double* S = ws.take<double>((size_t)QC * QC);
+  int* cand = ws.take<int>(QC);
+  int* hist = ws.take<int>(QBINS);
+  QrState* st = ws.take<QrState>(1);
+  if (!LT || !LP || !S || !cand || !hist || !st) return THC_ERR_NO_MEMORY;
+  hipLaunchKernelGGL(qr_begin, dim3(1), dim3(QB), 0, s, pv, pi, nparts, st, hist);
+  hipLaunchKernelGGL(qr_hist, dim3(nparts), dim3(QB), 0, s, d, n, st, hist);
+  // Every round chooses a pivot or ends the run.  The host looks after up to
+  // eight rounds, fewer where the pivots left should take fewer (16 a round);
+  // rounds past the end return at once.
+  int h[3] = {0, 0, 0};  // j, fail, done
+  for (int rounds = 0; rounds <= k + 8 && !h[2];) {
+    const int batch = std::max(1, std::min(8, (k - h[0] + 15) / 16));
+    for (int q = 0; q < batch; ++q) {
+      hipLaunchKernelGGL(qr_pick, dim3(nparts), dim3(QB), 0, s, d, n, nparts, pv, pi, hist, st, cand);
+      hipLaunchKernelGGL(qr_gather, dim3(256), dim3(QC), 0, s, L, ln, st, cand, LT);
+      hipLaunchKernelGGL(qr_gram<G>, dim3((QC / 16) * (QC / 16)), dim3(256), 0, s, phi, occ, m, mo, st, cand, LT, S);
+      hipLaunchKernelGGL(qr_run, dim3(1), dim3(1024), 0, s, S, d, cand, k, st, hist, piv, rd);
+      hipLaunchKernelGGL(qr_compact, dim3(64), dim3(256), 0, s, st, LT, LP);
+      hipLaunchKernelGGL(qr_apply<G>, dim3(nparts), dim3(64 * QW), 0, s, phi, occ, n, m, mo, d, L, ln, LP, st, pv, pi,
+                         hist);
+    }
+    rounds += batch;
+    THC_HIP(hipGetLastError());
+    THC_HIP(hipMemcpyAsync(h, &st->j, sizeof(h), hipMemcpyDeviceToHost, s));
+    THC_HIP(hipStreamSynchronize(s));
+  }
+  h[1] = h[2] ? h[1] : k + 1;
+  *fail = h[1];
+  return THC_OK;
+}
+
+}  // namespace
 
 int qrcp_points(const double* phi, const double* occ, long n, int m, int mo, int k, int* piv_out, double* rdiag_out,
                 Arena& ws, hipStream_t s, bool cplx) {
@@ -235,7 +800,7 @@ int qrcp_points(const double* phi, const double* occ, long n, int m, int mo, int
   if (cplx && (m % 2 || (occ && mo % 2))) return THC_ERR_ARG;
   const int mode = !cplx ? 0 : (occ ? 2 : 1);
   double* d = ws.take<double>((size_t)n);
-  double* L = ws.take<double>((size_t)n * k * (mode == 2 ? 2 : 1));
+  double* L = ws.take<double>((size_t)qr_ln(n) * k * (mode == 2 ? 2 : 1));
   double* pv[2] = {ws.take<double>(nparts), ws.take<double>(nparts)};
   int* pi[2] = {ws.take<int>(nparts), ws.take<int>(nparts)};
   int* piv = ws.take<int>(k);
@@ -243,29 +808,29 @@ int qrcp_points(const double* phi, const double* occ, long n, int m, int mo, int
   int* fail = ws.take<int>(1);
   if (!d || !L || !pv[0] || !pv[1] || !pi[0] || !pi[1] || !piv || !rd || !fail) return THC_ERR_NO_MEMORY;
   const size_t lds = sizeof(double) * ((size_t)m + (occ ? mo : 0) + (size_t)k * (mode == 2 ? 2 : 1));
-  const void* step_fn = mode == 0 ? (const void*)qr_step<0> : (mode == 1 ? (const void*)qr_step<1>
-                                                                          : (const void*)qr_step<2>);
   if (lds > 160 * 1024) return THC_ERR_UNSUPPORTED;
-  if (lds > 64 * 1024) THC_HIP(hipFuncSetAttribute(step_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  THC_HIP(hipMemsetAsync(fail, 0, sizeof(int), s));
   hipLaunchKernelGGL(qr_init, dim3((unsigned)nparts), dim3(QB), 0, s, phi, occ, n, m, mo, d, pv[0], pi[0]);
   THC_HIP(hipGetLastError());
-  for (int j = 0; j < k; ++j) {
-    const int in = j & 1;
-    if (mode == 0)
-      hipLaunchKernelGGL(qr_step<0>, dim3((unsigned)nparts), dim3(QB), lds, s, phi, occ, n, m, mo, j, (int)nparts, d,
-                         L, pv[in], pi[in], pv[in ^ 1], pi[in ^ 1], piv, rd, fail);
-    else if (mode == 1)
-      hipLaunchKernelGGL(qr_step<1>, dim3((unsigned)nparts), dim3(QB), lds, s, phi, occ, n, m, mo, j, (int)nparts, d,
-                         L, pv[in], pi[in], pv[in ^ 1], pi[in ^ 1], piv, rd, fail);
-    else
-      hipLaunchKernelGGL(qr_step<2>, dim3((unsigned)nparts), dim3(QB), lds, s, phi, occ, n, m, mo, j, (int)nparts, d,
-                         L, pv[in], pi[in], pv[in ^ 1], pi[in ^ 1], piv, rd, fail);
-  }
-  THC_HIP(hipGetLastError());
   int h_fail = 0;
+  if (mode == 2) {
+    if (lds > 64 * 1024)
+      THC_HIP(hipFuncSetAttribute((const void*)qr_step, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    THC_HIP(hipMemsetAsync(fail, 0, sizeof(int), s));
+    for (int j = 0; j < k; ++j) {
+      const int in = j & 1;
+      hipLaunchKernelGGL(qr_step, dim3((unsigned)nparts), dim3(QB), lds, s, phi, occ, n, m, mo, j, (int)nparts, d, L,
+                         pv[in], pi[in], pv[in ^ 1], pi[in ^ 1], piv, rd, fail);
+    }
+    THC_HIP(hipGetLastError());
+    THC_HIP(hipMemcpyAsync(&h_fail, fail, sizeof(int), hipMemcpyDeviceToHost, s));
+  } else if (mode == 1) {
+    THC_TRY(qr_rounds<G_MODULUS>(phi, nullptr, n, m, 0, k, d, L, pv[0], pi[0], piv, rd, &h_fail, ws, s));
+  } else if (occ) {
+    THC_TRY(qr_rounds<G_PRODUCT>(phi, occ, n, m, mo, k, d, L, pv[0], pi[0], piv, rd, &h_fail, ws, s));
+  } else {
+    THC_TRY(qr_rounds<G_SQUARE>(phi, nullptr, n, m, 0, k, d, L, pv[0], pi[0], piv, rd, &h_fail, ws, s));
+  }
   std::vector<int> h(k);
-  THC_HIP(hipMemcpyAsync(&h_fail, fail, sizeof(int), hipMemcpyDeviceToHost, s));
   THC_HIP(hipMemcpyAsync(h.data(), piv, sizeof(int) * k, hipMemcpyDeviceToHost, s));
   if (rdiag_out) THC_HIP(hipMemcpyAsync(rdiag_out, rd, sizeof(double) * k, hipMemcpyDeviceToHost, s));
   THC_HIP(hipStreamSynchronize(s));
