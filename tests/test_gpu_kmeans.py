@@ -213,3 +213,73 @@ def test_device_sqrt_correctly_rounded(ctx):
     ref = np.sqrt(x)
     bad = np.flatnonzero(got.view(np.int64) != ref.view(np.int64))
     assert bad.size == 0, (bad.size, x[bad[:5]], got[bad[:5]], ref[bad[:5]])
+
+
+@pytest.mark.parametrize("n,k,big", [(70000, 301, 42000), (200000, 90, 1500), (3000, 2, 1024), (3000, 2, 1025),
+                                     (2000, 3, 512), (2000, 3, 513)])
+def test_update_centroids_cluster_sizes(ctx, n, k, big):
+    """Clusters either side of what a workgroup sums at a time (512), keeps in registers (1024) and finds in its
+    bucket (8 n / k), members spread over several 65536-point windows of the index range."""
+    rng = np.random.default_rng(n + k + big)
+    grid = rng.uniform(0, 7, size=(n, 3))
+    rho = rng.uniform(0.1, 2.0, size=n)
+    gmap = np.empty(n, dtype=np.int32)
+    order = rng.permutation(n)
+    gmap[order[:big]] = k // 2
+    rest = np.array([c for c in range(k) if c != k // 2])
+    gmap[order[big:]] = rest[np.arange(n - big) % len(rest)]
+    got, st = ctx.update_centroids(rho, grid, gmap, k)
+    ref, crit = KO.update_centroids(rho, grid, gmap, k)
+    assert st == L.THC_OK and crit == 0
+    np.testing.assert_array_equal(got.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("k", [1, 256, 257, 1024, 1025, 2048, 2049, 4096])
+def test_kmeans_cluster_counts(ctx, k):
+    """Either side of the assignment's centroids-per-thread variants; a loop that no threshold can stop and one
+    with a threshold that is never reached give the same run."""
+    rng = np.random.default_rng(k)
+    n = 6000
+    grid = rng.uniform(0, 9, size=(n, 3))
+    rho = rng.uniform(0.1, 2.0, size=n)
+    ref = KO.kmeans(grid, rho, k, 3, -1.0, 5)
+    for thr in (-1.0, 0.0 if ref["diffs"][-1] > 0 else -2.0):
+        out = ctx.kmeans(grid, rho, k, 3, thr, 5, want_map=True, want_centroids=True)
+        np.testing.assert_array_equal(out["interp_idx"].cpu().numpy(), ref["interp_idx"])
+        np.testing.assert_array_equal(out["diffs"], ref["diffs"])
+        np.testing.assert_array_equal(out["pcts"], ref["pcts"])
+        np.testing.assert_array_equal(out["centroids"].cpu().numpy(), ref["centroids"])
+
+
+def test_kmeans_dense_clump(ctx):
+    """All but a few points in a clump that holds one starting centroid: a cluster beyond its bucket, and tiles
+    whose bounds keep almost every centroid."""
+    rng = np.random.default_rng(8)
+    n, k = 20000, 60
+    grid = rng.uniform(0, 30, size=(n, 3))
+    grid[100:] = 15.0 + 0.4 * rng.standard_normal((n - 100, 3))
+    rho = rng.uniform(0.1, 2.0, size=n)
+    init = np.concatenate([np.arange(k - 1), [150]]).astype(np.int32)
+    ref = KO.kmeans(grid, rho, k, 4, -1.0, 0, init_idx=init, keep_maps=True)
+    assert np.bincount(ref["maps"][0], minlength=k).max() > 8 * (n // k + 1)
+    for thr in (-1.0, 1e-300):
+        out = ctx.kmeans(grid, rho, k, 4, thr, 0, init_idx=init, want_map=True)
+        np.testing.assert_array_equal(out["interp_idx"].cpu().numpy(), ref["interp_idx"])
+        np.testing.assert_array_equal(out["diffs"], ref["diffs"])
+        np.testing.assert_array_equal(out["grid_map"].cpu().numpy(), ref["maps"][-1])
+
+
+@pytest.mark.parametrize("n,k,seed", [(40, 12, 132), (40, 12, 1857), (60, 25, 1710)])
+def test_kmeans_empty_cluster_later(ctx, n, k, seed):
+    """A weight that vanishes in the second iteration (densities over 13 decades) stops the run there, whether or
+    not the loop waits for the differences."""
+    rng = np.random.default_rng(seed)
+    grid = rng.integers(0, 5, size=(n, 3)).astype(float)
+    rho = 10.0 ** rng.uniform(-12, 1, size=n)
+    ref = KO.kmeans(grid, rho, k, 8, -1.0, seed)
+    assert ref["status"] == 1 and ref["iters"] == 2
+    for thr in (-1.0, 0.0):
+        out = ctx.kmeans(grid, rho, k, 8, thr, seed)
+        assert out["status"] == L.THC_ERR_EMPTY_CLUSTER
+        assert out["iters"] == 2
+        assert out["diffs"][0] == ref["diffs"][0]

@@ -10,6 +10,7 @@ constexpr int CS_TILE = 1024;  // points per counting-sort tile (index order)
 constexpr int CS_SCAN_W = 16;  // waves of a column-scan workgroup
 constexpr int MAXB = 4096;     // max bins: clusters, and Morton cells of the spatial sort
 constexpr int CAND_CAP = 512;  // candidate centroids cached in LDS per tile
+constexpr int CHG = 32;        // partial counts of changed points per iteration
 
 enum { MODE_LATEST = 0, MODE_FINAL = 1, MODE_ZEROS = 2 };
 
@@ -18,8 +19,7 @@ struct State {
   int done;        // loop ended: diff < threshold, or an error
   int final_buf;   // centroid buffer with the converged centroids (MODE_FINAL)
   int error;       // 1: a cluster weight < 1e-8 in an iteration the loop ran; 2: bad cluster key
-  int changed[2];  // points whose cluster changed, by iteration parity
-  int serr[2];     // a cluster weight < 1e-8 in the centroid sums, by iteration parity
+  int bad;         // first iteration with a cluster weight < 1e-8 (later ones do nothing), else INT_MAX
   int iters;       // iterations executed
   int mode;        // which centroids map_to_grid uses (MODE_*)
   int dups;        // repeated indices after map_to_grid

@@ -9,8 +9,8 @@
 //    (std::min_element), evaluated as a lexicographic (distance, index) minimum;
 //    sqrt is monotone, so a sqrt is only needed when d^2 improves;
 //  * centroid sums run per cluster in ascending grid index with the product
-//    rounded before the add (a stable counting sort supplies that order), and
-//    are divided once (IEEE double division);
+//    rounded before the add (a bitmap over the members' indices supplies that
+//    order), and are divided once (IEEE double division);
 //  * pruning of centroids (or grid tiles) is conservative: a candidate is
 //    dropped only if its distance bound exceeds the best bound by a relative
 //    1e-8 on squares, far above the few-ulp rounding of any distance.
@@ -18,6 +18,7 @@
 #include <atomic>
 #include <cfloat>
 #include <climits>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -62,13 +63,84 @@ __device__ inline double ub2_box(double cx, double cy, double cz, const double* 
 }
 constexpr double PRUNE = 1.0 + 1e-8;
 
+// Wave-wide reductions by DPP moves: within rows of 16 lanes by shifts, then
+// lane 15 of a row into the next row and lane 31 into the upper half, so lane
+// 63 ends with the result (about 25 cycles a step; a cross-lane permute through
+// LDS takes over 100).  Every lane of the wave must be active.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_min(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return fmin(v, __longlong_as_double(((long long)hi << 32) | (unsigned)lo));
+}
 __device__ inline double wave_min(double v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
+  v = dpp_min<0x111, 0xf>(v);
+  v = dpp_min<0x112, 0xf>(v);
+  v = dpp_min<0x114, 0xf>(v);
+  v = dpp_min<0x118, 0xf>(v);
+  v = dpp_min<0x142, 0xa>(v);
+  v = dpp_min<0x143, 0xc>(v);
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int CTRL, int ROWS>
+__device__ inline int dpp_get(int none, int v) { return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 0xf, false); }
+// inclusive sum over the lanes up to this one
+__device__ inline int wave_scan(int v) {
+  v += dpp_get<0x111, 0xf>(0, v);
+  v += dpp_get<0x112, 0xf>(0, v);
+  v += dpp_get<0x114, 0xf>(0, v);
+  v += dpp_get<0x118, 0xf>(0, v);
+  v += dpp_get<0x142, 0xa>(0, v);
+  v += dpp_get<0x143, 0xc>(0, v);
   return v;
 }
-__device__ inline int wave_sum(int v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+__device__ inline int wave_sum(int v) { return __builtin_amdgcn_readlane(wave_scan(v), 63); }
+__device__ inline int wave_min(int v) {
+  v = min(v, dpp_get<0x111, 0xf>(v, v));
+  v = min(v, dpp_get<0x112, 0xf>(v, v));
+  v = min(v, dpp_get<0x114, 0xf>(v, v));
+  v = min(v, dpp_get<0x118, 0xf>(v, v));
+  v = min(v, dpp_get<0x142, 0xa>(v, v));
+  v = min(v, dpp_get<0x143, 0xc>(v, v));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// acc + v[0] + v[1] + ... strictly left to right (one lane's chain), from LDS
+// at 16-byte alignment: the next sixteen terms are read while the current ones
+// are added.
+__device__ inline double seq_sum(double acc, const double* v, int len) {
+  const double2* p = reinterpret_cast<const double2*>(v);
+  const int nb = len / 16;
+  double2 a[8], b[8];
+  if (nb > 0) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) a[q] = p[q];
+  }
+  for (int i = 0; i < nb; i += 2) {
+    const int i1 = min(i + 1, nb - 1), i2 = min(i + 2, nb - 1);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) b[q] = p[8 * i1 + q];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      acc += a[q].x;
+      acc += a[q].y;
+    }
+    if (i + 1 >= nb) break;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) a[q] = p[8 * i2 + q];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      acc += b[q].x;
+      acc += b[q].y;
+    }
+  }
+  for (int i = 16 * nb; i < len; ++i) acc += v[i];
+  return acc;
 }
 
 // ------------------------------------------------------------------ setup
@@ -99,67 +171,59 @@ __global__ __launch_bounds__(256) void bbox_partial(const double* grid, long n, 
   bbox_partial_b(grid, n, part, (int)blockIdx.x, (int)gridDim.x);
 }
 
-__device__ __forceinline__ void bbox_final_b(const double* part, int nb, double* box, int bid, int nblk) {
-  const int d = threadIdx.x;
-  if (d >= 6) return;
-  double r = part[d];
-  for (int b = 1; b < nb; ++b) r = d < 3 ? fmin(r, part[b * 6 + d]) : fmax(r, part[b * 6 + d]);
-  box[d] = r;
-}
-__global__ void bbox_final(const double* part, int nb, double* box) {
-  bbox_final_b(part, nb, box, (int)blockIdx.x, (int)gridDim.x);
-}
-
 __device__ inline unsigned spread3(unsigned v) {
   unsigned r = 0;
   for (int b = 0; b < 10; ++b) r |= ((v >> b) & 1u) << (3 * b);
   return r;
 }
 
-__device__ __forceinline__ void morton_keys_b(const double* grid, long n, const double* box, int cells,
-                                                   int* keys, int bid, int nblk) {
-  const long i = bid * 256L + threadIdx.x;
+// Morton cell of every point inside the bounding box of the nb partial ones
+// (nb <= 256; every workgroup folds them by itself).
+__device__ __forceinline__ void morton_keys_b(const double* grid, long n, const double* part, int nb, int cells,
+                                                   int* keys, int bid) {
+  __shared__ double s[6][4];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  for (int d = 0; d < 3; ++d) {
+    const double a = wave_min(t < nb ? part[t * 6 + d] : DBL_MAX);
+    const double b = -wave_min(t < nb ? -part[t * 6 + 3 + d] : DBL_MAX);
+    if (lane == 0) { s[d][w] = a; s[3 + d][w] = b; }
+  }
+  __syncthreads();
+  const long i = bid * 256L + t;
   if (i >= n) return;
   unsigned c[3];
   for (int d = 0; d < 3; ++d) {
-    const double lo = box[d], ext = box[3 + d] - box[d];
+    const double lo = fmin(fmin(s[d][0], s[d][1]), fmin(s[d][2], s[d][3]));
+    const double ext = fmax(fmax(s[3 + d][0], s[3 + d][1]), fmax(s[3 + d][2], s[3 + d][3])) - lo;
     int v = 0;
     if (ext > 0) v = (int)((grid[i * 3 + d] - lo) / ext * cells);
     c[d] = (unsigned)min(max(v, 0), cells - 1);
   }
   keys[i] = (int)((spread3(c[0]) << 2) | (spread3(c[1]) << 1) | spread3(c[2]));
 }
-__global__ __launch_bounds__(256) void morton_keys(const double* grid, long n, const double* box, int cells,
+__global__ __launch_bounds__(256) void morton_keys(const double* grid, long n, const double* part, int nb, int cells,
                                                    int* keys) {
-  morton_keys_b(grid, n, box, cells, keys, (int)blockIdx.x, (int)gridDim.x);
+  morton_keys_b(grid, n, part, nb, cells, keys, (int)blockIdx.x);
 }
 
-__device__ __forceinline__ void gather_sorted_b(const double* grid, const int* perm, long n, double* sx,
-                                                     double* sy, double* sz, int bid, int nblk) {
-  const long p = bid * 256L + threadIdx.x;
-  if (p >= n) return;
-  const long i = perm[p];
-  sx[p] = grid[i * 3 + 0];
-  sy[p] = grid[i * 3 + 1];
-  sz[p] = grid[i * 3 + 2];
-}
-__global__ __launch_bounds__(256) void gather_sorted(const double* grid, const int* perm, long n, double* sx,
-                                                     double* sy, double* sz) {
-  gather_sorted_b(grid, perm, n, sx, sy, sz, (int)blockIdx.x, (int)gridDim.x);
-}
-
-__device__ __forceinline__ void tile_boxes_b(const double* sx, const double* sy, const double* sz, long n,
-                                                  double* boxes, int bid, int nblk) {
+// The sorted coordinates, the bounding box of each tile of TP of them and
+// those of its four runs of 64 (one wave of the assignment each).
+__device__ __forceinline__ void sorted_tiles_b(const double* grid, const int* perm, long n, double* sx, double* sy,
+                                                    double* sz, double* boxes, double* wboxes, int bid) {
   const long p = bid * (long)TP + threadIdx.x;
-  double v[3];
+  double v[3] = {0, 0, 0};
   const bool ok = p < n;
-  v[0] = ok ? sx[p] : 0;
-  v[1] = ok ? sy[p] : 0;
-  v[2] = ok ? sz[p] : 0;
+  if (ok) {
+    const long i = perm[p];
+    for (int d = 0; d < 3; ++d) v[d] = grid[i * 3 + d];
+    sx[p] = v[0];
+    sy[p] = v[1];
+    sz[p] = v[2];
+  }
   __shared__ double s[6][4];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   for (int d = 0; d < 3; ++d) {
-    double a = wave_min(ok ? v[d] : DBL_MAX), b = -wave_min(ok ? -v[d] : DBL_MAX);
+    const double a = wave_min(ok ? v[d] : DBL_MAX), b = -wave_min(ok ? -v[d] : DBL_MAX);
     if (lane == 0) { s[d][w] = a; s[3 + d][w] = b; }
   }
   __syncthreads();
@@ -169,47 +233,46 @@ __device__ __forceinline__ void tile_boxes_b(const double* sx, const double* sy,
     for (int q = 1; q < 4; ++q) r = d < 3 ? fmin(r, s[d][q]) : fmax(r, s[d][q]);
     boxes[bid * 6 + d] = r;
   }
+  if (threadIdx.x < 24) wboxes[bid * 24L + threadIdx.x] = s[threadIdx.x % 6][threadIdx.x / 6];
 }
-__global__ __launch_bounds__(256) void tile_boxes(const double* sx, const double* sy, const double* sz, long n,
-                                                  double* boxes) {
-  tile_boxes_b(sx, sy, sz, n, boxes, (int)blockIdx.x, (int)gridDim.x);
+__global__ __launch_bounds__(256) void sorted_tiles(const double* grid, const int* perm, long n, double* sx, double* sy,
+                                                    double* sz, double* boxes, double* wboxes) {
+  sorted_tiles_b(grid, perm, n, sx, sy, sz, boxes, wboxes, (int)blockIdx.x);
 }
 
-__device__ __forceinline__ void init_centroids_b(const double* grid, const int* idx, int k, double* cen, int bid, int nblk) {
+// Start of a run: the loop state, the starting centroids, empty buckets and
+// change counts.
+__device__ __forceinline__ void init_run_b(const double* grid, const int* idx, int k, double* cen, int* cnt, int* chg,
+                                                int nchg, State* st, int bid, int nblk) {
   const int j = bid * 256 + threadIdx.x;
+  for (int i = j; i < nchg; i += nblk * 256) chg[i] = 0;
+  if (j == 0) {
+    st->done = 0;
+    st->final_buf = 0;
+    st->error = 0;
+    st->bad = INT_MAX;
+    st->iters = 0;
+    st->mode = MODE_LATEST;
+    st->dups = 0;
+    st->last_diff = 0.0;
+  }
   if (j >= k) return;
+  if (cnt) cnt[j] = 0;
+  if (!idx) return;
   const long i = idx[j];
   cen[j * 3 + 0] = grid[i * 3 + 0];
   cen[j * 3 + 1] = grid[i * 3 + 1];
   cen[j * 3 + 2] = grid[i * 3 + 2];
 }
-__global__ __launch_bounds__(256) void init_centroids(const double* grid, const int* idx, int k, double* cen) {
-  init_centroids_b(grid, idx, k, cen, (int)blockIdx.x, (int)gridDim.x);
+__global__ __launch_bounds__(256) void init_run(const double* grid, const int* idx, int k, double* cen, int* cnt,
+                                                int* chg, int nchg, State* st) {
+  init_run_b(grid, idx, k, cen, cnt, chg, nchg, st, (int)blockIdx.x, (int)gridDim.x);
 }
 
-__device__ __forceinline__ void init_state_b(State* st, int mode, int bid, int nblk) {
-  if (threadIdx.x == 0) {
-    st->done = 0;
-    st->final_buf = 0;
-    st->error = 0;
-    st->changed[0] = st->changed[1] = 0;
-    st->serr[0] = st->serr[1] = 0;
-    st->iters = 0;
-    st->mode = mode;
-    st->dups = 0;
-    st->last_diff = 0.0;
-  }
-}
-__global__ void init_state(State* st, int mode) {
-  init_state_b(st, mode, (int)blockIdx.x, (int)gridDim.x);
-}
-
-// ------------------------------------------------------------------ stable counting sort
+// ------------------------------------------------------------------ stable counting sort (Morton cells)
 
 // Per index-order tile of CS_TILE points: histogram of keys.
-__device__ __forceinline__ void cs_hist_b(const int* keys, long n, int nbins, int* tile_count,
-                                               const State* st, int bid, int nblk) {
-  if (st && st->done) return;
+__device__ __forceinline__ void cs_hist_b(const int* keys, long n, int nbins, int* tile_count, int bid, int nblk) {
   __shared__ int h[MAXB];
   for (int b = threadIdx.x; b < nbins; b += 256) h[b] = 0;
   __syncthreads();
@@ -225,9 +288,8 @@ __device__ __forceinline__ void cs_hist_b(const int* keys, long n, int nbins, in
   int* out = tile_count + (long)bid * nbins;
   for (int b = threadIdx.x; b < nbins; b += 256) out[b] = h[b];
 }
-__global__ __launch_bounds__(256) void cs_hist(const int* keys, long n, int nbins, int* tile_count,
-                                               const State* st) {
-  cs_hist_b(keys, n, nbins, tile_count, st, (int)blockIdx.x, (int)gridDim.x);
+__global__ __launch_bounds__(256) void cs_hist(const int* keys, long n, int nbins, int* tile_count) {
+  cs_hist_b(keys, n, nbins, tile_count, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // Column scan over tiles, in place: tile_count[t][b] -> exclusive offset of
@@ -235,9 +297,7 @@ __global__ __launch_bounds__(256) void cs_hist(const int* keys, long n, int nbin
 // its CS_SCAN_W waves scan consecutive runs of the tiles, then add the earlier
 // runs' totals (16 waves: two dependent load rounds per wave at 256 tiles,
 // where 4 waves needed eight).
-__device__ __forceinline__ void cs_colscan_b(int* tile_count, int ntiles, int nbins, int* total,
-                                                  const State* st, int bid, int nblk) {
-  if (st && st->done) return;
+__device__ __forceinline__ void cs_colscan_b(int* tile_count, int ntiles, int nbins, int* total, int bid, int nblk) {
   __shared__ int part[CS_SCAN_W][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int b = bid * 64 + lane;
@@ -275,14 +335,12 @@ __device__ __forceinline__ void cs_colscan_b(int* tile_count, int ntiles, int nb
     if (wave == CS_SCAN_W - 1) total[b] = off;
   }
 }
-__global__ __launch_bounds__(64 * CS_SCAN_W) void cs_colscan(int* tile_count, int ntiles, int nbins, int* total,
-                                                  const State* st) {
-  cs_colscan_b(tile_count, ntiles, nbins, total, st, (int)blockIdx.x, (int)gridDim.x);
+__global__ __launch_bounds__(64 * CS_SCAN_W) void cs_colscan(int* tile_count, int ntiles, int nbins, int* total) {
+  cs_colscan_b(tile_count, ntiles, nbins, total, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // Exclusive scan of total[0..nbins) into start (one workgroup of 1024).
-__device__ __forceinline__ void cs_totscan_b(const int* total, int nbins, int* start, const State* st, int bid, int nblk) {
-  if (st && st->done) return;
+__device__ __forceinline__ void cs_totscan_b(const int* total, int nbins, int* start, int bid, int nblk) {
   __shared__ int s[1024];
   const int t = threadIdx.x;
   const int per = (nbins + 1023) / 1024;
@@ -308,8 +366,8 @@ __device__ __forceinline__ void cs_totscan_b(const int* total, int nbins, int* s
     }
   }
 }
-__global__ __launch_bounds__(1024) void cs_totscan(const int* total, int nbins, int* start, const State* st) {
-  cs_totscan_b(total, nbins, start, st, (int)blockIdx.x, (int)gridDim.x);
+__global__ __launch_bounds__(1024) void cs_totscan(const int* total, int nbins, int* start) {
+  cs_totscan_b(total, nbins, start, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // Stable scatter: out[start[key] + rank] = index, rank counting earlier
@@ -317,9 +375,7 @@ __global__ __launch_bounds__(1024) void cs_totscan(const int* total, int nbins, 
 // four waves go in order; inside a wave, lanes with equal keys are ranked by
 // lane through a 'nbits'-ballot match.
 __device__ __forceinline__ void cs_scatter_b(const int* keys, long n, int nbins, int nbits,
-                                                  const int* tile_off, const int* start, int* out,
-                                                  const State* st, int bid, int nblk) {
-  if (st && st->done) return;
+                                                  const int* tile_off, const int* start, int* out, int bid, int nblk) {
   __shared__ int cnt[MAXB];
   __shared__ int slot[256];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -354,29 +410,69 @@ __device__ __forceinline__ void cs_scatter_b(const int* keys, long n, int nbins,
   }
 }
 __global__ __launch_bounds__(256) void cs_scatter(const int* keys, long n, int nbins, int nbits,
-                                                  const int* tile_off, const int* start, int* out,
-                                                  const State* st) {
-  cs_scatter_b(keys, n, nbins, nbits, tile_off, start, out, st, (int)blockIdx.x, (int)gridDim.x);
+                                                  const int* tile_off, const int* start, int* out) {
+  cs_scatter_b(keys, n, nbins, nbits, tile_off, start, out, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ------------------------------------------------------------------ Lloyd iteration
 
+// Nearest centroid of the TP points of one tile.
+//
+// Centroids whose distance bound to the tile's box exceeds the best upper
+// bound are dropped; the others (about 40 at 256 points a cluster) are listed
+// in ascending index.  Every wave drops those that its own 64 points' box
+// excludes (about a third is left), and its points scan the rest.  The winner is the first
+// index of the smallest rounded distance, but the scan compares squares: one
+// below the best by a relative 2^-50 has a strictly smaller rounded root (the
+// roots differ by more than 2^-52, two roundings by less), one not below the
+// best has no smaller root, and only a group of candidates with a square in
+// between takes the roots themselves.  N = 262144, K = 1024: 14 us, 4 of them
+// the buckets, most of it latency (four waves a SIMD, each a chain of some ten
+// loads, reductions and barriers).  With a root whenever any lane improved and
+// the whole list for every wave it took 38 us.
+//
+// With buckets (cnt, bucket) the points of a cluster are also listed for
+// centroid_sums, cap of them at most, in any order: one device atomic per tile
+// and cluster that has points there.
+constexpr double SURE = 1.0 + 0x1p-49;
+
+//
+// CPT: centroids a thread looks at (k <= 256 CPT); the smallest that holds k
+// keeps the unrolled loops, their registers and the list short (K = 1024:
+// 18 us with 16 for every k).
+template <int CPT>
 __device__ __forceinline__ void assign_b(const double* sx, const double* sy, const double* sz,
-                                              const int* perm, long n, const double* boxes,
+                                              const int* perm, long n, const double* boxes, const double* wboxes,
                                               const double* cen, int k, int* map_new, const int* map_old,
-                                              State* st, int par, int bid, int nblk) {
-  if (st && st->done) return;
-  __shared__ int cidx[MAXB];
+                                              int* cnt, int* bucket, int cap, int* chg, const State* st, int it,
+                                              int bid) {
+  if (st && (st->done || st->bad < it)) return;
+  __shared__ int cidx[256 * CPT];
   __shared__ double ccx[CAND_CAP], ccy[CAND_CAP], ccz[CAND_CAP];
+  __shared__ int lcnt[CAND_CAP], lbase[CAND_CAP];
   __shared__ double redd[4];
-  __shared__ int redi[4];
+  __shared__ int redi[64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const double* b = boxes + (long)bid * 6;
-  double box[6];
-  for (int d = 0; d < 6; ++d) box[d] = b[d];
+  double box[6], wbox[6];
+  for (int d = 0; d < 6; ++d) {
+    box[d] = b[d];
+    wbox[d] = wboxes[((long)bid * 4 + wave) * 6 + d];
+  }
+  const long p = (long)bid * TP + tid;
+  const bool live = p < n;
+  double gx = 0.0, gy = 0.0, gz = 0.0;
+  int orig = 0, old = -1;
+  if (live) {
+    gx = sx[p];
+    gy = sy[p];
+    gz = sz[p];
+    orig = perm[p];
+    if (map_old) old = map_old[p];
+  }
 
-  // this thread's centroids j = q * 256 + tid (k <= MAXB), loaded once
-  constexpr int CPT = MAXB / 256;
+  // this thread's centroids j = q * 256 + tid, loaded once
+  static_assert(CPT * 4 <= 64, "one count per lane in the scan of the lists");
   double rx[CPT], ry[CPT], rz[CPT];
 #pragma unroll
   for (int q = 0; q < CPT; ++q) {
@@ -392,148 +488,340 @@ __device__ __forceinline__ void assign_b(const double* sx, const double* sy, con
     if (q * 256 + tid < k) u = fmin(u, ub2_box(rx[q], ry[q], rz[q], box));
   u = wave_min(u);
   if (lane == 0) redd[wave] = u;
+  for (int c = tid; c < CAND_CAP; c += TP) lcnt[c] = 0;
   __syncthreads();
   u = fmin(fmin(redd[0], redd[1]), fmin(redd[2], redd[3]));
   const double thr = u * PRUNE;
 
-  int ncand = 0;
+  // ascending list: counts per (q, wave), one scan of the 64 counts, one store
+  unsigned flags = 0;
 #pragma unroll
   for (int q = 0; q < CPT; ++q) {
-    if (q * 256 >= k) break;  // uniform over the workgroup
-    const int j = q * 256 + tid;
-    const double cx = rx[q], cy = ry[q], cz = rz[q];
-    const bool flag = j < k && lb2_box(cx, cy, cz, box) <= thr;
-    const unsigned long long bal = __ballot(flag);
-    __syncthreads();
-    if (lane == 0) redi[wave] = __popcll(bal);
-    __syncthreads();
-    int off = ncand;
-    for (int w = 0; w < wave; ++w) off += redi[w];
-    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    off += __popcll(bal & below);
-    if (flag) {
-      cidx[off] = j;
-      if (off < CAND_CAP) { ccx[off] = cx; ccy[off] = cy; ccz[off] = cz; }
+    int have = 0;
+    if (q * 256 < k) {  // uniform over the workgroup
+      const bool flag = q * 256 + tid < k && lb2_box(rx[q], ry[q], rz[q], box) <= thr;
+      flags |= flag ? 1u << q : 0u;
+      have = __popcll(__ballot(flag));
     }
-    ncand += redi[0] + redi[1] + redi[2] + redi[3];
+    if (lane == 0) redi[q * 4 + wave] = have;
+  }
+  __syncthreads();
+  const int mine = lane < CPT * 4 ? redi[lane] : 0, upto = wave_scan(mine);
+  const int ncand = __builtin_amdgcn_readlane(upto, 63);
+#pragma unroll
+  for (int q = 0; q < CPT; ++q) {
+    if (q * 256 >= k) break;
+    const bool flag = (flags >> q) & 1;
+    const unsigned long long bal = __ballot(flag);
+    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const int off = __builtin_amdgcn_readlane(upto - mine, q * 4 + wave) + __popcll(bal & below);
+    if (flag) {
+      cidx[off] = q * 256 + tid;
+      if (off < CAND_CAP) { ccx[off] = rx[q]; ccy[off] = ry[q]; ccz[off] = rz[q]; }
+    }
   }
   __syncthreads();
 
-  const long p = (long)bid * TP + tid;
-  int changed = 0;
-  if (p < n) {
-    const double gx = sx[p], gy = sy[p], gz = sz[p];
-    // ascending candidate order: only a strictly smaller rounded distance wins
-    int bj = cidx[0];
-    double bd2 = dist2(ccx[0], ccy[0], ccz[0], gx, gy, gz);
-    double bs = sqrt(bd2);
-    // eight candidates' distances at a time (their LDS reads in flight
-    // together), then the updates in ascending order as one by one
-    constexpr int U = 8;
-    const int cached = min(ncand, CAND_CAP);
-    int c = 1;
-    for (; c + U <= cached; c += U) {
+  // this wave's own bound over the listed candidates
+  const int cached = min(ncand, CAND_CAP);
+  double wu = DBL_MAX;
+  for (int c = lane; c < cached; c += 64) wu = fmin(wu, ub2_box(ccx[c], ccy[c], ccz[c], wbox));
+  const double wthr = wave_min(wu) * PRUNE;
+
+  // best candidate so far, by position in the list
+  int bc = 0;
+  double bd2 = 0.0;
+  bool first = true;
+  auto rooted = [&](double d2, int c) {  // the rule on rounded distances itself
+    if (d2 < bd2 && sqrt(d2) < sqrt(bd2)) {
+      bd2 = d2;
+      bc = c;
+    }
+  };
+  // eight candidates' distances at a time (their LDS reads in flight together);
+  // the last group repeats its last candidate, which changes nothing
+  constexpr int U = 8;
+  for (int c0 = 0; c0 < cached; c0 += 64) {
+    const int cl = c0 + lane;
+    unsigned long long left =
+        __ballot(cl < cached && lb2_box(ccx[cl & (CAND_CAP - 1)], ccy[cl & (CAND_CAP - 1)], ccz[cl & (CAND_CAP - 1)], wbox) <= wthr);
+    while (left) {
+      int at[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        at[q] = left ? c0 + __ffsll((long long)left) - 1 : at[q > 0 ? q - 1 : 0];
+        left &= left - 1;
+      }
       double d2v[U];
-      int jv[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) d2v[q] = dist2(ccx[at[q]], ccy[at[q]], ccz[at[q]], gx, gy, gz);
+      if (first) {
+        bd2 = d2v[0];
+        bc = at[0];
+        first = false;
+      }
+      double nd2 = bd2;
+      int nc = bc;
+      bool close = false;
 #pragma unroll
       for (int q = 0; q < U; ++q) {
-        jv[q] = cidx[c + q];
-        d2v[q] = dist2(ccx[c + q], ccy[c + q], ccz[c + q], gx, gy, gz);
+        const bool sure = d2v[q] * SURE <= nd2 && d2v[q] < nd2;
+        close |= d2v[q] < nd2 && !sure;
+        nd2 = sure ? d2v[q] : nd2;
+        nc = sure ? at[q] : nc;
       }
+      if (close) {
 #pragma unroll
-      for (int q = 0; q < U; ++q) {
-        if (d2v[q] < bd2) {
-          const double sq = sqrt(d2v[q]);
-          if (sq < bs) { bs = sq; bd2 = d2v[q]; bj = jv[q]; }
-        }
+        for (int q = 0; q < U; ++q) rooted(d2v[q], at[q]);
+      } else {
+        bd2 = nd2;
+        bc = nc;
       }
     }
-    for (; c < ncand; ++c) {
-      double cx, cy, cz;
-      const int j = cidx[c];
-      if (c < CAND_CAP) { cx = ccx[c]; cy = ccy[c]; cz = ccz[c]; }
-      else { cx = cen[j * 3]; cy = cen[j * 3 + 1]; cz = cen[j * 3 + 2]; }
-      const double d2 = dist2(cx, cy, cz, gx, gy, gz);
-      if (d2 < bd2) {
-        const double s = sqrt(d2);
-        if (s < bs) { bs = s; bd2 = d2; bj = j; }
-      }
-    }
-    const long orig = perm[p];
-    if (map_old) changed = (map_old[orig] != bj);
-    map_new[orig] = bj;
   }
-  if (st && map_old) {
-    changed = wave_sum(changed);
-    if (lane == 0 && changed) atomicAdd(&st->changed[par], changed);
+  if (first) bd2 = dist2(ccx[0], ccy[0], ccz[0], gx, gy, gz);
+  int c = cached;
+  for (; c < ncand; ++c) {
+    double cx, cy, cz;
+    if (c < CAND_CAP) { cx = ccx[c]; cy = ccy[c]; cz = ccz[c]; }
+    else { const int j = cidx[c]; cx = cen[j * 3]; cy = cen[j * 3 + 1]; cz = cen[j * 3 + 2]; }
+    rooted(dist2(cx, cy, cz, gx, gy, gz), c);
+  }
+  const int bj = cidx[bc];
+  if (!bucket) {  // one classification: the map in grid order
+    if (live) map_new[orig] = bj;
+    return;
+  }
+  int rank = 0;
+  if (live) {
+    map_new[p] = bj;
+    if (bc < CAND_CAP) rank = atomicAdd(&lcnt[bc], 1);
+  }
+  const int changed = wave_sum(live && map_old && old != bj ? 1 : 0);
+  if (lane == 0) redi[wave] = changed;
+  __syncthreads();
+  for (int q = tid; q < cached; q += TP) {
+    const int m = lcnt[q];
+    if (m) lbase[q] = atomicAdd(&cnt[cidx[q]], m);
+  }
+  if (tid == 0 && map_old) {
+    const int sum = redi[0] + redi[1] + redi[2] + redi[3];
+    if (sum) atomicAdd(&chg[bid % CHG], sum);
+  }
+  __syncthreads();
+  if (live) {
+    const int at = bc < CAND_CAP ? lbase[bc] + rank : atomicAdd(&cnt[bj], 1);
+    if (at < cap) bucket[(long)bj * cap + at] = orig;
   }
 }
+template <int CPT>
 __global__ __launch_bounds__(256) void assign(const double* sx, const double* sy, const double* sz,
-                                              const int* perm, long n, const double* boxes,
-                                              const double* cen, int k, int* map_new, const int* map_old,
-                                              State* st, int par) {
-  assign_b(sx, sy, sz, perm, n, boxes, cen, k, map_new, map_old, st, par, (int)blockIdx.x, (int)gridDim.x);
+                                              const int* perm, long n, const double* boxes, const double* wboxes,
+                                              const double* cen, int k, int* map_new, const int* map_old, int* cnt,
+                                              int* bucket, int cap, int* chg, const State* st, int it) {
+  assign_b<CPT>(sx, sy, sz, perm, n, boxes, wboxes, cen, k, map_new, map_old, cnt, bucket, cap, chg, st, it,
+                (int)blockIdx.x);
 }
 
-// One wave per cluster.  Lanes gather the members' rho and rho * x (each
-// product rounded on its own, as the reference's multiply-then-add does) into
-// LDS in ascending index order, then lanes 0..3 each run one of the four
-// sequential sums (w, x, y, z) over them.
-constexpr int CS_CHUNK = 256;
+// Buckets of an assignment given in grid order.
+__global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k, int* cnt, int* bucket, int cap) {
+  const long i = blockIdx.x * 256L + threadIdx.x;
+  if (i >= n) return;
+  const int key = map[i];
+  if ((unsigned)key >= (unsigned)k) return;
+  const int at = atomicAdd(&cnt[key], 1);
+  if (at < cap) bucket[(long)key * cap + at] = (int)i;
+}
 
-__device__ __forceinline__ void centroid_sums_b(const int* order, const int* start, const int* total,
-                                                     const double* rho, const double* grid, int k,
-                                                     double* cen_out, State* st, int par, int bid, int nblk) {
-  if (st && st->done) return;
-  __shared__ double buf[4][4][CS_CHUNK];  // [wave][w, x, y, z][member]
+// Weighted centroid of one cluster per workgroup, its members' rho and rho * x
+// (each product rounded on its own, as the reference's multiply-then-add does)
+// summed in ascending grid index.
+//
+// The bucket holds the members in no order.  They are set as bits of a window
+// of the index range (64 Ki points: a cluster of a few hundred points spans
+// less on a 64^3 grid), a scan of the words' bit counts gives every member its
+// rank, the values go to LDS by rank, and lanes 0..3 run the four sequential
+// sums.  Up to SB_R members a thread stay in registers, their values on the
+// way while the bits are counted; larger clusters, and index ranges wider than
+// the window, take the general passes, and a cluster with more members than
+// its bucket holds reads them from the whole map (perm: the map's order, null:
+// grid order).
+//
+// Bound by latency: two dependent loads and the chain of adds (about 9 ns
+// each).  N = 262144, K = 1024: 13 us, where the stable counting sort and the
+// sums that this replaces were five kernels of 40 us.
+constexpr int SB_W = 2048;  // words of the window
+constexpr int SB_M = 512;   // members summed at a time
+constexpr int SB_R = 4;     // members a thread of the register path
+
+struct SumsLds {
+  unsigned bm[SB_W];
+  unsigned short pre[SB_W];                            // members before a word (register path)
+  int list[SB_M];                                      // members in order (general passes)
+  __attribute__((aligned(16))) double buf[4][SB_M + 2];  // [w, x, y, z][member], rows on different banks
+  int red[4], red2[4];
+};
+
+// Members before this thread's words wb .. we - 1 of the window, and in all.
+__device__ inline void sums_rank(SumsLds& S, int wb, int we, int& pos, int& total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = bid * 4 + wave;
-  if (c >= k) return;
-  const int s = start[c], cnt = total[c];
-  double acc = 0.0;  // lane q < 4 owns accumulator q
-  for (int base = 0; base < cnt; base += CS_CHUNK) {
-    const int len = min(CS_CHUNK, cnt - base);
-    for (int t = lane; t < len; t += 64) {
-      const long i = order[s + base + t];
-      const double r = rho[i];
-      buf[wave][0][t] = r;
-      buf[wave][1][t] = r * grid[i * 3 + 0];
-      buf[wave][2][t] = r * grid[i * 3 + 1];
-      buf[wave][3][t] = r * grid[i * 3 + 2];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    if (lane < 4) {
-      const double* v = buf[wave][lane];
-      for (int t = 0; t < len; ++t) acc += v[t];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  int have = 0;
+  for (int w = wb; w < we; ++w) have += __popc(S.bm[w]);
+  const int upto = wave_scan(have);
+  if (lane == 63) S.red[wave] = upto;
+  __syncthreads();
+  pos = upto - have;
+  total = 0;
+  for (int w = 0; w < 4; ++w) {
+    if (w < wave) pos += S.red[w];
+    total += S.red[w];
   }
+}
+
+__device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int cap, const int* map, const int* perm,
+                                                     long n, const double* rho, const double* grid, double* cen_out,
+                                                     State* st, int it, int c) {
+  __shared__ SumsLds S;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int* mem = bucket + (long)c * cap;
+  int i[SB_R];
+#pragma unroll
+  for (int u = 0; u < SB_R; ++u) i[u] = tid + 256 * u < cap ? mem[tid + 256 * u] : 0;  // before the count is known
+  const int m = cnt[c];
+  if (st->done || st->bad < it) return;
+  const bool listed = m <= cap;
+  int lo = INT_MAX, hi = INT_MAX;  // hi negated: both are minima
+  double v[SB_R][4];
+  const bool few = listed && m <= 256 * SB_R;
+  if (few) {
+#pragma unroll
+    for (int u = 0; u < SB_R; ++u)
+      if (tid + 256 * u < m) {
+        lo = min(lo, i[u]);
+        hi = min(hi, -i[u]);
+        v[u][0] = rho[i[u]];
+        for (int d = 0; d < 3; ++d) v[u][1 + d] = grid[i[u] * 3L + d];
+      }
+  }
+  // every member: f(grid index)
+  auto members = [&](auto f) {
+    if (listed) {
+      for (int t = tid; t < m; t += 256) f(mem[t]);
+    } else {
+      for (long p = tid; p < n; p += 256)
+        if (map[p] == c) f(perm ? perm[p] : (int)p);
+    }
+  };
+  if (!few)
+    members([&](int e) {
+      lo = min(lo, e);
+      hi = min(hi, -e);
+    });
+  lo = wave_min(lo);
+  hi = wave_min(hi);
+  if (lane == 0) { S.red[wave] = lo; S.red2[wave] = hi; }
+  for (int w = tid; w < SB_W; w += 256) S.bm[w] = 0;
+  __syncthreads();
+  lo = min(min(S.red[0], S.red[1]), min(S.red[2], S.red[3])) & ~31;
+  hi = -min(min(S.red2[0], S.red2[1]), min(S.red2[2], S.red2[3]));
+  double acc = 0.0;  // lane q < 4 of wave 0 owns accumulator q
+  if (few && m > 0 && hi - lo < SB_W * 32) {
+    const int per = ((hi - lo) >> 13) + 1, wb = tid * per;  // words a thread, all inside the window
+#pragma unroll
+    for (int u = 0; u < SB_R; ++u)
+      if (tid + 256 * u < m) atomicOr(&S.bm[(i[u] - lo) >> 5], 1u << (i[u] & 31));
+    __syncthreads();
+    int pos, total;
+    sums_rank(S, wb, wb + per, pos, total);
+    for (int w = wb; w < wb + per; ++w) {
+      S.pre[w] = (unsigned short)pos;
+      pos += __popc(S.bm[w]);
+    }
+    __syncthreads();
+    for (int base = 0; base < m; base += SB_M) {
+#pragma unroll
+      for (int u = 0; u < SB_R; ++u)
+        if (tid + 256 * u < m) {
+          const int w = (i[u] - lo) >> 5;
+          const int r = S.pre[w] + __popc(S.bm[w] & ((1u << (i[u] & 31)) - 1)) - base;
+          if (r >= 0 && r < SB_M) {
+            S.buf[0][r] = v[u][0];
+            for (int d = 0; d < 3; ++d) S.buf[1 + d][r] = v[u][0] * v[u][1 + d];
+          }
+        }
+      __syncthreads();
+      if (tid < 4) acc = seq_sum(acc, S.buf[tid], min(SB_M, m - base));
+      if (base + SB_M < m) __syncthreads();
+    }
+  } else {
+    for (long w0 = lo; m > 0 && w0 <= hi; w0 += SB_W * 32L) {
+      const int nw = (int)min((long)SB_W, ((hi - w0) >> 5) + 1);
+      if (w0 > lo) {
+        for (int w = tid; w < nw; w += 256) S.bm[w] = 0;
+        __syncthreads();
+      }
+      members([&](int e) {
+        const long o = e - w0;
+        if (o >= 0 && o < SB_W * 32L) atomicOr(&S.bm[o >> 5], 1u << (o & 31));
+      });
+      __syncthreads();
+      const int per = (nw + 255) / 256, wb = min(nw, tid * per), we = min(nw, wb + per);
+      int pos, total;
+      sums_rank(S, wb, we, pos, total);
+      for (int base = 0; base < total; base += SB_M) {
+        int q = pos - base;
+        for (int w = wb; w < we; ++w)
+          for (unsigned bits = S.bm[w]; bits; bits &= bits - 1, ++q)
+            if (q >= 0 && q < SB_M) S.list[q] = (int)(w0 + 32 * w) + __ffs(bits) - 1;
+        __syncthreads();
+        const int len = min(SB_M, total - base);
+        for (int t = tid; t < len; t += 256) {
+          const long e = S.list[t];
+          const double r = rho[e];
+          S.buf[0][t] = r;
+          for (int d = 0; d < 3; ++d) S.buf[1 + d][t] = r * grid[e * 3 + d];
+        }
+        __syncthreads();
+        if (tid < 4) acc = seq_sum(acc, S.buf[tid], len);
+        __syncthreads();
+      }
+      __syncthreads();  // an empty window: its counts are read before they are cleared
+    }
+  }
+  if (tid >= 64) return;
   const double w = __shfl(acc, 0);
-  if (lane == 0 && w < 1e-8) atomicOr(&st->serr[par], 1);
+  if (lane == 0) {
+    cnt[c] = 0;  // empty for the next assignment
+    if (w < 1e-8) atomicMin(&st->bad, it);
+  }
   if (lane >= 1 && lane < 4) cen_out[c * 3 + lane - 1] = acc / w;
 }
-__global__ __launch_bounds__(256) void centroid_sums(const int* order, const int* start, const int* total,
-                                                     const double* rho, const double* grid, int k,
-                                                     double* cen_out, State* st, int par) {
-  centroid_sums_b(order, start, total, rho, grid, k, cen_out, st, par, (int)blockIdx.x, (int)gridDim.x);
+__global__ __launch_bounds__(256) void centroid_sums(int* cnt, const int* bucket, int cap, const int* map,
+                                                     const int* perm, long n, const double* rho, const double* grid,
+                                                     double* cen_out, State* st, int it) {
+  centroid_sums_b(cnt, bucket, cap, map, perm, n, rho, grid, cen_out, st, it, (int)blockIdx.x);
 }
 
 // normed_difference(new, cur) with the reference's sequential sum, % changed,
-// and the loop control of KMeansSolver::kernel (kmeans.cpp:233-257).
+// and the loop control of KMeansSolver::kernel (kmeans.cpp:233-257).  chg: the
+// iteration's CHG partial change counts.  Where the threshold cannot stop the
+// loop (Layout::defer) every iteration's is run after the loop, side by side.
 __device__ __forceinline__ void diff_control_b(const double* nxt, const double* cur, int k, long n,
                                                      double threshold, int it, int max_it, int nxt_buf,
-                                                     State* st, double* diffs, double* pcts, int bid, int nblk) {
-  if (st->done) return;
-  extern __shared__ double terms[];
+                                                     State* st, int* chg, double* diffs, double* pcts,
+                                                     bool defer) {
+  if (!defer && st->done) return;
+  extern __shared__ __attribute__((aligned(16))) double terms[];
   __shared__ double red[4][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int len = 3 * k, par = it & 1;
-  if (st->serr[par]) {
-    if (tid == 0) { st->error = 1; st->done = 1; st->iters = it + 1; }
+  const int len = 3 * k;
+  const int bad = st->bad;
+  if (bad <= it) {
+    if (bad == it && tid == 0) {
+      st->error = 1;
+      st->iters = it + 1;
+      if (!defer) st->done = 1;
+    }
     return;
   }
   double mxa = -DBL_MAX, mna = DBL_MAX, mxb = -DBL_MAX, mnb = DBL_MAX;
@@ -555,40 +843,16 @@ __device__ __forceinline__ void diff_control_b(const double* nxt, const double* 
     terms[i] = t * t;
   }
   __syncthreads();
-  if (tid == 0) {
-    // strictly left-to-right sum (the reference's order), with the LDS reads
-    // of the next 16 terms issued before the adds of the current 16
-    double acc = 0.0;
-    const int nb = len / 16;
-    double a[16], c[16];
-    if (nb > 0) {
-#pragma unroll
-      for (int q = 0; q < 16; ++q) a[q] = terms[q];
-    }
-    for (int bi = 0; bi < nb; bi += 2) {
-      const bool more = bi + 1 < nb;
-      if (more) {
-#pragma unroll
-        for (int q = 0; q < 16; ++q) c[q] = terms[(bi + 1) * 16 + q];
-      }
-#pragma unroll
-      for (int q = 0; q < 16; ++q) acc += a[q];
-      if (!more) break;
-      if (bi + 2 < nb) {
-#pragma unroll
-        for (int q = 0; q < 16; ++q) a[q] = terms[(bi + 2) * 16 + q];
-      }
-#pragma unroll
-      for (int q = 0; q < 16; ++q) acc += c[q];
-    }
-    for (int i = nb * 16; i < len; ++i) acc += terms[i];
-    const double diff = scale * sqrt(acc);
-    const double pct = 100 * ((double)st->changed[par]) / (double)n;
+  if (wave > 0) return;
+  const int changed = wave_sum(lane < CHG ? chg[lane] : 0);
+  if (!defer && lane < CHG) chg[lane] = 0;
+  if (lane == 0) {
+    const double diff = scale * sqrt(seq_sum(0.0, terms, len));  // the reference's order
+    const double pct = 100 * ((double)changed) / (double)n;
     diffs[it] = diff;
     pcts[it] = pct;
-    st->iters = it + 1;
-    st->last_diff = diff;
-    st->changed[par] = 0;  // the next iteration of this parity waits for this kernel
+    if (!defer || it == max_it - 1) st->iters = it + 1;
+    if (!defer || it == max_it - 1 || bad == it + 1) st->last_diff = diff;
     if (diff < threshold) {
       st->done = 1;
       st->mode = MODE_FINAL;
@@ -600,8 +864,16 @@ __device__ __forceinline__ void diff_control_b(const double* nxt, const double* 
 }
 __global__ __launch_bounds__(1024) void diff_control(const double* nxt, const double* cur, int k, long n,
                                                      double threshold, int it, int max_it, int nxt_buf,
-                                                     State* st, double* diffs, double* pcts) {
-  diff_control_b(nxt, cur, k, n, threshold, it, max_it, nxt_buf, st, diffs, pcts, (int)blockIdx.x, (int)gridDim.x);
+                                                     State* st, int* chg, double* diffs, double* pcts) {
+  diff_control_b(nxt, cur, k, n, threshold, it, max_it, nxt_buf, st, chg, diffs, pcts, false);
+}
+// all iterations of a run that kept every iteration's centroids
+__global__ __launch_bounds__(1024) void diff_control_all(const double* cen, int k, long n, double threshold, int max_it,
+                                                         State* st, int* chg, double* diffs, double* pcts) {
+  const int it = (int)blockIdx.x;
+  const long cs = 3L * k;
+  diff_control_b(cen + (it + 1) * cs, cen + it * cs, k, n, threshold, it, max_it, it + 1, st, chg + it * CHG, diffs,
+                 pcts, true);
 }
 
 // ------------------------------------------------------------------ map_to_grid
@@ -611,11 +883,11 @@ __global__ __launch_bounds__(1024) void diff_control(const double* nxt, const do
 __device__ __forceinline__ void map_to_grid_b(const double* sx, const double* sy, const double* sz,
                                                    const int* perm, long n, const double* boxes, int ntiles,
                                                    const double* cen3, long cstride, int latest_buf,
-                                                   const State* st, int* out, int bid, int nblk) {
+                                                   const State* st, int* out, int bid) {
   const int c = bid;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int mode = st ? st->mode : MODE_LATEST;
-  if (mode == MODE_ZEROS || (st && st->error)) {
+  if (mode == MODE_ZEROS || (st && st->bad != INT_MAX)) {
     if (tid == 0) out[c] = 0;
     return;
   }
@@ -669,15 +941,17 @@ __global__ __launch_bounds__(256) void map_to_grid(const double* sx, const doubl
                                                    const int* perm, long n, const double* boxes, int ntiles,
                                                    const double* cen3, long cstride, int latest_buf,
                                                    const State* st, int* out) {
-  map_to_grid_b(sx, sy, sz, perm, n, boxes, ntiles, cen3, cstride, latest_buf, st, out, (int)blockIdx.x, (int)gridDim.x);
+  map_to_grid_b(sx, sy, sz, perm, n, boxes, ntiles, cen3, cstride, latest_buf, st, out, (int)blockIdx.x);
 }
 
-// Sort the k indices ascending (bitonic in LDS) and count adjacent repeats.
-__device__ __forceinline__ void sort_indices_b(int* idx, int k, State* st, int bid, int nblk) {
+// Sort the k indices ascending (bitonic in LDS) and count adjacent repeats; a
+// run that ended without points (MODE_ZEROS, an error) has zeros.
+__device__ __forceinline__ void sort_indices_b(int* idx, int k, State* st) {
   __shared__ int s[MAXB];
   int p2 = 1;
   while (p2 < k) p2 <<= 1;
-  for (int i = threadIdx.x; i < p2; i += 1024) s[i] = i < k ? idx[i] : INT_MAX;
+  const bool none = st && (st->mode == MODE_ZEROS || st->bad != INT_MAX);
+  for (int i = threadIdx.x; i < p2; i += 1024) s[i] = i >= k ? INT_MAX : (none ? 0 : idx[i]);
   __syncthreads();
   for (int size = 2; size <= p2; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
@@ -701,7 +975,7 @@ __device__ __forceinline__ void sort_indices_b(int* idx, int k, State* st, int b
   if ((threadIdx.x & 63) == 0 && d && st) atomicAdd(&st->dups, d);
 }
 __global__ __launch_bounds__(1024) void sort_indices(int* idx, int k, State* st) {
-  sort_indices_b(idx, k, st, (int)blockIdx.x, (int)gridDim.x);
+  sort_indices_b(idx, k, st);
 }
 
 }  // namespace km
@@ -712,15 +986,16 @@ __global__ __launch_bounds__(1024) void sort_indices(int* idx, int k, State* st)
 namespace thc {
 namespace km {
 
-__global__ void copy_final(const int* map0, const int* map1, long n, const double* cen3, int k, int latest_buf,
-                           const State* st, int* map_out, double* cen_out) {
+// final assignment (kept in tile order) and centroids
+__global__ void copy_final(const int* map0, const int* map1, const int* perm, long n, const double* cen3, int k,
+                           int latest_buf, const State* st, int* map_out, double* cen_out) {
   const int iters = st->iters;
   const int mbuf = iters > 0 ? (iters - 1) & 1 : 0;
   const int cbuf = st->mode == MODE_FINAL ? st->final_buf : latest_buf;
   const int* m = mbuf ? map1 : map0;
   const double* c = cen3 + cbuf * 3L * k;
   for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += 256L * gridDim.x) {
-    if (map_out) map_out[i] = m[i];
+    if (map_out) map_out[perm[i]] = m[i];
     if (cen_out && i < 3L * k) cen_out[i] = c[i];
   }
   if (cen_out && n < 3L * k)
@@ -732,11 +1007,24 @@ __global__ void check_keys(const int* keys, long n, int nbins, State* st) {
     if ((unsigned)keys[i] >= (unsigned)nbins) atomicOr(&st->error, 2);
 }
 
+// f with the assignment's centroids a thread for k clusters, as a constant
+template <class F>
+static void with_cpt(int k, F f) {
+  if (k <= 256) f(std::integral_constant<int, 1>{});
+  else if (k <= 1024) f(std::integral_constant<int, 4>{});
+  else if (k <= 2048) f(std::integral_constant<int, 8>{});
+  else f(std::integral_constant<int, MAXB / 256>{});
+}
+
 struct Layout {
   long n;
   int k, max_it;
-  int cells, nbins_sp, nbits_sp, nbits_k;
+  int cells, nbins_sp, nbits_sp;
   int ntiles, ncs, nbb;
+  int cap;      // members a cluster's bucket holds
+  int defer;    // the threshold cannot stop the loop: every iteration's centroids are kept, the differences come last
+  int ncen;     // centroid buffers
+  int nchg;     // iterations' change counts kept
 };
 
 static int bits_for(int nb) {
@@ -745,7 +1033,20 @@ static int bits_for(int nb) {
   return b;
 }
 
-static Layout plan(long n, int k, int max_it) {
+// Members a cluster's bucket holds: eight times the average (the largest
+// clusters of the 64^3 systems reach four times), a larger cluster is read
+// from the map.
+static int bucket_cap(long n, int k) { return (int)std::min<long>(n, std::max<long>(256, 8 * ((n + k - 1) / k))); }
+
+// A normed difference is never negative, so a negative threshold never stops
+// the loop, and nothing in it waits for the differences.
+constexpr size_t DEFER_BYTES = size_t(64) << 20;  // kept centroids of one run
+static bool can_defer(int k, int max_it, double threshold) {
+  const size_t each = sizeof(double) * 3 * (size_t)k + sizeof(int) * CHG;
+  return !(threshold >= 0.0) && each * ((size_t)max_it + 1) <= DEFER_BYTES;
+}
+
+static Layout plan(long n, int k, int max_it, bool defer) {
   Layout L;
   L.n = n; L.k = k; L.max_it = max_it;
   int cells = 1;
@@ -753,132 +1054,158 @@ static Layout plan(long n, int k, int max_it) {
   L.cells = cells;
   L.nbins_sp = cells * cells * cells;
   L.nbits_sp = bits_for(L.nbins_sp);
-  L.nbits_k = bits_for(k);
   L.ntiles = ceil_div(n, TP);
   L.ncs = ceil_div(n, CS_TILE);
   L.nbb = (int)std::min<long>(256, (n + 255) / 256);
+  L.cap = bucket_cap(n, k);
+  L.defer = defer;
+  L.ncen = defer ? max_it + 1 : 3;
+  L.nchg = defer ? max_it : 4;
   return L;
 }
 
 struct Bufs {
-  double *part, *box, *sx, *sy, *sz, *boxes, *cen3, *diffs, *pcts;  // cen3: three centroid buffers
-  int *keys, *perm, *map[2], *order, *tc, *total, *start, *idx0;
+  double *part, *sx, *sy, *sz, *boxes, *wboxes, *cen, *diffs, *pcts;  // cen: L.ncen centroid buffers
+  int *keys, *perm, *map[2], *tc, *total, *start, *idx0;     // map: in tile order
+  int *cnt, *bucket, *chg;
   State* st;
 };
 
 static size_t bytes_for(const Layout& L, bool full) {
   const long n = L.n;
-  const int nb = std::max(L.nbins_sp, L.k);
+  const int nb = L.nbins_sp;
   size_t b = 0;
-  b += carve_bytes<double>(L.nbb * 6) + carve_bytes<double>(6);
-  b += 3 * carve_bytes<double>(n) + carve_bytes<double>((size_t)L.ntiles * 6);
+  b += carve_bytes<double>(L.nbb * 6);
+  b += 3 * carve_bytes<double>(n) + carve_bytes<double>((size_t)L.ntiles * 6) + carve_bytes<double>((size_t)L.ntiles * 24);
   b += 2 * carve_bytes<int>(n);                       // keys, perm
   b += carve_bytes<int>((size_t)L.ncs * nb) + 2 * carve_bytes<int>(nb);
   b += carve_bytes<State>(1);
   if (full) {
-    b += carve_bytes<double>(9L * L.k) + 2 * carve_bytes<double>(std::max(1, L.max_it));
-    b += 3 * carve_bytes<int>(n) + carve_bytes<int>(L.k);
+    b += carve_bytes<double>(3L * L.k * L.ncen) + 2 * carve_bytes<double>(std::max(1, L.max_it));
+    b += 2 * carve_bytes<int>(n) + carve_bytes<int>(L.k);
+    b += carve_bytes<int>(L.k) + carve_bytes<int>((size_t)L.k * L.cap) + carve_bytes<int>((size_t)L.nchg * CHG);
   }
   return b;
 }
 
 static bool carve(Arena& a, const Layout& L, Bufs& b, bool full) {
   const long n = L.n;
-  const int nb = std::max(L.nbins_sp, L.k);
+  const int nb = L.nbins_sp;
   b = Bufs{};
   b.part = a.take<double>(L.nbb * 6);
-  b.box = a.take<double>(6);
   b.sx = a.take<double>(n);
   b.sy = a.take<double>(n);
   b.sz = a.take<double>(n);
   b.boxes = a.take<double>((size_t)L.ntiles * 6);
+  b.wboxes = a.take<double>((size_t)L.ntiles * 24);
   b.keys = a.take<int>(n);
   b.perm = a.take<int>(n);
   b.tc = a.take<int>((size_t)L.ncs * nb);
   b.total = a.take<int>(nb);
   b.start = a.take<int>(nb);
   b.st = a.take<State>(1);
-  bool ok = b.part && b.box && b.sx && b.sy && b.sz && b.boxes && b.keys && b.perm && b.tc && b.total &&
-            b.start && b.st;
+  bool ok = b.part && b.sx && b.sy && b.sz && b.boxes && b.wboxes && b.keys && b.perm && b.tc && b.total && b.start && b.st;
   if (full) {
-    b.cen3 = a.take<double>(9L * L.k);
+    b.cen = a.take<double>(3L * L.k * L.ncen);
     b.diffs = a.take<double>(std::max(1, L.max_it));
     b.pcts = a.take<double>(std::max(1, L.max_it));
     b.map[0] = a.take<int>(n);
     b.map[1] = a.take<int>(n);
-    b.order = a.take<int>(n);
     b.idx0 = a.take<int>(L.k);
-    ok = ok && b.cen3 && b.diffs && b.pcts && b.map[0] && b.map[1] && b.order && b.idx0;
+    b.cnt = a.take<int>(L.k);
+    b.bucket = a.take<int>((size_t)L.k * L.cap);
+    b.chg = a.take<int>((size_t)L.nchg * CHG);
+    ok = ok && b.cen && b.diffs && b.pcts && b.map[0] && b.map[1] && b.idx0 && b.cnt && b.bucket && b.chg;
   }
   return ok;
 }
 
-// Stable counting sort of keys[0..n) (values < nbins) into out (indices).
-static void enqueue_sort(const Layout& L, const Bufs& b, const int* keys, int nbins, int nbits, int* out,
-                         const State* st, hipStream_t s) {
-  hipLaunchKernelGGL(cs_hist, dim3(L.ncs), dim3(256), 0, s, keys, L.n, nbins, b.tc, st);
-  hipLaunchKernelGGL(cs_colscan, dim3(ceil_div(nbins, 64)), dim3(64 * CS_SCAN_W), 0, s, b.tc, L.ncs, nbins, b.total,
-                     st);
-  hipLaunchKernelGGL(cs_totscan, dim3(1), dim3(1024), 0, s, b.total, nbins, b.start, st);
-  hipLaunchKernelGGL(cs_scatter, dim3(L.ncs), dim3(256), 0, s, keys, L.n, nbins, nbits, b.tc, b.start, out, st);
-}
-
-// Spatially sorted copy of the grid (Morton cells, stable) and tile boxes.
+// Spatially sorted copy of the grid (a stable counting sort by Morton cell)
+// and tile boxes.
 static void enqueue_setup(const Layout& L, const Bufs& b, const double* grid, hipStream_t s) {
   hipLaunchKernelGGL(bbox_partial, dim3(L.nbb), dim3(256), 0, s, grid, L.n, b.part);
-  hipLaunchKernelGGL(bbox_final, dim3(1), dim3(64), 0, s, b.part, L.nbb, b.box);
-  hipLaunchKernelGGL(morton_keys, dim3(ceil_div(L.n, 256)), dim3(256), 0, s, grid, L.n, b.box, L.cells, b.keys);
-  enqueue_sort(L, b, b.keys, L.nbins_sp, L.nbits_sp, b.perm, nullptr, s);
-  hipLaunchKernelGGL(gather_sorted, dim3(ceil_div(L.n, 256)), dim3(256), 0, s, grid, b.perm, L.n, b.sx, b.sy, b.sz);
-  hipLaunchKernelGGL(tile_boxes, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, L.n, b.boxes);
+  hipLaunchKernelGGL(morton_keys, dim3(ceil_div(L.n, 256)), dim3(256), 0, s, grid, L.n, b.part, L.nbb, L.cells, b.keys);
+  hipLaunchKernelGGL(cs_hist, dim3(L.ncs), dim3(256), 0, s, b.keys, L.n, L.nbins_sp, b.tc);
+  hipLaunchKernelGGL(cs_colscan, dim3(ceil_div(L.nbins_sp, 64)), dim3(64 * CS_SCAN_W), 0, s, b.tc, L.ncs, L.nbins_sp,
+                     b.total);
+  hipLaunchKernelGGL(cs_totscan, dim3(1), dim3(1024), 0, s, b.total, L.nbins_sp, b.start);
+  hipLaunchKernelGGL(cs_scatter, dim3(L.ncs), dim3(256), 0, s, b.keys, L.n, L.nbins_sp, L.nbits_sp, b.tc, b.start,
+                     b.perm);
+  hipLaunchKernelGGL(sorted_tiles, dim3(L.ntiles), dim3(256), 0, s, grid, b.perm, L.n, b.sx, b.sy, b.sz, b.boxes,
+                     b.wboxes);
 }
 
-// The loop control of iteration it (diff_control: the sequential normed
-// difference, the stop test) runs on the second stream beside iteration
-// it + 1's assignment, sort and centroid sums, which do not need its result:
-// if iteration it stops the loop, iteration it + 1 (already started) only
-// writes buffers the final state does not use, and iteration it + 2 waits for
-// it and returns at once.  Hence three centroid buffers (iteration it reads
-// it % 3, writes (it+1) % 3, and diff_control(it) still reads both while
-// iteration it + 1 writes (it+2) % 3), and change counts / empty-cluster flags
-// kept per iteration parity (diff_control(it) reads and clears its parity's
-// before iteration it + 2 runs).  With sa == s the same code runs in order on
-// one stream.
+// centroid buffer iteration 'it' reads; it writes that of it + 1
+__host__ __device__ inline int cen_buf(const Layout& L, int it) { return L.defer ? it : it % 3; }
+// and its change counts (iteration it + 4 starts after the loop control of it,
+// which clears them)
+__host__ __device__ inline long chg_at(const Layout& L, int it) { return (long)(L.defer ? it : it & 3) * CHG; }
+
+// An iteration is two kernels, the assignment and the centroid sums.
+//
+// Where the threshold cannot stop the loop (L.defer) it keeps every
+// iteration's centroids, and the normed differences -- chains of 3 k
+// sequential adds -- are formed after it, one workgroup per iteration, beside
+// map_to_grid on the second stream.
+//
+// Otherwise the loop control of iteration it (diff_control: the difference,
+// the stop test) runs on the second stream beside iteration it + 1, which does
+// not need its result: if iteration it stops the loop, iteration it + 1
+// (already started) only writes buffers the final state does not use, and
+// iteration it + 2 waits for it and returns at once.  Hence three centroid
+// buffers (iteration it reads it % 3, writes (it+1) % 3, and diff_control(it)
+// still reads both while iteration it + 1 writes (it+2) % 3).  With sa == s
+// the same code runs in order on one stream.
 static int enqueue_kmeans(const Layout& L, const Bufs& b, const double* grid, const double* rho, double threshold,
                           int* interp_idx, int* map_out, double* cen_out, hipStream_t s, hipStream_t sa,
                           const hipEvent_t kev[3]) {
   const long cs = 3L * L.k;
   const bool two = sa != s;
-  hipLaunchKernelGGL(init_state, dim3(1), dim3(64), 0, s, b.st, (int)MODE_LATEST);
+  hipLaunchKernelGGL(init_run, dim3(ceil_div(L.k, 256)), dim3(256), 0, s, grid, b.idx0, L.k, b.cen, b.cnt, b.chg,
+                     L.nchg * CHG, b.st);
   enqueue_setup(L, b, grid, s);
-  hipLaunchKernelGGL(init_centroids, dim3(ceil_div(L.k, 256)), dim3(256), 0, s, grid, b.idx0, L.k, b.cen3);
   const size_t dyn = (size_t)3 * L.k * sizeof(double);
   for (int it = 0; it < L.max_it; ++it) {
-    const int cur = it % 3, nxt = (it + 1) % 3, par = it & 1;
+    const int cur = cen_buf(L, it), nxt = cen_buf(L, it + 1), par = it & 1;
     int* mnew = b.map[par];
     const int* mold = it == 0 ? nullptr : b.map[par ^ 1];
-    if (two && it >= 2) THC_HIP(hipStreamWaitEvent(s, kev[1 + par], 0));  // diff_control(it - 2)
-    hipLaunchKernelGGL(assign, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes,
-                       b.cen3 + cur * cs, L.k, mnew, mold, b.st, par);
-    enqueue_sort(L, b, mnew, L.k, L.nbits_k, b.order, b.st, s);
-    hipLaunchKernelGGL(centroid_sums, dim3(ceil_div(L.k, 4)), dim3(256), 0, s, b.order, b.start, b.total, rho,
-                       grid, L.k, b.cen3 + nxt * cs, b.st, par);
+    if (!L.defer && two && it >= 2) THC_HIP(hipStreamWaitEvent(s, kev[1 + par], 0));  // diff_control(it - 2)
+    with_cpt(L.k, [&](auto cpt) {
+      hipLaunchKernelGGL(assign<cpt.value>, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes,
+                         b.wboxes, b.cen + cur * cs, L.k, mnew, mold, b.cnt, b.bucket, L.cap, b.chg + chg_at(L, it),
+                         b.st, it);
+    });
+    hipLaunchKernelGGL(centroid_sums, dim3(L.k), dim3(256), 0, s, b.cnt, b.bucket, L.cap, mnew, b.perm, L.n, rho, grid,
+                       b.cen + nxt * cs, b.st, it);
+    if (L.defer) continue;
     if (two) {
       THC_HIP(hipEventRecord(kev[0], s));
       THC_HIP(hipStreamWaitEvent(sa, kev[0], 0));
     }
-    hipLaunchKernelGGL(diff_control, dim3(1), dim3(1024), dyn, sa, b.cen3 + nxt * cs, b.cen3 + cur * cs, L.k, L.n,
-                       threshold, it, L.max_it, nxt, b.st, b.diffs, b.pcts);
+    hipLaunchKernelGGL(diff_control, dim3(1), dim3(1024), dyn, sa, b.cen + nxt * cs, b.cen + cur * cs, L.k, L.n,
+                       threshold, it, L.max_it, nxt, b.st, b.chg + chg_at(L, it), b.diffs, b.pcts);
     if (two) THC_HIP(hipEventRecord(kev[1 + par], sa));
   }
-  if (two) THC_HIP(hipStreamWaitEvent(s, kev[1 + ((L.max_it - 1) & 1)], 0));  // last loop control
-  const int latest = L.max_it % 3;
+  const int last = 1 + ((L.max_it - 1) & 1);
+  if (L.defer) {
+    if (two) {
+      THC_HIP(hipEventRecord(kev[0], s));
+      THC_HIP(hipStreamWaitEvent(sa, kev[0], 0));
+    }
+    hipLaunchKernelGGL(diff_control_all, dim3(L.max_it), dim3(1024), dyn, sa, b.cen, L.k, L.n, threshold, L.max_it,
+                       b.st, b.chg, b.diffs, b.pcts);
+    if (two) THC_HIP(hipEventRecord(kev[last], sa));
+  }
+  // the last loop control: map_to_grid goes by its verdict where there is one
+  if (two && !L.defer) THC_HIP(hipStreamWaitEvent(s, kev[last], 0));
+  const int latest = cen_buf(L, L.max_it);
   hipLaunchKernelGGL(map_to_grid, dim3(L.k), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes, L.ntiles,
-                     b.cen3, cs, latest, b.st, interp_idx);
+                     b.cen, cs, latest, b.st, interp_idx);
+  if (two && L.defer) THC_HIP(hipStreamWaitEvent(s, kev[last], 0));
   hipLaunchKernelGGL(sort_indices, dim3(1), dim3(1024), 0, s, interp_idx, L.k, b.st);
   if (map_out || cen_out)
-    hipLaunchKernelGGL(copy_final, dim3(256), dim3(256), 0, s, b.map[0], b.map[1], L.n, b.cen3, L.k, latest, b.st,
-                       map_out, cen_out);
+    hipLaunchKernelGGL(copy_final, dim3(256), dim3(256), 0, s, b.map[0], b.map[1], b.perm, L.n, b.cen, L.k, latest,
+                       b.st, map_out, cen_out);
   THC_HIP(hipGetLastError());
   return THC_OK;
 }
@@ -886,9 +1213,9 @@ static int enqueue_kmeans(const Layout& L, const Bufs& b, const double* grid, co
 // ------------------------------------------------------------------ batches
 //
 // A batch runs the k-means of many systems together: every launch below
-// covers one step (setup, assignment, sort, centroid sums, loop control, map
-// to grid) of all the systems, so a 20-iteration batch of 32 systems is about
-// 160 launches instead of 32 times that.  Each workgroup finds its system in
+// covers one step (setup, assignment, centroid sums, loop control, map to
+// grid) of all the systems, so a 20-iteration batch of 32 systems is about 50
+// launches instead of 32 times that.  Each workgroup finds its system in
 // a prefix table of per-system block counts and runs the same device code as
 // the single-system kernels with that system's sizes and buffers, so every
 // system's result is bit-identical to its own thc_kmeans.
@@ -903,7 +1230,7 @@ struct Job {
 };
 
 // block-count tables, one row of nj + 1 prefix sums per kind
-enum { JK_NBB, JK_N256, JK_NCS, JK_COLSP, JK_COLK, JK_TILES, JK_K256, JK_K4, JK_K, JK_COUNT };
+enum { JK_NBB, JK_N256, JK_NCS, JK_COLSP, JK_TILES, JK_K256, JK_K, JK_COUNT };
 
 inline int job_blocks(const Layout& L, int kind) {
   switch (kind) {
@@ -911,10 +1238,8 @@ inline int job_blocks(const Layout& L, int kind) {
     case JK_N256: return (int)ceil_div(L.n, 256);
     case JK_NCS: return L.ncs;
     case JK_COLSP: return ceil_div(L.nbins_sp, 64);
-    case JK_COLK: return ceil_div(L.k, 64);
     case JK_TILES: return L.ntiles;
     case JK_K256: return ceil_div(L.k, 256);
-    case JK_K4: return ceil_div(L.k, 4);
     default: return L.k;
   }
 }
@@ -935,117 +1260,88 @@ __device__ inline int job_of(const int* off, int nj, int b) {
   const Job& q = jobs[j_];                          \
   const int bid = (int)blockIdx.x - OFF[j_], nblk = OFF[j_ + 1] - OFF[j_];
 
-__global__ void init_state_m(const Job* jobs) { init_state_b(jobs[blockIdx.x].b.st, MODE_LATEST, 0, 1); }
+__global__ __launch_bounds__(256) void init_run_m(const Job* jobs, const int* off, int nj) {
+  KM_JOB(off)
+  init_run_b(q.grid, q.b.idx0, q.L.k, q.b.cen, q.b.cnt, q.b.chg, q.L.nchg * CHG, q.b.st, bid, nblk);
+}
 
 __global__ __launch_bounds__(256) void bbox_partial_m(const Job* jobs, const int* off, int nj) {
   KM_JOB(off)
   bbox_partial_b(q.grid, q.L.n, q.b.part, bid, nblk);
 }
 
-__global__ void bbox_final_m(const Job* jobs) {
-  const Job& q = jobs[blockIdx.x];
-  bbox_final_b(q.b.part, q.L.nbb, q.b.box, 0, 1);
-}
-
 __global__ __launch_bounds__(256) void morton_keys_m(const Job* jobs, const int* off, int nj) {
   KM_JOB(off)
-  morton_keys_b(q.grid, q.L.n, q.b.box, q.L.cells, q.b.keys, bid, nblk);
+  (void)nblk;
+  morton_keys_b(q.grid, q.L.n, q.b.part, q.L.nbb, q.L.cells, q.b.keys, bid);
 }
 
-__global__ __launch_bounds__(256) void gather_sorted_m(const Job* jobs, const int* off, int nj) {
+__global__ __launch_bounds__(256) void cs_hist_m(const Job* jobs, const int* off, int nj) {
   KM_JOB(off)
-  gather_sorted_b(q.grid, q.b.perm, q.L.n, q.b.sx, q.b.sy, q.b.sz, bid, nblk);
+  cs_hist_b(q.b.keys, q.L.n, q.L.nbins_sp, q.b.tc, bid, nblk);
 }
 
-__global__ __launch_bounds__(256) void tile_boxes_m(const Job* jobs, const int* off, int nj) {
+__global__ __launch_bounds__(64 * CS_SCAN_W) void cs_colscan_m(const Job* jobs, const int* off, int nj) {
   KM_JOB(off)
-  tile_boxes_b(q.b.sx, q.b.sy, q.b.sz, q.L.n, q.b.boxes, bid, nblk);
+  cs_colscan_b(q.b.tc, q.L.ncs, q.L.nbins_sp, q.b.total, bid, nblk);
 }
 
-__global__ __launch_bounds__(256) void init_centroids_m(const Job* jobs, const int* off, int nj) {
-  KM_JOB(off)
-  init_centroids_b(q.grid, q.b.idx0, q.L.k, q.b.cen3, bid, nblk);
-}
-
-// Counting sort of one batch: mode 0 sorts the Morton keys into perm (setup),
-// mode 1 the iteration's cluster map into order.  Systems past their last
-// iteration skip mode 1.
-struct SortArgs {
-  const int* keys;
-  int nbins, nbits;
-  int* out;
-  const State* st;
-};
-__device__ inline bool sort_args(const Job& q, int mode, int it, SortArgs& a) {
-  if (mode == 0) {
-    a = SortArgs{q.b.keys, q.L.nbins_sp, q.L.nbits_sp, q.b.perm, nullptr};
-    return true;
-  }
-  a = SortArgs{q.b.map[it & 1], q.L.k, q.L.nbits_k, q.b.order, q.b.st};
-  return it < q.L.max_it;
-}
-
-__global__ __launch_bounds__(256) void cs_hist_m(const Job* jobs, const int* off, int nj, int mode, int it) {
-  KM_JOB(off)
-  SortArgs a;
-  if (!sort_args(q, mode, it, a)) return;
-  cs_hist_b(a.keys, q.L.n, a.nbins, q.b.tc, a.st, bid, nblk);
-}
-
-__global__ __launch_bounds__(64 * CS_SCAN_W) void cs_colscan_m(const Job* jobs, const int* off, int nj, int mode,
-                                                                 int it) {
-  KM_JOB(off)
-  SortArgs a;
-  if (!sort_args(q, mode, it, a)) return;
-  cs_colscan_b(q.b.tc, q.L.ncs, a.nbins, q.b.total, a.st, bid, nblk);
-}
-
-__global__ __launch_bounds__(1024) void cs_totscan_m(const Job* jobs, int mode, int it) {
+__global__ __launch_bounds__(1024) void cs_totscan_m(const Job* jobs) {
   const Job& q = jobs[blockIdx.x];
-  SortArgs a;
-  if (!sort_args(q, mode, it, a)) return;
-  cs_totscan_b(q.b.total, a.nbins, q.b.start, a.st, 0, 1);
+  cs_totscan_b(q.b.total, q.L.nbins_sp, q.b.start, 0, 1);
 }
 
-__global__ __launch_bounds__(256) void cs_scatter_m(const Job* jobs, const int* off, int nj, int mode, int it) {
+__global__ __launch_bounds__(256) void cs_scatter_m(const Job* jobs, const int* off, int nj) {
   KM_JOB(off)
-  SortArgs a;
-  if (!sort_args(q, mode, it, a)) return;
-  cs_scatter_b(a.keys, q.L.n, a.nbins, a.nbits, q.b.tc, q.b.start, a.out, a.st, bid, nblk);
+  cs_scatter_b(q.b.keys, q.L.n, q.L.nbins_sp, q.L.nbits_sp, q.b.tc, q.b.start, q.b.perm, bid, nblk);
 }
 
+__global__ __launch_bounds__(256) void sorted_tiles_m(const Job* jobs, const int* off, int nj) {
+  KM_JOB(off)
+  (void)nblk;
+  sorted_tiles_b(q.grid, q.b.perm, q.L.n, q.b.sx, q.b.sy, q.b.sz, q.b.boxes, q.b.wboxes, bid);
+}
+
+__device__ inline double* job_cen(const Job& q, int it) { return q.b.cen + cen_buf(q.L, it) * 3L * q.L.k; }
+
+template <int CPT>
 __global__ __launch_bounds__(256) void assign_m(const Job* jobs, const int* off, int nj, int it) {
   KM_JOB(off)
+  (void)nblk;
   if (it >= q.L.max_it) return;
   const int par = it & 1;
-  assign_b(q.b.sx, q.b.sy, q.b.sz, q.b.perm, q.L.n, q.b.boxes, q.b.cen3 + (it % 3) * 3L * q.L.k, q.L.k,
-           q.b.map[par], it == 0 ? nullptr : q.b.map[par ^ 1], q.b.st, par, bid, nblk);
+  assign_b<CPT>(q.b.sx, q.b.sy, q.b.sz, q.b.perm, q.L.n, q.b.boxes, q.b.wboxes, job_cen(q, it), q.L.k, q.b.map[par],
+           it == 0 ? nullptr : q.b.map[par ^ 1], q.b.cnt, q.b.bucket, q.L.cap, q.b.chg + chg_at(q.L, it), q.b.st, it,
+           bid);
 }
 
 __global__ __launch_bounds__(256) void centroid_sums_m(const Job* jobs, const int* off, int nj, int it) {
   KM_JOB(off)
+  (void)nblk;
   if (it >= q.L.max_it) return;
-  centroid_sums_b(q.b.order, q.b.start, q.b.total, q.rho, q.grid, q.L.k, q.b.cen3 + ((it + 1) % 3) * 3L * q.L.k,
-                  q.b.st, it & 1, bid, nblk);
+  centroid_sums_b(q.b.cnt, q.b.bucket, q.L.cap, q.b.map[it & 1], q.b.perm, q.L.n, q.rho, q.grid, job_cen(q, it + 1),
+                  q.b.st, it, bid);
 }
 
-__global__ __launch_bounds__(1024) void diff_control_m(const Job* jobs, int it) {
+// loop control of iteration it0 + blockIdx.y
+__global__ __launch_bounds__(1024) void diff_control_m(const Job* jobs, int it0) {
   const Job& q = jobs[blockIdx.x];
+  const int it = it0 + (int)blockIdx.y;
   if (it >= q.L.max_it) return;
-  const long cs = 3L * q.L.k;
-  diff_control_b(q.b.cen3 + ((it + 1) % 3) * cs, q.b.cen3 + (it % 3) * cs, q.L.k, q.L.n, q.threshold, it,
-                 q.L.max_it, (it + 1) % 3, q.b.st, q.b.diffs, q.b.pcts, 0, 1);
+  diff_control_b(job_cen(q, it + 1), job_cen(q, it), q.L.k, q.L.n, q.threshold, it, q.L.max_it,
+                 cen_buf(q.L, it + 1), q.b.st, q.b.chg + chg_at(q.L, it), q.b.diffs, q.b.pcts, q.L.defer);
 }
 
 __global__ __launch_bounds__(256) void map_to_grid_m(const Job* jobs, const int* off, int nj) {
   KM_JOB(off)
-  map_to_grid_b(q.b.sx, q.b.sy, q.b.sz, q.b.perm, q.L.n, q.b.boxes, q.L.ntiles, q.b.cen3, 3L * q.L.k,
-                q.L.max_it % 3, q.b.st, q.interp_idx, bid, nblk);
+  (void)nblk;
+  map_to_grid_b(q.b.sx, q.b.sy, q.b.sz, q.b.perm, q.L.n, q.b.boxes, q.L.ntiles, q.b.cen, 3L * q.L.k,
+                cen_buf(q.L, q.L.max_it), q.b.st, q.interp_idx, bid);
 }
 
 __global__ __launch_bounds__(1024) void sort_indices_m(const Job* jobs) {
   const Job& q = jobs[blockIdx.x];
-  sort_indices_b(q.interp_idx, q.L.k, q.b.st, 0, 1);
+  sort_indices_b(q.interp_idx, q.L.k, q.b.st);
 }
 
 // every system's State, diffs and pcts into one block for a single copy back:
@@ -1071,10 +1367,9 @@ __global__ void collect_m(const Job* jobs, char* out, long stride, int max_it) {
 static std::atomic<int> km_attrs_done{0};  // batched calls run two k-means at once
 static int km_set_attrs() {
   if (km_attrs_done) return THC_OK;
-  THC_HIP(hipFuncSetAttribute((const void*)km::diff_control, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              3 * km::MAXB * (int)sizeof(double)));
-  THC_HIP(hipFuncSetAttribute((const void*)km::diff_control_m, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              3 * km::MAXB * (int)sizeof(double)));
+  for (const void* f : {(const void*)km::diff_control, (const void*)km::diff_control_all,
+                        (const void*)km::diff_control_m})
+    THC_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 3 * km::MAXB * (int)sizeof(double)));
   km_attrs_done = 1;
   return THC_OK;
 }
@@ -1093,7 +1388,7 @@ int kmeans_run(thc_ctx* ctx, const double* grid, const double* rho, long n, int 
     }
   THC_HIP(hipSetDevice(ctx->device));
   THC_TRY(km_set_attrs());
-  const Layout L = plan(n, k, max_it);
+  const Layout L = plan(n, k, max_it, can_defer(k, max_it, threshold));
   const size_t need = bytes_for(L, true);
   if (need > ctx->kmws.cap) {
     if (ctx->kmgraph) ctx->kmgraph->reset();
@@ -1176,6 +1471,11 @@ int kmeans_run_many(thc_ctx* ctx, int nj, const KmSpec* spec, int* status, thc_k
   size_t need = 0;
   int max_it = 1, maxk = 1;
   long idx_total = 0;
+  // the differences come after the loop only if no system's threshold can stop it
+  bool defer = true;
+  for (int j = 0; j < nj; ++j)
+    if (spec[j].k >= 1 && spec[j].max_it >= 1)
+      defer = defer && can_defer(spec[j].k, spec[j].max_it, spec[j].threshold);
   for (int j = 0; j < nj; ++j) {
     const KmSpec& q = spec[j];
     status[j] = THC_OK;
@@ -1193,7 +1493,7 @@ int kmeans_run_many(thc_ctx* ctx, int nj, const KmSpec* spec, int* status, thc_k
       status[j] = THC_ERR_ARG;
       continue;
     }
-    lay[j] = plan(q.n, q.k, q.max_it);
+    lay[j] = plan(q.n, q.k, q.max_it, defer);
     need += bytes_for(lay[j], true);
     max_it = std::max(max_it, q.max_it);
     maxk = std::max(maxk, q.k);
@@ -1255,29 +1555,31 @@ int kmeans_run_many(thc_ctx* ctx, int nj, const KmSpec* spec, int* status, thc_k
   auto grid_of = [&](int kind) { return dim3((unsigned)total_blocks[kind]); };
   THC_HIP(hipEventRecord(ctx->ev[0], s));
   THC_HIP(hipMemcpyAsync(dblob, hb, blob, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(init_state_m, dim3(nl), dim3(64), 0, s, dj);
+  hipLaunchKernelGGL(init_run_m, grid_of(JK_K256), dim3(256), 0, s, dj, off(JK_K256), nl);
   hipLaunchKernelGGL(bbox_partial_m, grid_of(JK_NBB), dim3(256), 0, s, dj, off(JK_NBB), nl);
-  hipLaunchKernelGGL(bbox_final_m, dim3(nl), dim3(64), 0, s, dj);
   hipLaunchKernelGGL(morton_keys_m, grid_of(JK_N256), dim3(256), 0, s, dj, off(JK_N256), nl);
-  auto sort = [&](int mode, int it) {
-    const int col = mode == 0 ? JK_COLSP : JK_COLK;
-    hipLaunchKernelGGL(cs_hist_m, grid_of(JK_NCS), dim3(256), 0, s, dj, off(JK_NCS), nl, mode, it);
-    hipLaunchKernelGGL(cs_colscan_m, grid_of(col), dim3(64 * CS_SCAN_W), 0, s, dj, off(col), nl, mode, it);
-    hipLaunchKernelGGL(cs_totscan_m, dim3(nl), dim3(1024), 0, s, dj, mode, it);
-    hipLaunchKernelGGL(cs_scatter_m, grid_of(JK_NCS), dim3(256), 0, s, dj, off(JK_NCS), nl, mode, it);
-  };
-  sort(0, 0);
-  hipLaunchKernelGGL(gather_sorted_m, grid_of(JK_N256), dim3(256), 0, s, dj, off(JK_N256), nl);
-  hipLaunchKernelGGL(tile_boxes_m, grid_of(JK_TILES), dim3(256), 0, s, dj, off(JK_TILES), nl);
-  hipLaunchKernelGGL(init_centroids_m, grid_of(JK_K256), dim3(256), 0, s, dj, off(JK_K256), nl);
+  hipLaunchKernelGGL(cs_hist_m, grid_of(JK_NCS), dim3(256), 0, s, dj, off(JK_NCS), nl);
+  hipLaunchKernelGGL(cs_colscan_m, grid_of(JK_COLSP), dim3(64 * CS_SCAN_W), 0, s, dj, off(JK_COLSP), nl);
+  hipLaunchKernelGGL(cs_totscan_m, dim3(nl), dim3(1024), 0, s, dj);
+  hipLaunchKernelGGL(cs_scatter_m, grid_of(JK_NCS), dim3(256), 0, s, dj, off(JK_NCS), nl);
+  hipLaunchKernelGGL(sorted_tiles_m, grid_of(JK_TILES), dim3(256), 0, s, dj, off(JK_TILES), nl);
   const size_t dyn = (size_t)3 * maxk * sizeof(double);
   for (int it = 0; it < max_it; ++it) {
-    hipLaunchKernelGGL(assign_m, grid_of(JK_TILES), dim3(256), 0, s, dj, off(JK_TILES), nl, it);
-    sort(1, it);
-    hipLaunchKernelGGL(centroid_sums_m, grid_of(JK_K4), dim3(256), 0, s, dj, off(JK_K4), nl, it);
-    hipLaunchKernelGGL(diff_control_m, dim3(nl), dim3(1024), dyn, s, dj, it);
+    with_cpt(maxk, [&](auto cpt) {
+      hipLaunchKernelGGL(assign_m<cpt.value>, grid_of(JK_TILES), dim3(256), 0, s, dj, off(JK_TILES), nl, it);
+    });
+    hipLaunchKernelGGL(centroid_sums_m, grid_of(JK_K), dim3(256), 0, s, dj, off(JK_K), nl, it);
+    if (!defer) hipLaunchKernelGGL(diff_control_m, dim3(nl), dim3(1024), dyn, s, dj, it);
+  }
+  if (defer) {  // beside map_to_grid, as in a single run
+    THC_HIP(hipEventRecord(ctx->kev[0], s));
+    THC_HIP(hipStreamWaitEvent(ctx->aux, ctx->kev[0], 0));
+    for (int it = 0; it < max_it; it += 32768)
+      hipLaunchKernelGGL(diff_control_m, dim3(nl, std::min(32768, max_it - it)), dim3(1024), dyn, ctx->aux, dj, it);
+    THC_HIP(hipEventRecord(ctx->kev[1], ctx->aux));
   }
   hipLaunchKernelGGL(map_to_grid_m, grid_of(JK_K), dim3(256), 0, s, dj, off(JK_K), nl);
+  if (defer) THC_HIP(hipStreamWaitEvent(s, ctx->kev[1], 0));
   hipLaunchKernelGGL(sort_indices_m, dim3(nl), dim3(1024), 0, s, dj);
   hipLaunchKernelGGL(collect_m, dim3(nl), dim3(256), 0, s, dj, dres, res_stride, max_it);
   THC_HIP(hipGetLastError());
@@ -1315,15 +1617,18 @@ int kmeans_classify(thc_ctx* ctx, const double* grid, long n, const double* cent
   if (!ctx || !grid || !centroids || !grid_map || n < 1 || k < 1 || n > 0x7fffffffL) return THC_ERR_ARG;
   if (k > MAXB) return THC_ERR_UNSUPPORTED;
   THC_HIP(hipSetDevice(ctx->device));
-  const Layout L = plan(n, k, 1);
+  const Layout L = plan(n, k, 1, false);
   THC_TRY(ctx->ws.reserve(bytes_for(L, false)));
   ctx->ws.reset();
   Bufs b;
   if (!carve(ctx->ws, L, b, false)) return THC_ERR_NO_MEMORY;
   hipStream_t s = ctx->stream;
   enqueue_setup(L, b, grid, s);
-  hipLaunchKernelGGL(assign, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes, centroids, k,
-                     grid_map, (const int*)nullptr, (State*)nullptr, 0);
+  with_cpt(k, [&](auto cpt) {
+    hipLaunchKernelGGL(assign<cpt.value>, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes,
+                       b.wboxes, centroids, k, grid_map, (const int*)nullptr, (int*)nullptr, (int*)nullptr, 0,
+                       (int*)nullptr, (const State*)nullptr, 0);
+  });
   THC_HIP(hipGetLastError());
   THC_HIP(hipStreamSynchronize(s));
   return THC_OK;
@@ -1335,28 +1640,29 @@ int kmeans_update(thc_ctx* ctx, const double* rho, const double* grid, long n, c
   if (!ctx || !rho || !grid || !grid_map || !centroids || n < 1 || k < 1 || n > 0x7fffffffL) return THC_ERR_ARG;
   if (k > MAXB) return THC_ERR_UNSUPPORTED;
   THC_HIP(hipSetDevice(ctx->device));
-  const Layout L = plan(n, k, 1);
-  THC_TRY(ctx->ws.reserve(bytes_for(L, false) + carve_bytes<int>(n)));
+  const int cap = bucket_cap(n, k);
+  THC_TRY(ctx->ws.reserve(carve_bytes<State>(1) + carve_bytes<int>(k) + carve_bytes<int>((size_t)k * cap)));
   ctx->ws.reset();
-  Bufs b;
-  if (!carve(ctx->ws, L, b, false)) return THC_ERR_NO_MEMORY;
-  int* order = ctx->ws.take<int>(n);
-  if (!order) return THC_ERR_NO_MEMORY;
+  State* st = ctx->ws.take<State>(1);
+  int* cnt = ctx->ws.take<int>(k);
+  int* bucket = ctx->ws.take<int>((size_t)k * cap);
+  if (!st || !cnt || !bucket) return THC_ERR_NO_MEMORY;
   hipStream_t s = ctx->stream;
-  hipLaunchKernelGGL(init_state, dim3(1), dim3(64), 0, s, b.st, (int)MODE_LATEST);
-  hipLaunchKernelGGL(check_keys, dim3(256), dim3(256), 0, s, grid_map, n, k, b.st);
-  enqueue_sort(L, b, grid_map, k, L.nbits_k, order, nullptr, s);
-  hipLaunchKernelGGL(centroid_sums, dim3(ceil_div(k, 4)), dim3(256), 0, s, order, b.start, b.total, rho, grid, k,
-                     centroids, b.st, 0);
+  hipLaunchKernelGGL(init_run, dim3(ceil_div(k, 256)), dim3(256), 0, s, grid, (const int*)nullptr, k, (double*)nullptr,
+                     cnt, (int*)nullptr, 0, st);
+  hipLaunchKernelGGL(check_keys, dim3(256), dim3(256), 0, s, grid_map, n, k, st);
+  hipLaunchKernelGGL(bucket_map, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, grid_map, n, k, cnt, bucket, cap);
+  hipLaunchKernelGGL(centroid_sums, dim3(k), dim3(256), 0, s, cnt, bucket, cap, grid_map, (const int*)nullptr, n, rho,
+                     grid, centroids, st, 0);
   THC_HIP(hipGetLastError());
   State hst;
-  THC_HIP(hipMemcpyAsync(&hst, b.st, sizeof(State), hipMemcpyDeviceToHost, s));
+  THC_HIP(hipMemcpyAsync(&hst, st, sizeof(State), hipMemcpyDeviceToHost, s));
   THC_HIP(hipStreamSynchronize(s));
   if (hst.error & 2) {
     set_last_error("a grid_map entry lies outside [0, k)", __FILE__, __LINE__);
     return THC_ERR_ARG;
   }
-  if (hst.serr[0]) return THC_ERR_EMPTY_CLUSTER;
+  if (hst.bad == 0) return THC_ERR_EMPTY_CLUSTER;
   return THC_OK;
 }
 
@@ -1365,13 +1671,14 @@ int kmeans_map_to_grid(thc_ctx* ctx, const double* grid, long n, const double* c
   if (!ctx || !grid || !centroids || !interp_idx || n < 1 || k < 1 || n > 0x7fffffffL) return THC_ERR_ARG;
   if (k > MAXB) return THC_ERR_UNSUPPORTED;
   THC_HIP(hipSetDevice(ctx->device));
-  const Layout L = plan(n, k, 1);
+  const Layout L = plan(n, k, 1, false);
   THC_TRY(ctx->ws.reserve(bytes_for(L, false)));
   ctx->ws.reset();
   Bufs b;
   if (!carve(ctx->ws, L, b, false)) return THC_ERR_NO_MEMORY;
   hipStream_t s = ctx->stream;
-  hipLaunchKernelGGL(init_state, dim3(1), dim3(64), 0, s, b.st, (int)MODE_LATEST);
+  hipLaunchKernelGGL(init_run, dim3(1), dim3(256), 0, s, grid, (const int*)nullptr, 0, (double*)nullptr,
+                     (int*)nullptr, (int*)nullptr, 0, b.st);
   enqueue_setup(L, b, grid, s);
   hipLaunchKernelGGL(map_to_grid, dim3(k), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes, L.ntiles,
                      centroids, 0L, 0, (const State*)nullptr, interp_idx);
