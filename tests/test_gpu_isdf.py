@@ -69,6 +69,29 @@ def test_cholesky_not_posdef(ctx, k, bad):
     assert info == bad + 1
 
 
+@pytest.mark.parametrize("k", [15, 16, 17, 33, 47, 48, 49, 79, 81, 143])
+def test_cholesky_panel_edges(ctx, k):
+    """Block edges inside the 64-column block.  Componentwise backward error
+    |L L^T - A| <= gamma |L| |L^T| with k + 1 roundings a product sum plus a few
+    for a root that is not correctly rounded; the inverse blocks go through the
+    solve; a negative pivot is named in every panel and half panel."""
+    rng = np.random.default_rng(k)
+    b = rng.standard_normal((k, k + 4))
+    a = b @ b.T / k + 0.1 * np.eye(k)
+    l, info = ctx.cholesky(a)
+    l = l.cpu().numpy()
+    assert info == 0
+    lo = np.longdouble(l)
+    assert (np.abs(lo @ lo.T - a) <= (k + 8) * 2.0 ** -53 * (np.abs(l) @ np.abs(l).T)).all()
+    z = rng.standard_normal((k, 37))
+    x = ctx.least_squares(a, z).cpu().numpy()
+    assert rel(a @ x, z) < 1e-12
+    for bad in sorted({0, 7, 8, k // 2, k - 1} & set(range(k))):
+        m = a.copy()
+        m[bad, bad] -= 1.5 * l[bad, bad] ** 2
+        assert ctx.cholesky(m)[1] == bad + 1
+
+
 @pytest.mark.parametrize("k,n", [(100, 5000), (513, 20000), (1100, 3000), (2048, 2500)])
 def test_least_squares(ctx, k, n):
     rng = np.random.default_rng(k)

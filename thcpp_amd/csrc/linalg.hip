@@ -22,48 +22,6 @@ namespace {
 
 constexpr int NB = 64;
 
-__device__ inline void wave_sync_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
-// Lower NB x NB block at (i0, j0) of a, jb x jb valid, as rows of an LDS
-// array; outside jb it is the identity.  Load r reads one matrix row (the 64
-// lanes read 64 consecutive doubles).  All 64 loads are issued before the
-// first LDS store (masked lanes read a[0], which exists), so the block costs
-// one memory round trip.  TRANS stores the block transposed.
-template <bool TRANS>
-__device__ inline void load_lower_block(const double* a, long lda, int i0, int j0, int jb, double (*Ls)[NB + 1]) {
-  const int t = threadIdx.x;
-  double v[NB];
-#pragma unroll
-  for (int rr = 0; rr < NB; ++rr) {
-    const bool ok = rr < jb && t <= rr;
-    v[rr] = a[ok ? (long)(i0 + rr) * lda + j0 + t : 0];
-  }
-#pragma unroll
-  for (int rr = 0; rr < NB; ++rr) {
-    const bool ok = rr < jb && t <= rr;
-    const double x = ok ? v[rr] : ((rr >= jb && rr == t) ? 1.0 : 0.0);
-    if (TRANS) Ls[t][rr] = x;
-    else Ls[rr][t] = x;
-  }
-}
-
-// Forward substitution for one row held in registers: x L^T = b, with L given
-// transposed (Lt[c][c2] = L[c2][c], a broadcast read for the whole wave).
-// Right-looking: once x[c] is final every later entry drops its x[c] term, so
-// the updates of one step are independent of each other.
-__device__ inline void solve_row(double (&x)[NB], const double (*Lt)[NB + 1]) {
-#pragma unroll
-  for (int c = 0; c < NB; ++c) {
-    x[c] = x[c] / Lt[c][c];
-#pragma unroll
-    for (int c2 = c + 1; c2 < NB; ++c2) x[c2] = fma(-x[c], Lt[c][c2], x[c2]);
-  }
-}
-
 // ---- fused right-looking Cholesky ------------------------------------------
 // The matrix is taken in 64 x 64 blocks, extended by the identity beyond k.
 // Step j (one kernel) owns panel j: its diagonal block was factored by step
@@ -73,10 +31,8 @@ __device__ inline void solve_row(double (&x)[NB], const double (*Lt)[NB + 1]) {
 //      panel rows, so the panel itself is never rewritten during the step);
 //   2. applies A_IJ -= L_I L_J^T (MFMA);
 //   3. for I = J, parks L_I transposed in the unused upper block (j, I);
-//   4. tile (j+1, j+1) -- workgroup 0 -- then factors its block: wave 0 runs
-//      the pivot steps with lane r owning row r in registers, and wave 1,
-//      in lockstep one barrier behind each pivot, forms W_{j+1} column by
-//      column (lane c solves L x = e_c, right-looking).
+//   4. tile (j+1, j+1) -- workgroup 0 -- then factors its block in panels of
+//      16 columns (factor_block) and forms W_{j+1}.
 // A last kernel moves the parked panels into the lower triangle and zeroes
 // the upper one.  Step -1 only factors block 0.
 constexpr int CB = NB;      // block size
@@ -142,107 +98,166 @@ __device__ inline void panel_rows(double (*X)[CB + 1], const double (*W)[CB + 1]
     for (int v = 0; v < 4; ++v) X[16 * w + (l >> 4) + 4 * v][16 * cb + (l & 15)] = acc[cb][v];
 }
 
-// One pivot step KK of factor_block (after its barrier).  Wave 0 (lane r
-// owns row r of the block in x): column KK + 1 takes step KK's update first,
-// with L[KK+1][KK] read from lane KK + 1's register, so the next pivot, its
-// Newton steps and the scaled column KK + 1 (published as row KK + 1 of Lt)
-// follow without an LDS round trip; the other columns read row KK of Lt, up
-// to RA entries of it issued before that dependent chain so that the LDS
-// latency hides behind it.  Wave 1 (lane c owns column c of W = L^-1 in x)
-// takes substitution step KK with row KK of Lt and Rs[KK].
-constexpr int RA = 32;
+// ---- 64 x 64 block factor and inverse ---------------------------------------
+// Both work in panels of PB = 16 columns.  What a panel does to the rows and
+// columns behind it is a rank-16 update on the matrix cores: an f64 MFMA adds
+// its four products as one chain of fused multiply-adds in ascending k, so an
+// element sees exactly the operations, in the order, that updating it column
+// by column would give.
+//
+// Panels are a loop and everything in it is inlined by force.  Unrolled over
+// all 64 pivots the code runs once per launch, and fetching it (some 50 KB)
+// took as long as running it; called as a function (the compiler's own choice)
+// inverse_rows spends 6900 cycles instead of 2700, saving its registers.
+// Measured: factor and inverse of a block 60000 -> 28000 cycles, a Cholesky
+// step of the 2048 x 2048 CC^T 30 -> 21 us.
+constexpr int PB = 16;
 
-template <int KK>
-__device__ __forceinline__ void pivot_step(double (&x)[CB], double& v, int& bad, double (*Lt)[CB + 1], double* Rs,
-                                           int w, int l, bool need_w) {
-  if (w == 0) {
-    if (KK + 1 < CB) {
-      constexpr int c0 = KK + 2, na = CB - c0 < RA ? CB - c0 : RA;
-      double ra[na > 0 ? na : 1];
+typedef double (*Blk)[CB + 1];
+
+// 16 x 16 tile at (r0, c0) of T  -=  rows r0.. of A x columns: A[r][k0 + k] B(k, c)
+//   TB: B(k, c) = B[c0 + c][k0 + k] (a transposed factor), else B[k0 + k][c0 + c]
+template <bool TB>
+__device__ __forceinline__ void tile_update(Blk T, Blk A, Blk B, int r0, int c0, int k0, bool zero) {
+  const int l = threadIdx.x & 63, l16 = l & 15, l4 = l >> 4;
+  double av[PB / 4], bv[PB / 4];
 #pragma unroll
-      for (int i = 0; i < na; ++i) ra[i] = Lt[KK][c0 + i];
-      __asm__ volatile("" ::: "memory");
-      x[KK + 1] = fma(-v, readlane_d(v, KK + 1), x[KK + 1]);
-      const double d = readlane_d(x[KK + 1], KK + 1);
-      if (!(d > 0.0) && bad == 0) bad = KK + 2;
-      double s, rs;
-      sqrt_rsqrt(d, s, rs);
-      const double vn = (l == KK + 1) ? s : x[KK + 1] * rs;
-#pragma unroll
-      for (int i = 0; i < na; ++i) x[c0 + i] = fma(-v, ra[i], x[c0 + i]);
-#pragma unroll
-      for (int c = c0 + na; c < CB; ++c) x[c] = fma(-v, Lt[KK][c], x[c]);
-      x[KK + 1] = vn;
-      Lt[KK + 1][l] = vn;
-      if (l == KK + 1) Rs[KK + 1] = rs;
-      v = vn;
-    }
-  } else if (w == 1 && need_w) {
-    constexpr int c0 = KK + 1, na = CB - c0 < RA ? CB - c0 : RA;
-    const double r = Rs[KK];
-    double ra[na > 0 ? na : 1];
-#pragma unroll
-    for (int i = 0; i < na; ++i) ra[i] = Lt[KK][c0 + i];
-    __asm__ volatile("" ::: "memory");
-    x[KK] *= r;
-#pragma unroll
-    for (int i = 0; i < na; ++i) x[c0 + i] = fma(-ra[i], x[KK], x[c0 + i]);
-#pragma unroll
-    for (int c = c0 + na; c < CB; ++c) x[c] = fma(-Lt[KK][c], x[KK], x[c]);
+  for (int q = 0; q < PB / 4; ++q) {
+    av[q] = -A[r0 + l16][k0 + 4 * q + l4];
+    bv[q] = TB ? B[c0 + l16][k0 + 4 * q + l4] : B[k0 + 4 * q + l4][c0 + l16];
   }
+  d4 acc;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) acc[v] = zero ? 0.0 : T[r0 + l4 + 4 * v][c0 + l16];
+#pragma unroll
+  for (int q = 0; q < PB / 4; ++q) acc = mfma_f64(av[q], bv[q], acc);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) T[r0 + l4 + 4 * v][c0 + l16] = acc[v];
 }
 
-template <int... K>
-__device__ __forceinline__ void pivot_steps(std::integer_sequence<int, K...>, double (&x)[CB], double& v, int& bad,
-                                            double (*Lt)[CB + 1], double* Rs, int w, int l, bool need_w) {
-  ((__syncthreads(), pivot_step<K>(x, v, bad, Lt, Rs, w, l, need_w)), ...);
+// Rows of panel p of X = L^-1, all 64 columns (one wave, lane c column c):
+// forward substitution, by the diagonal of L (DIV) or by its reciprocals Rs.
+// Each step reads the next column of L while it uses its own; the empty asm
+// statements keep the compiler from regrouping the steps into one chain of up
+// to sixteen dependent operations per row.
+template <bool DIV>
+__device__ __forceinline__ void inverse_rows(Blk X, Blk L, const double* Rs, int p) {
+  const int c = threadIdx.x & 63, r0 = PB * p, q = c / PB;
+  double y[PB], dg[PB], col[2][PB];
+#pragma unroll
+  for (int i = 0; i < PB; ++i) {
+    y[i] = q < p ? X[r0 + i][c] : (r0 + i == c ? 1.0 : 0.0);
+    dg[i] = DIV ? L[r0 + i][r0 + i] : Rs[r0 + i];
+    if (i > 0) col[0][i] = L[r0 + i][r0];
+  }
+#pragma unroll
+  for (int k = 0; k < PB; ++k) {
+#pragma unroll
+    for (int i = k + 2; i < PB; ++i) col[(k + 1) & 1][i] = L[r0 + i][r0 + k + 1];
+    y[k] = DIV ? y[k] / dg[k] : y[k] * dg[k];
+    asm volatile("" : "+v"(y[k]));
+#pragma unroll
+    for (int i = k + 1; i < PB; ++i) {
+      y[i] = fma(-col[k & 1][i], y[k], y[i]);
+      asm volatile("" : "+v"(y[i]));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < PB; ++i) X[r0 + i][c] = y[i];
+}
+
+// What panel p of X does to the rows of the later panels: tiles (o, q), o > p
+// >= q, dealt to nw waves (this one is w).  A tile's first update starts it.
+__device__ __forceinline__ void inverse_update(Blk X, Blk L, int p, int w, int nw) {
+  const int n = (CB / PB - 1 - p) * (p + 1);
+#pragma unroll 1
+  for (int t = w; t < n; t += nw) {
+    const int q = t % (p + 1), o = p + 1 + t / (p + 1);
+    tile_update<false>(X, L, X, PB * o, PB * q, PB * p, p == q);
+  }
 }
 
 // Factor the block in C (LDS, lower part read) at global rows/cols base ..
 // base + 63 (jb of them inside the matrix): L (lower) to adiag, W = L^-1 to
-// w_out (row-major 64 x 64, zero above the diagonal) when need_w.  Lt (row kk
-// = column kk of L) and Rs (1 / L[kk][kk]) are LDS scratch.  All four waves
-// call this (the barriers are workgroup-wide); waves 0 and 1 work in
-// lockstep, one barrier per pivot.  info: first non-positive pivot (1-based,
+// w_out (row-major 64 x 64, zero above the diagonal) when need_w.  X and Rs
+// (1 / L[k][k]) are LDS scratch.  info: first non-positive pivot (1-based,
 // global), kept if already set.
-__device__ void factor_block(double (*C)[CB + 1], double (*Lt)[CB + 1], double* Rs, bool need_w, double* adiag,
-                             long lda, int jb, double* w_out, int* info, int base) {
+//
+// Wave 0 runs the pivots of a panel with lane r owning row r of its 16 columns
+// in registers and other lanes' entries by readlane: no barrier and no LDS
+// round trip inside half a panel (with the columns behind the pivot read back
+// from LDS instead, a block took a sixth longer).  One wave issues an FP64
+// operation every 5 to 9 cycles and its result takes 9, so a pivot (410 cycles)
+// costs the chain through its root and its column updates.  Waves 1 to 3
+// do what the previous panel left: its rows of W and its update of the tiles
+// that the current panel does not need, then, beside the second half, its
+// update of W.
+__device__ __forceinline__ void factor_block(Blk C, Blk X, double* Rs, bool need_w, double* adiag, long lda, int jb,
+                                             double* w_out, int* info, int base) {
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
-  double x[CB];
-  int bad = 0;
-  double v = 0.0;
-  if (w == 0) {
+  constexpr int NP = CB / PB, H = PB / 2;
+  double x[PB], v = 0.0, own = 1.0, mine = 0.0;  // own: this lane's pivot, mine: its reciprocal root
+#pragma unroll 1
+  for (int p = 0; p < NP; ++p) {
+    const int c0 = PB * p;
+    // pivot k beside the updates by column k - 1 of the columns behind k; the
+    // fence keeps later broadcasts from piling up in scalar registers
+    auto pivot = [&](int k) {
+      if (k > 0) x[k] = fma(-v, readlane_d(v, c0 + k), x[k]);
+      if (l == c0 + k) own = x[k];
+      double s, rs;
+      sqrt_rsqrt(readlane_d(x[k], c0 + k), s, rs);
 #pragma unroll
-    for (int c = 0; c < CB; ++c) x[c] = C[l][c];
-    const double d = readlane_d(x[0], 0);
-    if (!(d > 0.0)) bad = 1;
-    double s, rs;
-    sqrt_rsqrt(d, s, rs);
-    v = (l == 0) ? s : x[0] * rs;
-    x[0] = v;
-    Lt[0][l] = v;
-    if (l == 0) Rs[0] = rs;
-  } else if (w == 1) {
+      for (int c = k + 1; c < PB; ++c)
+        if (k > 0) x[c] = fma(-v, readlane_d(v, c0 + c), x[c]);
+      if (l == c0 + k) mine = rs;
+      v = (l == c0 + k) ? s : x[k] * rs;
+      x[k] = v;
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (w == 0) {
 #pragma unroll
-    for (int c = 0; c < CB; ++c) x[c] = (c == l) ? 1.0 : 0.0;
+      for (int k = 0; k < PB; ++k) x[k] = C[l][c0 + k];
+#pragma unroll
+      for (int k = 0; k < H; ++k) pivot(k);
+    } else if (w == 1) {
+      if (need_w && p > 0) inverse_rows<false>(X, C, Rs, p - 1);
+    } else if (p == 1) {  // tiles (I, J), J > p, of panel p - 1
+      tile_update<true>(C, C, C, PB * w, PB * 2, c0 - PB, false);
+      if (w == 3) tile_update<true>(C, C, C, PB * 3, PB * 3, c0 - PB, false);
+    } else if (p == 2 && w == 2) {
+      tile_update<true>(C, C, C, PB * 3, PB * 3, c0 - PB, false);
+    }
+    __syncthreads();
+    if (w == 0) {
+#pragma unroll
+      for (int k = H; k < PB; ++k) pivot(k);
+#pragma unroll
+      for (int k = 0; k < PB; ++k) C[l][c0 + k] = x[k];
+      if (l >= c0 && l < c0 + PB) Rs[l] = mine;
+    } else if (need_w && p > 0) {
+      inverse_update(X, C, p - 1, w - 1, 3);
+    }
+    __syncthreads();
+    // panel p + 1 first: tiles (I, p + 1)
+    if (w < NP - 1 - p) tile_update<true>(C, C, C, PB * (p + 1 + w), PB * (p + 1), c0, false);
+    __syncthreads();
   }
-  pivot_steps(std::make_integer_sequence<int, CB>{}, x, v, bad, Lt, Rs, w, l, need_w);
-  // after the last barrier only wave 1 reads Lt (row 63, no entries) and Rs
   if (w == 0) {
-    if (l == 0 && bad && *info == 0) *info = base + bad;
-#pragma unroll
-    for (int c = 0; c < CB; ++c) C[l][c] = x[c];
-  } else if (w == 1 && need_w) {
-#pragma unroll
-    for (int c = 0; c < CB; ++c) Lt[c][l] = x[c];
+    const unsigned long long not_pos = __ballot(!(own > 0.0));
+    if (l == 0 && not_pos && *info == 0) *info = base + __ffsll((long long)not_pos);
+    if (need_w) inverse_rows<false>(X, C, Rs, NP - 1);
+  } else {
+    for (int r = w - 1; r < CB; r += 3)
+      if (r < jb && l <= r) adiag[(long)r * lda + l] = C[r][l];
   }
   __syncthreads();
-  const int c = l, rb = w;
+  if (need_w) {
 #pragma unroll
-  for (int i = 0; i < CB / 4; ++i) {
-    const int r = rb + 4 * i;
-    if (r < jb && c <= r) adiag[(long)r * lda + c] = C[r][c];
-    if (need_w) w_out[r * CB + c] = Lt[r][c];
+    for (int i = 0; i < CB / 4; ++i) {
+      const int r = w + 4 * i;
+      w_out[r * CB + l] = X[r][l];
+    }
   }
 }
 
@@ -384,19 +399,24 @@ __global__ __launch_bounds__(256) void pad_lower(const double* l, int k, long ld
   }
 }
 
-// Invert each 64 x 64 lower diagonal block of lp into linv (same positions):
-// thread t solves x L^T = e_t, i.e. x = column t of L^-1.
-__global__ __launch_bounds__(64) void invert_diag_blocks(const double* lp, int kp, double* linv) {
-  __shared__ double Lt[NB][NB + 1];
-  const int j0 = blockIdx.x * NB, t = threadIdx.x;
-  load_lower_block<true>(lp, kp, j0, j0, NB, Lt);
-  wave_sync_lds();
-  double x[NB];
+// Invert each 64 x 64 lower diagonal block of lp into linv (same positions),
+// one block per workgroup.
+__global__ __launch_bounds__(CT) void invert_diag_blocks(const double* lp, int kp, double* linv) {
+  __shared__ double Ls[CB][CB + 1];
+  __shared__ double Xs[CB][CB + 1];
+  const long j0 = (long)blockIdx.x * CB;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  load_tile(lp, kp, kp, j0, j0, Ls);
+  __syncthreads();
+#pragma unroll 1
+  for (int p = 0; p < CB / PB; ++p) {
+    if (w == 0) inverse_rows<true>(Xs, Ls, nullptr, p);
+    __syncthreads();
+    inverse_update(Xs, Ls, p, w, 4);
+    __syncthreads();
+  }
 #pragma unroll
-  for (int c = 0; c < NB; ++c) x[c] = (c == t) ? 1.0 : 0.0;
-  solve_row(x, Lt);
-#pragma unroll
-  for (int i = 0; i < NB; ++i) linv[(long)(j0 + i) * kp + j0 + t] = x[i];
+  for (int i = 0; i < CB / 4; ++i) linv[(j0 + w + 4 * i) * kp + j0 + l] = Xs[w + 4 * i][l];
 }
 
 __global__ __launch_bounds__(256) void fill_zero(double* a, long count) {
@@ -625,7 +645,7 @@ int spd_inverse_from_chol(const double* l, int k, long lda, double* ainv, void* 
   const long kk = (long)kp * kp;
   hipLaunchKernelGGL(pad_lower, dim3(grid_for(kk)), dim3(256), 0, s, l, k, lda, lp, kp);
   hipLaunchKernelGGL(fill_zero, dim3(grid_for(kk)), dim3(256), 0, s, linv, kk);
-  hipLaunchKernelGGL(invert_diag_blocks, dim3(kp / NB), dim3(64), 0, s, lp, kp, linv);
+  hipLaunchKernelGGL(invert_diag_blocks, dim3(kp / NB), dim3(CT), 0, s, lp, kp, linv);
   THC_HIP(hipGetLastError());
   for (int sz = NB; sz < kp; sz *= 2) {
     const int pairs = kp / (2 * sz);
