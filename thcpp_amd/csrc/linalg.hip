@@ -81,17 +81,19 @@ __device__ inline void load_tile(const double* a, long lda, int k, long r0, long
 }
 
 // Rows 16 w .. 16 w + 15 of X become X W^T (wave w; only its own rows are
-// read and then rewritten).  f64 MFMA D layout: lane l holds column l % 16 of
-// rows l / 16 + 4 v.
-__device__ inline void panel_rows(double (*X)[CB + 1], const double (*W)[CB + 1]) {
+// read and then rewritten).  wf: fragments of W, which is lower triangular, so
+// that wf[q][cb] is read for 16 cb + 15 >= 4 q only.  f64 MFMA D layout: lane
+// l holds column l % 16 of rows l / 16 + 4 v.
+__device__ __forceinline__ void panel_rows(double (*X)[CB + 1], const double (&wf)[CB / 4][4]) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   d4 acc[4] = {};
+  double af[CB / 4];
 #pragma unroll
-  for (int q0 = 0; q0 < CB; q0 += 4) {
-    const double av = X[16 * w + (l & 15)][q0 + (l >> 4)];
+  for (int q = 0; q < CB / 4; ++q) af[q] = X[16 * w + (l & 15)][4 * q + (l >> 4)];
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb) acc[cb] = mfma_f64(av, W[16 * cb + (l & 15)][q0 + (l >> 4)], acc[cb]);
-  }
+  for (int q = 0; q < CB / 4; ++q)
+#pragma unroll
+    for (int cb = q / 4; cb < 4; ++cb) acc[cb] = mfma_f64(af[q], wf[q][cb], acc[cb]);
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
@@ -269,13 +271,21 @@ __device__ inline void lower_tile_of(int t, int& ti, int& tj) {
   tj = t - i * (i + 1) / 2;
 }
 
-__global__ __launch_bounds__(CT) void chol_step(double* a, long lda, int k, int nb, int j,
-                                                const double* __restrict__ w_in, double* __restrict__ w_out, int* info) {
-  __shared__ double Ws[CB][CB + 1];
+// Two blocks of LDS (W is read into registers): 67 KB, and at most 256
+// registers, fit beside one workgroup of the ZC^T GEMM on the other stream; with
+// 100 KB a step waited until a CU had none of them left.  The waves go first
+// where they share a SIMD with it: a step is a chain of latencies that everything
+// else waits for (half-rotated 48^3 points, K 1024: 5.60 ms without, 5.42 with).
+// Alone a step of the 2048 x 2048 CC^T takes 20 us: block factor and inverse 13,
+// two 64^3 products on the matrix cores 3.5, loads and launch the rest.
+__global__ __launch_bounds__(CT, 2) void chol_step(double* a, long lda, int k, int nb, int j,
+                                                   const double* __restrict__ w_in, double* __restrict__ w_out,
+                                                   int* info) {
   __shared__ double Xi[CB][CB + 1];
   __shared__ double Xj[CB][CB + 1];
   __shared__ double Rs[CB];
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  __builtin_amdgcn_s_setprio(3);
   int ti, tj;
   lower_tile_of((int)blockIdx.x, ti, tj);
   const int I = j + 1 + ti, J = j + 1 + tj;
@@ -283,18 +293,39 @@ __global__ __launch_bounds__(CT) void chol_step(double* a, long lda, int k, int 
   const bool factor = blockIdx.x == 0;  // tile (j + 1, j + 1)
   if (j >= 0) {
     const long cj = (long)j * CB;
-    load_tile(a, lda, k, rI, cj, Xi);
-    if (J != I) load_tile(a, lda, k, rJ, cj, Xj);
-    {
-      double v[CB / 4];
+    // wave w loads rows 16 w .. of everything, whole rows at a time
+    double vi[CB / 4], vw[CB / 4], vj[CB / 4], wf[CB / 4][4];
 #pragma unroll
-      for (int i = 0; i < CB / 4; ++i) v[i] = w_in[(w + 4 * i) * CB + l];
+    for (int i = 0; i < CB / 4; ++i) {
+      vi[i] = ext_at(a, lda, k, rI + 16 * w + i, cj + l);
+      vw[i] = w_in[(16 * w + i) * CB + l];
+    }
+    if (J != I) {
 #pragma unroll
-      for (int i = 0; i < CB / 4; ++i) Ws[w + 4 * i][l] = v[i];
+      for (int i = 0; i < CB / 4; ++i) vj[i] = ext_at(a, lda, k, rJ + 16 * w + i, cj + l);
+    }
+    d4 acc[4];
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[cb][v] = ext_at(a, lda, k, rI + 16 * w + (l >> 4) + 4 * v, rJ + 16 * cb + (l & 15));
+#pragma unroll
+    for (int i = 0; i < CB / 4; ++i) {
+      Xi[16 * w + i][l] = vi[i];
+      Xj[16 * w + i][l] = vw[i];
     }
     __syncthreads();
-    panel_rows(Xi, Ws);
-    if (J != I) panel_rows(Xj, Ws);
+#pragma unroll
+    for (int q = 0; q < CB / 4; ++q)
+#pragma unroll
+      for (int cb = q / 4; cb < 4; ++cb) wf[q][cb] = Xj[16 * cb + (l & 15)][4 * q + (l >> 4)];
+    panel_rows(Xi, wf);
+    if (J != I) {
+      __syncthreads();  // W has been read: its block takes A_Jj
+#pragma unroll
+      for (int i = 0; i < CB / 4; ++i) Xj[16 * w + i][l] = vj[i];
+      panel_rows(Xj, wf);
+    }
     __syncthreads();
     const double(*Lj)[CB + 1] = (J != I) ? Xj : Xi;
     if (I == J) {
@@ -305,11 +336,6 @@ __global__ __launch_bounds__(CT) void chol_step(double* a, long lda, int k, int 
         if (rI + l < k) a[(cj + c) * lda + rI + l] = Xi[l][c];
       }
     }
-    d4 acc[4];
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[cb][v] = ext_at(a, lda, k, rI + 16 * w + (l >> 4) + 4 * v, rJ + 16 * cb + (l & 15));
 #pragma unroll
     for (int q0 = 0; q0 < CB; q0 += 4) {
       const double av = -Xi[16 * w + (l & 15)][q0 + (l >> 4)];
@@ -334,7 +360,7 @@ __global__ __launch_bounds__(CT) void chol_step(double* a, long lda, int k, int 
     load_tile(a, lda, k, 0, 0, Xj);
   }
   __syncthreads();
-  factor_block(Xj, Ws, Rs, j + 2 < nb, a + rI * lda + rI, lda, (int)std::min<long>(CB, k - rI), w_out, info,
+  factor_block(Xj, Xi, Rs, j + 2 < nb, a + rI * lda + rI, lda, (int)std::min<long>(CB, k - rI), w_out, info,
                (int)rI);
 }
 
