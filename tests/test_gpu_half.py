@@ -96,3 +96,29 @@ def test_isdf_half_rejects_empty_occupied_set(ctx, half_case):
     s, occ, idx = half_case
     out = ctx.isdf_half(s.aoR, np.zeros((s.N, 0)), idx, s.n, s.coulG)
     assert out["status"] == L.THC_ERR_ARG
+
+
+@pytest.mark.parametrize("n,m,k", [((4, 4, 4), 1, 1), ((5, 7, 9), 7, 17), ((8, 8, 8), 20, 129), ((13, 10, 5), 17, 127),
+                                   ((9, 8, 8), 33, 33), ((16, 9, 8), 64, 300)])
+def test_digit_planes_of_czt(ctx, n, m, k):
+    """The digits that the ZC^T GEMM writes are those of a stored ZC^T split
+    afterwards (the route of complex orbitals, here with no imaginary part), at
+    the edges of its tiles and of the 32-column blocks.  Orbitals of a few bits
+    make every product sum exact, so X has to agree bit for bit; in the
+    half-rotated product P o Pocc with Pocc = S P S for signs S, X changes by
+    exactly those signs, which takes the digits of negative values."""
+    from thcpp_amd import synthetic
+    rng = np.random.default_rng(k)
+    N = int(np.prod(n))
+    a = (2.0 * rng.integers(-4, 4, (N, m)) + 1.0) / 8.0
+    idx = np.sort(rng.choice(N, k, replace=False)).astype(np.int32)
+    cg = synthetic.coulomb_kernel(6.0, n)
+    full = ctx.isdf(a, idx, n, cg, precision=L.PREC_MIXED, want_xi=True)
+    stored = ctx.isdf_complex(a.astype(complex), idx, n, cg, precision=L.PREC_MIXED, want_xi=True)
+    assert full["cct_info"] == 0
+    x = full["xi"].cpu().numpy()
+    assert np.isfinite(x).all()
+    np.testing.assert_array_equal(x, stored["xi"].cpu().numpy())
+    sign = rng.choice([-1.0, 1.0], N)
+    half = ctx.isdf_half(a, sign[:, None] * a, idx, n, cg, precision=L.PREC_MIXED, want_xi=True)
+    np.testing.assert_array_equal(half["xi"].cpu().numpy(), sign[idx][:, None] * x * sign[None, :])

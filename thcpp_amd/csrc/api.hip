@@ -349,10 +349,8 @@ int isdf_run(thc_ctx* ctx, const double* aoR, const double* aoR_half, long n, in
   THC_HIP(hipEventRecord(ctx->fork, s));
   THC_HIP(hipStreamWaitEvent(sa, ctx->fork, 0));
   double* rk_d = reinterpret_cast<double*>(ctx->pinned);
-  // The digit epilogue runs on the one-workgroup-per-CU 128 x 128 x 32 tile, the
-  // tile the ZC^T GEMM takes anyway for inner dimensions up to 256; deeper
-  // products (M > 256) run faster on the two-per-CU tile with a separate split.
-  const bool fuse_split = prec == THC_PREC_MIXED && !aoR_half && !cplx && refine == 0 && m <= 256;
+  // mixed path without refinement: nothing but the solve reads Zt
+  const bool fuse_split = prec == THC_PREC_MIXED && !ch && !cplx && refine == 0;
   if (ch) {
     // 1 + 2, complex half-rotated: the stacked ZC^T (the X buffer as scratch),
     // then CC^T's real embedding gathered from it, its Cholesky factor and
@@ -398,32 +396,22 @@ int isdf_run(thc_ctx* ctx, const double* aoR, const double* aoR_half, long n, in
     }
     hipLaunchKernelGGL(copy_f64, dim3(grid_for((long)k * k)), dim3(256), 0, sa, B.c, B.l, (long)k * k);
     THC_HIP(hipGetLastError());
-    THC_TRY(cholesky_f64(B.l, k, k, B.info, B.chol_w, sa));
-    THC_TRY(spd_inverse_from_chol(B.l, k, k, B.ci, B.inv_w, sa));
-    THC_HIP(hipEventRecord(ctx->join, sa));
-    // rank diagnostic (IVecs::check_rank) after the join: nothing on the main
-    // stream waits for it; its tridiagonal form lands in pinned host memory
-    if (want_rank) THC_TRY(sym_tridiag(B.c, k, k, rk_d, rk_d + k, B.rank_w, sa));
     // 1. Zt = (Phi Phi_mu^T)^2, N x K row-major (Zt[r][mu] = ZC^T[mu][r]): B rows
     //    gathered by idx, epilogue squares; this layout lets the solve read both
     //    operands along k and keeps the 4 GB store row-contiguous
     //    Half-rotated (setup_CZt_half): Zt = P o Pocc, P stored first, then the
     //    occupied-orbital product multiplied into it in the epilogue.
-    //    Mixed path without refinement: nothing but the solve reads Zt, so the
-    //    GEMM's epilogue writes the solve's int8 digit planes of Zt directly
-    //    (the same values as splitting the FP64 Zt afterwards) and Zt itself is
-    //    never stored.
-    {
+    //    Where only the int8 solve reads Zt, its digit planes are written instead
+    //    (the same values as splitting the FP64 Zt afterwards).
+    if (fuse_split) {
+      THC_TRY(oz_solve_zct(k, n, idx, aoR, m, aoR_half, aoR_half ? m_occ : 0, B.solve_w, s));
+    } else {
       GemmArgs g = {};
       g.m = n; g.n = k; g.k = m;
       g.a = aoR; g.lda = m; g.a_trans = 0;
       g.b = aoR; g.ldb = m; g.b_trans = 1; g.b_rows = idx; g.b_nrows = n;
       g.c = B.z; g.ldc = k; g.c_trans = 0;
       g.alpha = 1.0; g.beta = 0.0; g.epi_square = aoR_half ? 0 : 1; g.batch = 1;
-      if (fuse_split) {
-        THC_TRY(oz_solve_prepare(k, n, idx, aoR, m, B.solve_w, g, s));
-        g.epi_square = 0;
-      }
       THC_TRY(gemm_f64(g, s));
       if (aoR_half) {
         GemmArgs h = g;
@@ -441,6 +429,12 @@ int isdf_run(thc_ctx* ctx, const double* aoR, const double* aoR_half, long n, in
       }
     }
     THC_HIP(hipEventRecord(ev[1], s));
+    THC_TRY(cholesky_f64(B.l, k, k, B.info, B.chol_w, sa));
+    THC_TRY(spd_inverse_from_chol(B.l, k, k, B.ci, B.inv_w, sa));
+    THC_HIP(hipEventRecord(ctx->join, sa));
+    // rank diagnostic (IVecs::check_rank) after the join: nothing on the main
+    // stream waits for it; its tridiagonal form lands in pinned host memory
+    if (want_rank) THC_TRY(sym_tridiag(B.c, k, k, rk_d, rk_d + k, B.rank_w, sa));
   }
   // join: the solve needs (CC^T)^-1
   THC_HIP(hipStreamWaitEvent(s, ctx->join, 0));

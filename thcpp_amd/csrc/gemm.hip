@@ -48,8 +48,8 @@ template <> struct Mfma<float> {
   __device__ static inline int row(int lane, int v) { return 4 * (lane >> 4) + v; }
 };
 
-enum { EPI_STORE = 0, EPI_SQUARE = 1, EPI_PARTIAL = 2, EPI_HADAMARD = 3, EPI_ADDSQUARE = 4, EPI_DIGITS = 5 };
 constexpr int DIG_PLANES = 7;  // digits of the mixed solve's ZC^T operand (ozaki.hip)
+enum { EPI_STORE = 0, EPI_SQUARE = 1, EPI_PARTIAL = 2, EPI_HADAMARD = 3, EPI_ADDSQUARE = 4 };
 
 struct KArgs {
   long m, n, k;
@@ -62,11 +62,6 @@ struct KArgs {
   int c_f32;
   long stride_a, stride_b, stride_c;
   long kchunk;  // split-K chunk (EPI_PARTIAL)
-  signed char* dig_out;  // EPI_DIGITS (see GemmArgs)
-  const double* dig_s;
-  const double* dig_inv2;
-  long dig_nr;
-  int dig_kp;
 };
 
 __device__ inline bool tile_coords(const KArgs& p, int BM, int BN, int& tm, int& tn) {
@@ -318,68 +313,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(KArgs p) {
     }
   }
 
-  if constexpr (EPI == EPI_DIGITS) {
-    // x = (acc^2 * inv2[col]) / s[row] cut into DIG_PLANES digits (x *= 128,
-    // d = trunc(x), x -= d: exact in FP64), the same arithmetic as the
-    // standalone split of ZC^T.  All planes of the tile are staged in the
-    // free operand LDS (planes 0-3 in As, 4-6 in Bs) as [32-column
-    // block][row][32 bytes], then, after one barrier, stored as whole 16-byte
-    // pieces of the k-blocked planes: a 4 KB contiguous run per block.
-    static_assert(sizeof(T) == 8 && BM == 128 && BN == 128 && DIG_PLANES == 7, "digit epilogue: FP64 128 x 128");
-    static_assert(sizeof(As) >= 4 * BM * BN && sizeof(Bs) >= 3 * BM * BN, "seven staged planes fit the operand LDS");
-    signed char* stg_a = reinterpret_cast<signed char*>(&As[0][0]);
-    signed char* stg_b = reinterpret_cast<signed char*>(&Bs[0][0]);
-    double x[TM][TN][4];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const long r = m0 + wm * WTM + i * 16 + Mfma<T>::row(lane, v);
-          const long cc = n0 + wn * WTN + j * 16 + l16;
-          double xv = 0.0;
-          if (r < p.m && cc < p.n) {
-            const double sr = p.dig_s[r];
-            const double isr = sr > 0.0 ? 1.0 / sr : 0.0;
-            const double a = p.alpha * acc[i][j][v];
-            xv = a * a * p.dig_inv2[cc] * isr;
-          }
-          x[i][j][v] = xv;
-        }
-    __syncthreads();  // every wave is past its last fragment read of As / Bs
-#pragma unroll
-    for (int q = 0; q < DIG_PLANES; ++q) {
-      signed char* stg = q < 4 ? stg_a + q * (BM * BN) : stg_b + (q - 4) * (BM * BN);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int rl = wm * WTM + i * 16 + Mfma<T>::row(lane, v);
-            const int cl = wn * WTN + j * 16 + l16;
-            x[i][j][v] *= 128.0;
-            const double d = trunc(x[i][j][v]);
-            x[i][j][v] -= d;
-            stg[(cl >> 5) * (BM * 32) + rl * 32 + (cl & 31)] = (signed char)(int)d;
-          }
-    }
-    __syncthreads();
-    const long plane = p.dig_nr * (long)p.dig_kp;
-#pragma unroll
-    for (int q = 0; q < DIG_PLANES; ++q) {
-      const signed char* stg = q < 4 ? stg_a + q * (BM * BN) : stg_b + (q - 4) * (BM * BN);
-      for (int t = tid; t < BM * BN / 16; t += NT) {
-        const int cb = t / (BM * 2), rem = t % (BM * 2), rl = rem >> 1, h = rem & 1;
-        const long gr = m0 + rl, gc = n0 + cb * 32;
-        if (gr < p.dig_nr && gc < p.dig_kp)
-          *reinterpret_cast<int4*>(p.dig_out + q * plane + (gc >> 5) * p.dig_nr * 32 + gr * 32 + h * 16) =
-              *reinterpret_cast<const int4*>(stg + cb * (BM * 32) + rl * 32 + h * 16);
-      }
-    }
-    return;
-  }
   if (EPI == EPI_PARTIAL) {
     const long tile_lin = (long)tm * (tm + 1) / 2 + tn;
     const long ntiles = gridDim.x;
@@ -579,6 +512,165 @@ __global__ __launch_bounds__(DTL_THREADS) void gemm_dtl_kernel(KArgs p) {
       }
 }
 
+// ---- ZC^T straight into the int8 solve's digit planes (ZctDigits) -----------
+// Tile of 128 grid rows r x 128 points nu, waves of 32 x 64 as above, both
+// operands contiguous along the orbitals, the points' rows gathered.  The
+// product is formed transposed (points along the D rows, so a lane holds one r
+// and four points of every MFMA block) and the points are staged in LDS in an
+// order that makes a lane's 4 x 4 points consecutive: its 16 digits of a plane
+// are one 16-byte store of the k-blocked layout, half a wave's store covers
+// 512 contiguous bytes, and the epilogue needs neither LDS nor a barrier: the
+// two workgroups of a CU run past each other, one cutting digits while the
+// other multiplies.  Bound by the FP64 product and the store of seven bytes an
+// element.  262144 x 2048 points with 128 orbitals: 3.1 ms, 4.2 with bytes
+// staged through LDS by one workgroup of a CU (44 TF/s, from 33; 64-row tiles,
+// three of a CU, made the whole factorisation 2.5 % slower); 884736 x 3456 with
+// 432 orbitals 43 ms, 50 with a stored product split afterwards; 110592 x 1024
+// half-rotated (128 and 64 orbitals) 1.1 ms, 2.0 as two products and a split.
+//
+// Digits: the value has at most 49 bits above its last digit; 21 of them, then
+// 28, are cut off as integers (exact: power-of-two scalings, a truncation and
+// the exact remainder), which gives the digits of the repeated
+// x = 128 x, d = trunc(x), x -= d.
+//
+// TWO: the half-rotated product P o Pocc with both factors accumulated side by
+// side.
+struct ZctArgs {
+  KArgs g;  // m = grid points, n = points; operands of the first factor
+  const double *a2, *b2;
+  long k2, lda2, ldb2;
+  signed char* out;
+  const double *sc, *inv2;
+  long nr;
+  int kp;
+};
+
+// byte b of words p[0] .. p[3] -> word b
+__device__ inline void bytes_transpose(const unsigned p[4], unsigned w[4]) {
+  const unsigned t0 = __builtin_amdgcn_perm(p[1], p[0], 0x05010400), t1 = __builtin_amdgcn_perm(p[3], p[2], 0x05010400);
+  const unsigned t2 = __builtin_amdgcn_perm(p[1], p[0], 0x07030602), t3 = __builtin_amdgcn_perm(p[3], p[2], 0x07030602);
+  w[0] = __builtin_amdgcn_perm(t1, t0, 0x05040100);
+  w[1] = __builtin_amdgcn_perm(t1, t0, 0x07060302);
+  w[2] = __builtin_amdgcn_perm(t3, t2, 0x05040100);
+  w[3] = __builtin_amdgcn_perm(t3, t2, 0x07060302);
+}
+
+template <bool TWO, bool VEC>
+__global__ __launch_bounds__(512, TWO ? 2 : 4) void zct_digits_kernel(ZctArgs z) {
+  constexpr int BM = 128, BN = 128, BK = 16, NT = 512, LEN = BK + 1;
+  constexpr int TM = 2, TN = 4, RA = BM * BK / NT, RB = BN * BK / NT;
+  __shared__ double As[2][BM * LEN], Bs[2][BN * LEN];
+  int tm, tn;
+  if (!tile_coords(z.g, BM, BN, tm, tn)) return;
+  const long m0 = (long)tm * BM, n0 = (long)tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1, l16 = lane & 15, l4 = lane >> 4;
+
+  const int a_line = tid / (BK / RA), a_off = tid % (BK / RA) * RA;
+  const int b_line = tid / (BK / RB), b_off = tid % (BK / RB) * RB;
+  const bool a_ok = m0 + a_line < z.g.m;
+  const long a_row = a_ok ? m0 + a_line : 0;
+  // LDS line 64 wn + 16 j + 4 v + g holds point 64 wn + 16 g + 4 j + v
+  const long gn = n0 + (b_line & 64) + 16 * (b_line & 3) + 4 * ((b_line >> 4) & 3) + ((b_line >> 2) & 3);
+  long b_row = gn < z.g.n ? (long)z.g.b_rows[gn] : -1;
+  const bool b_ok = b_row >= 0 && b_row < z.g.b_nrows;
+  if (!b_ok) b_row = 0;
+
+  auto product = [&](const double* a, long lda, const double* b, long ldb, long kend, d4(&acc)[TM][TN]) {
+    const double* ap = a + a_row * lda + a_off;
+    const double* bp = b + b_row * ldb + b_off;
+    double ra[RA], rb[RB];
+    auto load = [&](long k0) {
+      if (k0 + BK <= kend) {
+        load_run<double, RA>(ap + k0, ra, VEC);
+        load_run<double, RB>(bp + k0, rb, VEC);
+      } else {
+#pragma unroll
+        for (int e = 0; e < RA; ++e) ra[e] = k0 + a_off + e < kend ? ap[k0 + e] : 0.0;
+#pragma unroll
+        for (int e = 0; e < RB; ++e) rb[e] = k0 + b_off + e < kend ? bp[k0 + e] : 0.0;
+      }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+      for (int e = 0; e < RA; ++e) As[buf][a_line * LEN + a_off + e] = a_ok ? ra[e] : 0.0;
+#pragma unroll
+      for (int e = 0; e < RB; ++e) Bs[buf][b_line * LEN + b_off + e] = b_ok ? rb[e] : 0.0;
+    };
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    load(0);
+    store(0);
+    __syncthreads();
+    for (long k0 = 0; k0 < kend; k0 += BK) {
+      const int buf = (int)(k0 / BK) & 1;
+      if (k0 + BK < kend) load(k0 + BK);
+#pragma unroll
+      for (int k4 = 0; k4 < BK / 4; ++k4) {
+        double af[TM], bf[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) af[i] = As[buf][(wm * 32 + i * 16 + l16) * LEN + 4 * k4 + l4];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bf[j] = Bs[buf][(wn * 64 + j * 16 + l16) * LEN + 4 * k4 + l4];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = Mfma<double>::op(bf[j], af[i], acc[i][j]);
+      }
+      if (k0 + BK < kend) store(buf ^ 1);
+      __syncthreads();
+    }
+  };
+  d4 acc[TM][TN], acc2[TWO ? TM : 1][TWO ? TN : 1];
+  product(reinterpret_cast<const double*>(z.g.a), z.g.lda, reinterpret_cast<const double*>(z.g.b), z.g.ldb, z.g.k, acc);
+  if constexpr (TWO) product(z.a2, z.lda2, z.b2, z.ldb2, z.k2, acc2);
+
+  const long c0 = n0 + 64 * wn + 16 * l4;
+  if (c0 >= z.kp) return;
+  const long plane = z.nr * (long)z.kp;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const long r = m0 + 32 * wm + 16 * i + l16;
+    if (r >= z.nr) continue;
+    const double sr = r < z.g.m ? z.sc[r] : 0.0;
+    const double isr = sr > 0.0 ? 1.0 / sr : 0.0;
+    unsigned w[DIG_PLANES][4];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      unsigned hi[4], lo[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        double x = acc[i][j][v];
+        if constexpr (TWO) x = acc2[i][j][v] * x;
+        else x = x * x;
+        x = x * z.inv2[c0 + 4 * j + v] * isr;
+        const double y = fabs(x) * 0x1p21, t = trunc(y);
+        const unsigned h = (unsigned)t, l = (unsigned)((y - t) * 0x1p28);
+        hi[v] = ((h >> 14) & 0xffu) | ((h << 1) & 0x7f00u) | ((h << 16) & 0x7f0000u);
+        lo[v] = ((l >> 21) & 0x7fu) | ((l >> 6) & 0x7f00u) | ((l << 9) & 0x7f0000u) |
+                ((l << 24) & 0x7f000000u);
+        if (TWO && x < 0.0) {  // every digit takes the sign
+          hi[v] = (0x80808080u - hi[v]) ^ 0x80808080u;
+          lo[v] = (0x80808080u - lo[v]) ^ 0x80808080u;
+        }
+      }
+      unsigned wh[4], wl[4];
+      bytes_transpose(hi, wh);
+      bytes_transpose(lo, wl);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[q][j] = wh[q];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) w[3 + q][j] = wl[q];
+    }
+    signed char* o = z.out + (c0 >> 5) * z.nr * 32 + r * 32 + (c0 & 16);
+#pragma unroll
+    for (int q = 0; q < DIG_PLANES; ++q)
+      *reinterpret_cast<uint4*>(o + q * plane) = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
+  }
+}
+
 // V = FP64 sum over the split-K partials (in split order), mirrored to the
 // upper triangle: one workgroup per 32 x 32 block of a lower tile, thread t
 // owning row t / 8 and columns 4 (t % 8) .. + 3; the mirror image goes
@@ -630,7 +722,6 @@ KArgs make_args(const GemmArgs& g) {
   p.tri = g.tri;
   p.c_f32 = g.c_f32;
   p.stride_a = g.stride_a; p.stride_b = g.stride_b; p.stride_c = g.stride_c;
-  p.dig_out = g.dig_out; p.dig_s = g.dig_s; p.dig_inv2 = g.dig_inv2; p.dig_nr = g.dig_nr; p.dig_kp = g.dig_kp;
   return p;
 }
 
@@ -684,26 +775,6 @@ int launch_layout(const GemmArgs& g, const KArgs& p, dim3 grid, hipStream_t s) {
 template <class T, class C>
 int launch(const GemmArgs& g, hipStream_t s) {
   const KArgs p = make_args(g);
-  if (g.epi_digits) {
-    // B rows gathered, both operands k-contiguous, the deep-k tile (its
-    // operand LDS holds one staged digit plane)
-    if constexpr (std::is_same<T, double>::value && std::is_same<C, CfgDeepK>::value) {
-      if (g.lower || g.tri || g.a_rows || !g.b_rows || g.a_trans != 0 || g.b_trans != 1 || g.batch != 1 ||
-          g.epi_square || g.epi_hadamard || g.epi_addsquare || !g.dig_out || !g.dig_s || !g.dig_inv2 ||
-          g.dig_kp % 32 != 0 || g.dig_nr % 64 != 0)
-        return THC_ERR_ARG;
-      const long nblk = ((g.m + C::BM - 1) / C::BM) * ((g.n + C::BN - 1) / C::BN);
-      if (nblk <= 0) return THC_OK;
-      if (nblk > 0x7fffffffL) return THC_ERR_ARG;
-      const int vw = 16 / (int)sizeof(T);
-      const bool vec = aligned16(g.a) && aligned16(g.b) && g.lda % vw == 0 && g.ldb % vw == 0;
-      launch_vec<T, C, EPI_DIGITS, true, true, false, true>(p, vec, dim3((unsigned)nblk), s);
-      THC_HIP(hipGetLastError());
-      return THC_OK;
-    } else {
-      return THC_ERR_ARG;
-    }
-  }
   const long nbm = (g.m + C::BM - 1) / C::BM, nbn = (g.n + C::BN - 1) / C::BN;
   const long nblk = g.lower ? nbm * (nbm + 1) / 2 : nbm * nbn;
   if (nblk <= 0 || g.batch <= 0) return THC_OK;
@@ -797,7 +868,6 @@ int gemm_dispatch(const GemmArgs& g, hipStream_t s) {
   if (g.c_f32 && (sizeof(T) != 8 || g.beta != 0.0 || g.epi_square || g.epi_hadamard || g.epi_addsquare))
     return THC_ERR_ARG;
   if (g.cfg < 0 || g.cfg >= GEMM_CFG_COUNT) return THC_ERR_ARG;
-  if (g.epi_digits) return launch<T, CfgDeepK>(g, s);
   const int cfg = g.cfg != GEMM_CFG_AUTO ? g.cfg : tuned_cfg(g);
   if (cfg != GEMM_CFG_AUTO) {
     const int r = launch_cfg<T>(g, cfg, s);
@@ -824,6 +894,27 @@ int gemm_dispatch(const GemmArgs& g, hipStream_t s) {
 constexpr int SY_BM = CfgLarge::BM, SY_BN = CfgLarge::BN, SY_BK = CfgLarge::BK;
 
 }  // namespace
+
+int zct_digits(const ZctDigits& d, hipStream_t s) {
+  ZctArgs z = {};
+  z.g.m = d.n; z.g.n = d.k; z.g.k = d.ma;
+  z.g.a = d.phi_a; z.g.lda = d.ma;
+  z.g.b = d.phi_a; z.g.ldb = d.ma; z.g.b_rows = d.idx; z.g.b_nrows = d.n;
+  z.a2 = d.phi_b; z.b2 = d.phi_b; z.k2 = z.lda2 = z.ldb2 = d.mb;
+  z.out = d.out; z.sc = d.sc; z.inv2 = d.inv2; z.nr = d.nr; z.kp = d.kp;
+  if (d.n <= 0 || d.k <= 0) return THC_OK;
+  if (d.kp % 32 != 0 || d.kp < d.k || d.nr % 64 != 0 || d.nr < d.n) return THC_ERR_ARG;
+  const bool vec = aligned16(d.phi_a) && d.ma % 2 == 0 && (!d.phi_b || (aligned16(d.phi_b) && d.mb % 2 == 0));
+  const long nblk = ((d.n + 127) / 128) * ((d.k + 127) / 128);
+  if (nblk > 0x7fffffffL) return THC_ERR_ARG;
+  const dim3 grid((unsigned)nblk), block(512);
+  if (d.phi_b && vec) hipLaunchKernelGGL((zct_digits_kernel<true, true>), grid, block, 0, s, z);
+  else if (d.phi_b) hipLaunchKernelGGL((zct_digits_kernel<true, false>), grid, block, 0, s, z);
+  else if (vec) hipLaunchKernelGGL((zct_digits_kernel<false, true>), grid, block, 0, s, z);
+  else hipLaunchKernelGGL((zct_digits_kernel<false, false>), grid, block, 0, s, z);
+  THC_HIP(hipGetLastError());
+  return THC_OK;
+}
 
 int gemm_tune_flags(const GemmArgs& g) {
   return (g.a_rows || g.b_rows ? 1 : 0) | (g.lower ? 2 : 0) | (g.epi_square ? 4 : 0) | (g.tri ? 8 : 0);

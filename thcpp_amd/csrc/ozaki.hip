@@ -707,19 +707,13 @@ size_t oz_solve_work_bytes(int k, long n) {
          align_up(sizeof(double) * (size_t)P.kp, 256) + 1024;
 }
 
-int oz_solve_prepare(int k, long n, const int* idx, const double* phi_a, int ma, void* work, GemmArgs& g,
-                     hipStream_t s) {
+int oz_solve_zct(int k, long n, const int* idx, const double* phi_a, int ma, const double* phi_b, int mb, void* work,
+                 hipStream_t s) {
   if (k <= 0 || n <= 0) return THC_OK;
   const SvPlan P = sv_plan(k, n);
   const SvWork W = sv_carve(P, n, work);
-  THC_TRY(sv_scales(P, W, k, n, idx, phi_a, ma, nullptr, 0, s));
-  g.epi_digits = 1;
-  g.dig_out = W.SZ;
-  g.dig_s = W.sc;
-  g.dig_inv2 = W.inv2;
-  g.dig_nr = P.nr;
-  g.dig_kp = P.kp;
-  return THC_OK;
+  THC_TRY(sv_scales(P, W, k, n, idx, phi_a, ma, phi_b, mb, s));
+  return zct_digits({n, k, idx, phi_a, phi_b, ma, mb, W.SZ, W.sc, W.inv2, P.nr, P.kp}, s);
 }
 
 namespace {
