@@ -69,6 +69,21 @@ def test_cholesky_not_posdef(ctx, k, bad):
     assert info == bad + 1
 
 
+@pytest.mark.parametrize("k,g", [(1, 16), (127, 48), (128, 65552), (129, 4112), (300, 131072), (1024, 1040), (400, 99),
+                                 (2100, 2064)])
+def test_muv_splits(ctx, k, g):
+    """V = B B^T over every kind of split: fewer columns than a split, one split,
+    workgroup counts that are no multiple of the eight XCDs, an odd row length;
+    elementwise within the rounding of g products summed in any order."""
+    b = np.random.default_rng(k + g).standard_normal((k, g))
+    v = ctx.construct_muv(b).cpu().numpy()
+    np.testing.assert_array_equal(v, v.T)
+    r = np.random.default_rng(1).integers(0, k, 40)
+    ref = np.longdouble(b[r]) @ np.longdouble(b[r].T)
+    bound = (np.sqrt(g) * 8 + 16) * 2.0 ** -53 * (np.abs(b[r]) @ np.abs(b[r].T))
+    assert (np.abs(v[np.ix_(r, r)] - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("k", [15, 16, 17, 33, 47, 48, 49, 79, 81, 143])
 def test_cholesky_panel_edges(ctx, k):
     """Block edges inside the 64-column block.  Componentwise backward error

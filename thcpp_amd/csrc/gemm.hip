@@ -64,6 +64,14 @@ struct KArgs {
   long kchunk;  // split-K chunk (EPI_PARTIAL)
 };
 
+__device__ inline void lower_coords(int id, int& tm, int& tn) {
+  int t = (int)((sqrt(8.0 * id + 1.0) - 1.0) * 0.5);
+  while ((long)(t + 1) * (t + 2) / 2 <= id) ++t;
+  while ((long)t * (t + 1) / 2 > id) --t;
+  tm = t;
+  tn = id - t * (t + 1) / 2;
+}
+
 __device__ inline bool tile_coords(const KArgs& p, int BM, int BN, int& tm, int& tn) {
   const int nbm = (int)((p.m + BM - 1) / BM);
   const int nbn = (int)((p.n + BN - 1) / BN);
@@ -72,11 +80,7 @@ __device__ inline bool tile_coords(const KArgs& p, int BM, int BN, int& tm, int&
   // ids reach the 8 XCDs round-robin: give each XCD a contiguous run of tiles
   if ((nb & 7) == 0) id = (id & 7) * (nb >> 3) + (id >> 3);
   if (p.lower) {
-    int t = (int)((sqrt(8.0 * id + 1.0) - 1.0) * 0.5);
-    while ((long)(t + 1) * (t + 2) / 2 <= id) ++t;
-    while ((long)t * (t + 1) / 2 > id) --t;
-    tm = t;
-    tn = id - t * (t + 1) / 2;
+    lower_coords(id, tm, tn);
     return tm < nbm;
   }
   // walk groups of up to 4 tile rows column by column: the B column block a
@@ -372,8 +376,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(KArgs p) {
 // order is permuted so one 16-byte read feeds two k-steps: in half h, k-step s,
 // lane group l4 contributes k = 8 h + 2 l4 + s of both operands.  Rows past m
 // (n) read row m - 1 (n - 1); they only feed outputs that are never stored.
-// PARTIAL: split-K partial tiles of the lower triangle (blockIdx.y = split,
-// k range [y kchunk, min(k, (y + 1) kchunk))), stored whole as in gemm_kernel.
+// PARTIAL: split-K partial tiles of the lower triangle (one workgroup per tile
+// and split y, k range [y kchunk, min(k, (y + 1) kchunk))), stored whole.
 typedef __attribute__((address_space(3))) void lds_void;
 constexpr int DTL_BM = 128, DTL_BN = 128, DTL_BK = 16, DTL_WN = 2, DTL_THREADS = 512;
 
@@ -394,8 +398,21 @@ __global__ __launch_bounds__(DTL_THREADS) void gemm_dtl_kernel(KArgs p) {
   // wait for the loads before reading
   __shared__ __attribute__((aligned(16))) double As0[BM * BK], As1[BM * BK];
   __shared__ __attribute__((aligned(16))) double Bs0[BN * BK], Bs1[BN * BK];
-  int tm, tn;
-  if (!tile_coords(p, BM, BN, tm, tn)) return;
+  int tm, tn, tile = 0, split = 0;
+  if (PARTIAL) {
+    // each XCD (workgroup i runs on XCD i % 8) takes whole splits one after the
+    // other, so a column of the operand reaches one L2 instead of all eight
+    // (with the split counts of syrk_plan: V of 1024 x 270336 in FP64 5.00 ->
+    // 4.59 ms, 69.5 TF/s of 72.7; leaving out the upper halves of the diagonal
+    // tiles gave nothing on top, the clock makes up for idle matrix cores)
+    const int id = blockIdx.y * gridDim.x + blockIdx.x, total = gridDim.x * gridDim.y;
+    const int xcd = id & 7, item = xcd * (total >> 3) + min(xcd, total & 7) + (id >> 3);
+    tile = item % (int)gridDim.x;
+    split = item / (int)gridDim.x;
+    lower_coords(tile, tm, tn);
+  } else if (!tile_coords(p, BM, BN, tm, tn)) {
+    return;
+  }
   const long m0 = (long)tm * BM, n0 = (long)tn * BN;
   const int bz = blockIdx.z;
   const double* A = reinterpret_cast<const double*>(p.a) + (long)bz * p.stride_a;
@@ -433,7 +450,7 @@ __global__ __launch_bounds__(DTL_THREADS) void gemm_dtl_kernel(KArgs p) {
 
   long kbeg = 0, kend = p.k;
   if (PARTIAL) {
-    kbeg = (long)blockIdx.y * p.kchunk;
+    kbeg = (long)split * p.kchunk;
     kend = min(p.k, kbeg + p.kchunk);
   }
   const long nk = (kend - kbeg) / BK;
@@ -476,8 +493,7 @@ __global__ __launch_bounds__(DTL_THREADS) void gemm_dtl_kernel(KArgs p) {
   }
 
   if (PARTIAL) {
-    const long tile_lin = (long)tm * (tm + 1) / 2 + tn;
-    double* W = reinterpret_cast<double*>(p.c) + ((long)blockIdx.y * gridDim.x + tile_lin) * (BM * BN);
+    double* W = reinterpret_cast<double*>(p.c) + ((long)split * gridDim.x + tile) * (BM * BN);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -878,12 +894,10 @@ int gemm_dispatch(const GemmArgs& g, hipStream_t s) {
   long tiles64 = ((g.m + 63) / 64) * ((g.n + 63) / 64);
   if (g.lower) tiles64 = (tiles64 + (g.m + 63) / 64) / 2;
   tiles64 *= g.batch;
-  // The ZC^T GEMM (N x K output, inner dimension M): with one workgroup per CU
-  // a CU empties completely whenever a tile finishes, and the latency-bound
-  // CC^T Cholesky and inverse on the second stream get CUs between tiles; two
-  // workgroups per CU finish out of step and keep every CU occupied.  Measured:
-  // ZC^T 3.8 ms with the second stream hidden, against 2.9 ms + 1.6 ms exposed.
-  if (g.k <= 256 && g.m >= 65536 && !g.lower) return launch<T, CfgDeepK>(g, s);
+  // The ZC^T GEMM (N x K output, inner dimension M): short tiles with a long
+  // epilogue, so two workgroups per CU, whatever the count (262144 x 1024 x 128
+  // in FP64: 1.30 ms, with one workgroup per CU on the deep-k tile 1.49)
+  if (g.k <= 256 && g.m >= 65536 && !g.lower) return launch<T, CfgLarge>(g, s);
   // too few 64 x 64 tiles to fill 256 CUs a few times over: single-wave tiles
   if (tiles64 < 1024) return launch<T, CfgTiny>(g, s);
   if (tiles128 < 512) return launch<T, CfgSmall>(g, s);
@@ -939,8 +953,19 @@ int gemm_f32(const GemmArgs& g, hipStream_t s) { return gemm_dispatch<float>(g, 
 static void syrk_plan(long m, long k, long& ntiles, int& nsplit, long& kchunk) {
   const long nb = (m + SY_BM - 1) / SY_BM;
   ntiles = nb * (nb + 1) / 2;
-  long want = (2048 + ntiles - 1) / ntiles;
-  long maxsplit = (k + 4 * SY_BK - 1) / (4 * SY_BK);
+  // Splits: the count up to 2048 workgroups that fills the last round of the 512
+  // resident ones best (57 splits of the 36 tiles at m = 1024 left four
+  // workgroups to a fifth round), with 1024 or more k per split where 512
+  // workgroups allow it: each one writes a 128 KB partial.
+  long want = 1;
+  double best = 0.0;
+  for (long w = 1; w * ntiles <= 2048; ++w) {
+    if (w * ntiles > 512 && k / w < 1024) break;
+    const long rounds = (w * ntiles + 511) / 512;
+    const double fill = (double)(w * ntiles) / (512.0 * rounds);
+    if (fill >= best) best = fill, want = w;
+  }
+  const long maxsplit = (k + 4 * SY_BK - 1) / (4 * SY_BK);
   if (want > maxsplit) want = maxsplit;
   if (want < 1) want = 1;
   kchunk = (k + want - 1) / want;
