@@ -329,3 +329,34 @@ def test_isdf_solve_large_tiles(ctx, n, k):
     e = rel(out["xi"].cpu().numpy(), xr)
     print("k %d cond(CC^T) %.2e rel xi %.3e" % (k, cond, e))
     assert e < max(1e-13, 1e-15 * cond) and e < 1e-6
+
+
+@pytest.mark.parametrize("grid", [(1, 1, 1), (2, 2, 2), (3, 1, 8), (8, 4, 5), (4, 9, 1), (9, 25, 27), (20, 3, 25),
+                                  (50, 50, 50), (64, 60, 54), (72, 96, 64), (15, 8, 128), (100, 128, 6)])
+def test_fft_stage_classes(ctx, grid):
+    """Transforms of one stage (read from memory and stored by the same
+    butterflies), of length one (no stage), an odd number of rows, and grids in
+    every register class of the run-time plans.  At most 9 stages, each within
+    4 roundings of 2^-53 of the line's norm: 4e-15."""
+    rng = np.random.default_rng(sum(grid))
+    n = int(np.prod(grid))
+    x = rng.standard_normal((3, n))
+    cg = rng.random(n) + 0.5
+    got = ctx.fft_vectors(x, grid, cg).cpu().numpy()
+    assert rel(got, _half_spectrum_ref(x, grid, cg)) < 4e-15
+
+
+@pytest.mark.parametrize("grid", [(5, 6, 4), (9, 5, 8), (2, 12, 16), (25, 3, 5), (50, 4, 18)])
+def test_mixed_digits_of_short_lines(ctx, grid):
+    """Digits are stored two values at a time: lines with an odd number of values
+    and run-time plans.  V of six points against FP64; FP32 rounding of xi and
+    of at most 6 stages and the weights, 2^-24 each, twice in V: 1e-6."""
+    from thcpp_amd import synthetic
+    rng = np.random.default_rng(sum(grid))
+    n = int(np.prod(grid))
+    a = rng.standard_normal((n, 6))
+    idx = np.sort(rng.choice(n, 6, replace=False)).astype(np.int32)
+    cg = synthetic.coulomb_kernel(5.0, grid)
+    ref = ctx.isdf(a, idx, grid, cg, precision=L.PREC_FP64, want_luv=False)["V"].cpu().numpy()
+    got = ctx.isdf(a, idx, grid, cg, precision=L.PREC_MIXED, want_luv=False)["V"].cpu().numpy()
+    assert rel(got, ref) < 1e-6

@@ -22,17 +22,26 @@
 //
 // LDS layout: every transform line is contiguous, lines ls = n rounded up to
 // 32 elements apart, and element pos of line l sits at l ls + (pos ^ h(l)).
-// The XOR spreads the lines of one wave over the banks: a Stockham read takes
-// elements t + q nb of 8 lines (t < 8 across lanes) and a first-stage write
-// elements 8 t + q; h puts the line in bits 0-2 and bits 3-4 of the position,
-// so both touch every bank pair once per 32 lanes.  The transposes between
-// transforms (z-lines to y-lines, the strided x-lines of the global layout)
-// are done on the way into LDS, so no stage reads a strided line.
+// The XOR spreads the lines of one wave over the banks (h puts the line in bits
+// 0-2 and bits 3-4 of the position): the same element of 32 consecutive lines
+// touches every bank pair once, and so do 8 consecutive elements of 4 lines.
+// The transposes between transforms (z-lines to y-lines, the strided x-lines of
+// the global layout) lie in the reads of a first stage or the stores of a last
+// one.
 //
-// The passes are bound by their VALU work (index arithmetic of the LDS
-// stages as much as the butterflies), so cubic grids of the common edges (32,
-// 64, 96) run instantiations compiled for their size: every divisor, stride,
-// twiddle step and loop bound is a constant (64^3 FP32 pass A: 1.60 -> 1.18 ms).
+// Each transform's first stage reads where its data is (memory, or for y the
+// spectrum of z being unpacked) and the last stage along y and x stores to
+// memory, so a 64-point pass A goes through LDS three times and pass B once
+// (twice with digits), where loading, unpacking and storing each took a round
+// trip and two barriers.  64^3, 1024 vectors, FP64: pass A 1.24 -> 0.81 ms, pass
+// B 1.23 -> 1.00 ms (4.4 TB/s, a 2 GB copy reaches 4.9); 2048 vectors in FP32:
+// 1.19 -> 0.78 ms and, with digits, 1.24 -> 1.07 ms; 48 x 45 x 40, 512 vectors,
+// FP64: 0.54 -> 0.39 ms in all.  Measured and dropped: pass B's workgroups in
+// contiguous runs per XCD (cubes within 2 %, 48 x 45 x 40 10 % slower).
+//
+// The index arithmetic of the LDS stages costs as much as the butterflies, so
+// cubic grids of the common edges run instantiations compiled for their size:
+// every divisor, stride, twiddle step and loop bound is a constant.
 #include <tuple>
 #include <algorithm>
 #include <type_traits>
@@ -70,14 +79,39 @@ struct Plan1D {
   int n;
   int nst;
   int rad[MAXR];
+  // stage s: length ns of the transforms it joins, the magic number of a
+  // division by ns (FDiv), and its twiddle step n / (ns rad)
+  int ns[MAXR];
+  unsigned mns[MAXR];
+  int tstep[MAXR];
 };
+constexpr unsigned fdiv_magic(int d) { return d > 1 ? 0xFFFFFFFFu / (unsigned)d + 1u : 0u; }
+
+// The plan of a length: radix 8, then 4, 2, 3, 5 (pl.n = 0 where it has another
+// factor).
+constexpr Plan1D plan_of(int n) {
+  Plan1D pl{};
+  int m = n, ns = 1;
+  const int rs[5] = {8, 4, 2, 3, 5};
+  for (int i = 0; i < 5; ++i)
+    while (m % rs[i] == 0 && pl.nst < MAXR) {
+      const int s = pl.nst++;
+      pl.rad[s] = rs[i];
+      pl.ns[s] = ns;
+      pl.mns[s] = fdiv_magic(ns);
+      pl.tstep[s] = n / (ns * rs[i]);
+      ns *= rs[i];
+      m /= rs[i];
+    }
+  pl.n = m == 1 ? n : 0;
+  return pl;
+}
 
 struct FftParams {
   int k, n0, n1, n2, n2h;
   int lsz, lsy, lsx;  // LDS line strides of the z, y and x transforms
   Plan1D pz, py, px;
   const void* twz; const void* twy; const void* twx;
-  int vec_out;  // output aligned to two elements: one vector store per complex value
   signed char* dig_s;  // digit output of pass B (FftDigits): planes, exponents, strides
   int* dig_e;
   long dig_plane, dig_row;
@@ -90,7 +124,8 @@ struct FftParams {
 // Here e < 2^14 and d <= 128.
 struct FDiv {
   unsigned d, m;
-  __device__ explicit FDiv(int dd) : d((unsigned)dd), m(dd > 1 ? 0xFFFFFFFFu / (unsigned)dd + 1u : 0u) {}
+  __device__ explicit FDiv(int dd) : d((unsigned)dd), m(fdiv_magic(dd)) {}
+  __device__ FDiv(int dd, unsigned mm) : d((unsigned)dd), m(mm) {}
   __device__ int div(int e) const { return d > 1 ? (int)__umulhi((unsigned)e, m) : e; }
 };
 
@@ -210,64 +245,116 @@ __device__ C2<T>* fft_lines(C2<T>* a, C2<T>* b, const Plan1D& pl, int nlines, in
   return a;
 }
 
-// In-place variant: each thread reads the inputs of all its butterflies (at
-// most IPV / R of them) into registers, then after a barrier writes the
-// outputs into the same buffer.  One LDS buffer instead of two lets a CU hold
-// up to twice the workgroups, which is what these latency-bound passes need;
-// the smaller IPV budget (16 complex values) keeps FP32 passes at about 64
-// VGPRs and seven workgroups per CU, 24 covers 96-point lines.
+// One stage whose inputs and outputs stay with the caller: load(line, pos)
+// gives an element, store(i, q, line, pos, y) takes output q of the thread's
+// butterfly i.  Each thread reads the inputs of all its butterflies (at most
+// NB) before it writes any output; with SYNC a barrier lies between, and one
+// LDS buffer is enough.
+// Lines run fastest over the threads (LF): the lanes of a wave then read and
+// write one position of consecutive lines, which the XOR of swz spreads over
+// the banks, share their twiddles, and meet the global layouts of the last
+// transform along y and both ends of the one along x, where consecutive lines
+// are consecutive in memory.
 constexpr int FT = 256;  // threads per workgroup of both passes
 
-template <class T, int R, int IPV>
-__device__ inline void stage_ip(C2<T>* buf, int n, int ns, int nlines, int ls, const C2<T>* __restrict__ tw) {
-  constexpr int NB = IPV / R > 0 ? IPV / R : 1;
+template <class T, int R, int NB, bool LF, bool SYNC, class Load, class Store>
+__device__ __forceinline__ void stage_io(int n, int ns, FDiv fns, int tstep, int nlines, FDiv fw,
+                                         const C2<T>* __restrict__ tw, Load load, Store store) {
   const int nb = n / R;
   const int total = nlines * nb;
-  const int tstep = n / (ns * R);
-  const FDiv fnb(nb), fns(ns);
   C2<T> x[NB][R];
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     const int w = threadIdx.x + i * FT;
     if (w < total) {
-      const int line = fnb.div(w), t = w - line * nb;
+      const int hi = fw.div(w), lo = w - hi * (LF ? nlines : nb);
+      const int line = LF ? lo : hi, t = LF ? hi : lo;
 #pragma unroll
-      for (int q = 0; q < R; ++q) x[i][q] = buf[swz(line, t + q * nb, ls)];
+      for (int q = 0; q < R; ++q) x[i][q] = load(line, t + q * nb);
     }
   }
-  __syncthreads();
+  if (SYNC) __syncthreads();
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     const int w = threadIdx.x + i * FT;
     if (w < total) {
-      const int line = fnb.div(w), t = w - line * nb;
+      const int hi = fw.div(w), lo = w - hi * (LF ? nlines : nb);
+      const int line = LF ? lo : hi, t = LF ? hi : lo;
       const int tq = fns.div(t), j = t - tq * ns;
       C2<T> y[R];
       butterfly<T, R>(x[i], y, n, ns, j, tstep, tw);
       const int d0 = tq * ns * R + j;
 #pragma unroll
-      for (int q = 0; q < R; ++q) buf[swz(line, d0 + q * ns, ls)] = y[q];
+      for (int q = 0; q < R; ++q) store(i, q, line, d0 + q * ns, y[q]);
     }
   }
-  __syncthreads();
 }
 
-template <class T, int IPV>
-__device__ void fft_lines_ip(C2<T>* buf, const Plan1D& pl, int nlines, int ls, const C2<T>* tw) {
-  int ns = 1;
-  for (int s = 0; s < pl.nst; ++s) {
-    const int r = pl.rad[s];
-    if (r == 8) stage_ip<T, 8, IPV>(buf, pl.n, ns, nlines, ls, tw);
-    else if (r == 4) stage_ip<T, 4, IPV>(buf, pl.n, ns, nlines, ls, tw);
-    else if (r == 2) stage_ip<T, 2, IPV>(buf, pl.n, ns, nlines, ls, tw);
-    else if (r == 3) stage_ip<T, 3, IPV>(buf, pl.n, ns, nlines, ls, tw);
-    else stage_ip<T, 5, IPV>(buf, pl.n, ns, nlines, ls, tw);
-    ns *= r;
+// Stage s of a plan, f(radix, values), radix an integral constant: of the
+// run-time plan, or (N > 0) of the plan of length N with s = S.
+template <int N, int S, class F>
+__device__ __forceinline__ void with_radix(const Plan1D& pl, int s, F f) {
+  if constexpr (N > 0) {
+    constexpr Plan1D cp = plan_of(N);
+    f(std::integral_constant<int, cp.rad[S]>{}, cp.ns[S], FDiv(cp.ns[S]), cp.tstep[S]);
+  } else {
+    const FDiv fns(pl.ns[s], pl.mns[s]);
+    switch (pl.rad[s]) {
+      case 8: f(std::integral_constant<int, 8>{}, pl.ns[s], fns, pl.tstep[s]); break;
+      case 4: f(std::integral_constant<int, 4>{}, pl.ns[s], fns, pl.tstep[s]); break;
+      case 2: f(std::integral_constant<int, 2>{}, pl.ns[s], fns, pl.tstep[s]); break;
+      case 3: f(std::integral_constant<int, 3>{}, pl.ns[s], fns, pl.tstep[s]); break;
+      default: f(std::integral_constant<int, 5>{}, pl.ns[s], fns, pl.tstep[s]); break;
+    }
+  }
+}
+
+// A transform of nlines lines through the LDS buffer: first(line, pos) supplies
+// the inputs of its first stage (LF1: line-fast; SYNC1: they come from the
+// buffer itself), last(i, q, line, pos, y) takes the outputs of its last unless
+// TOBUF.  Its stages in between, and all that TOBUF adds, go through the buffer
+// in place; every write to the buffer is followed by a barrier.
+template <class T, int IPV, int N, bool LF1, bool SYNC1, bool TOBUF, int S = 0, class First, class Last>
+__device__ __forceinline__ void fft_lines_io(C2<T>* buf, const Plan1D& pl, int n, int nlines, int ls,
+                                             const C2<T>* tw, First first, Last last) {
+  const FDiv fl(nlines);
+  auto rd = [&](int line, int pos) { return buf[swz(line, pos, ls)]; };
+  auto wr = [&](int, int, int line, int pos, C2<T> y) { buf[swz(line, pos, ls)] = y; };
+  auto one = [&](auto first_stage, auto last_stage, auto st, int s) {
+    constexpr bool F = decltype(first_stage)::value, L = decltype(last_stage)::value && !TOBUF;
+    with_radix<N, decltype(st)::value>(pl, s, [&](auto r, int ns, FDiv fns, int tstep) {
+      constexpr int R = decltype(r)::value, NB = IPV / R > 0 ? IPV / R : 1;
+      constexpr bool LF = !F || LF1;
+      const FDiv fw = LF ? fl : FDiv(n / R);
+      if constexpr (F && L) stage_io<T, R, NB, LF, false>(n, ns, fns, tstep, nlines, fw, tw, first, last);
+      else if constexpr (F) stage_io<T, R, NB, LF, SYNC1>(n, ns, fns, tstep, nlines, fw, tw, first, wr);
+      else if constexpr (L) stage_io<T, R, NB, LF, false>(n, ns, fns, tstep, nlines, fw, tw, rd, last);
+      else stage_io<T, R, NB, LF, true>(n, ns, fns, tstep, nlines, fw, tw, rd, wr);
+    });
+    if constexpr (!L) __syncthreads();
+  };
+  using std::false_type;
+  using std::true_type;
+  if constexpr (N > 0) {
+    constexpr int nst = plan_of(N).nst;
+    one(std::bool_constant<S == 0>{}, std::bool_constant<S == nst - 1>{}, std::integral_constant<int, S>{}, S);
+    if constexpr (S + 1 < nst)
+      fft_lines_io<T, IPV, N, LF1, SYNC1, TOBUF, S + 1>(buf, pl, n, nlines, ls, tw, first, last);
+  } else {
+    const std::integral_constant<int, 0> z{};
+    if (pl.nst == 1) {
+      one(true_type{}, true_type{}, z, 0);
+    } else {
+      one(true_type{}, false_type{}, z, 0);
+      for (int s = 1; s < pl.nst - 1; ++s) one(false_type{}, false_type{}, z, s);
+      one(false_type{}, true_type{}, z, pl.nst - 1);
+    }
   }
 }
 
 // Whether every stage of a plan over nlines lines keeps to ipv values per thread.
 bool fits_ip(const Plan1D& pl, int nlines, int ipv) {
+  if (pl.nst == 0) return false;  // one point: no stage to load or store through
   for (int s = 0; s < pl.nst; ++s) {
     const int r = pl.rad[s];
     const long per = ((long)nlines * (pl.n / r) + FT - 1) / FT;
@@ -275,41 +362,17 @@ bool fits_ip(const Plan1D& pl, int nlines, int ipv) {
   }
   return true;
 }
-constexpr int UPV = 12;  // elements per thread of the in-place unpack
-
-// The plan of a transform length known at compile time (make_plan's rule:
-// radix 8, then 4, 2, 3, 5).
-constexpr Plan1D plan_of(int n) {
-  Plan1D pl{};
-  pl.n = n;
-  pl.nst = 0;
-  int m = n;
-  const int rs[5] = {8, 4, 2, 3, 5};
-  for (int i = 0; i < 5; ++i)
-    while (m % rs[i] == 0 && pl.nst < MAXR) {
-      pl.rad[pl.nst++] = rs[i];
-      m /= rs[i];
-    }
-  return pl;
-}
-
-// fft_lines_ip for a length N fixed at compile time: the stages unrolled, so
-// every index divisor, twiddle stride and loop bound is a constant.
-template <class T, int IPV, int N, int S = 0, int NS = 1>
-__device__ __forceinline__ void fft_lines_ct(C2<T>* buf, int nlines, int ls, const C2<T>* tw) {
-  constexpr Plan1D pl = plan_of(N);
-  if constexpr (S < pl.nst) {
-    constexpr int R = pl.rad[S];
-    stage_ip<T, R, IPV>(buf, N, NS, nlines, ls, tw);
-    fft_lines_ct<T, IPV, N, S + 1, NS * R>(buf, nlines, ls, tw);
-  }
-}
+// Waves per SIMD asked of the compiler.  The FP64 kernels with run-time plans and
+// 12 values take 132 VGPRs unasked, three waves, and 128 without a spill; the
+// larger budgets spill at one wave more and lose by it (100 x 128 x 72: 0.98
+// -> 1.31 ms).
+constexpr int min_waves(size_t elem, int ipv, int cn) { return elem == 8 && ipv == 12 && cn == 0 ? 4 : 1; }
 
 // x: (k, n0, n1, n2) real, FP64 or FP32 (rounded to T as it is read); t: (k,
 // n0, n1, n2h) complex.  CN > 0: a cubic grid of edge CN, compiled for that
 // size (in-place stages only); 0: sizes and plans from p.
 template <class T, int IPV, class X, int CN = 0>  // IPV = 0: ping-pong stages
-__global__ __launch_bounds__(FT) void pass_a(const X* __restrict__ x, C2<T>* __restrict__ t, FftParams p) {
+__global__ __launch_bounds__(FT, min_waves(sizeof(T), IPV, CN)) void pass_a(const X* __restrict__ x, C2<T>* __restrict__ t, FftParams p) {
   constexpr bool ip = IPV > 0;
   static_assert(CN == 0 || ip, "compile-time sizes use the in-place stages");
   extern __shared__ unsigned char smem_raw[];
@@ -327,61 +390,52 @@ __global__ __launch_bounds__(FT) void pass_a(const X* __restrict__ x, C2<T>* __r
   for (int j = threadIdx.x; j < n1; j += blockDim.x) twy[j] = reinterpret_cast<const C2<T>*>(p.twy)[j];
   const int n0 = CN ? CN : p.n0;
   const X* src = x + (mu * n0 + ix) * (long)n1 * n2;
-  // pack rows (2r, 2r+1) as re/im; LB loads per thread are issued before the
-  // first LDS store so the plane is fetched in one or two memory round trips
-  constexpr int LB = 8;
-  const int tot = n1p * n2;
+  C2<T>* dst = t + (mu * n0 + ix) * (long)n1 * n2h;
   const FDiv fn2(n2), fn2h(n2h);
-  for (int e0 = threadIdx.x; e0 < tot; e0 += LB * blockDim.x) {
-    X re[LB], im[LB];
-#pragma unroll
-    for (int b = 0; b < LB; ++b) {
-      const int e = e0 + b * (int)blockDim.x;
-      const int r = fn2.div(e), z = e - r * n2;
-      const bool ok = e < tot, ok1 = ok && 2 * r + 1 < n1;
-      re[b] = src[ok ? (long)(2 * r) * n2 + z : 0];
-      im[b] = ok1 ? src[(long)(2 * r + 1) * n2 + z] : X(0);
-    }
-#pragma unroll
-    for (int b = 0; b < LB; ++b) {
-      const int e = e0 + b * (int)blockDim.x;
-      const int r = fn2.div(e), z = e - r * n2;
-      if (e < tot) bufa[swz(r, z, lsz)] = C2<T>{(T)re[b], (T)im[b]};
-    }
-  }
-  __syncthreads();
-  // unpack: A(k) = (Z(k) + conj Z(-k)) / 2, B(k) = (Z(k) - conj Z(-k)) / (2i),
-  // written transposed: y-line kz holds A and B of every row pair
-  C2<T>* fin;
-  if (ip) {
-    if constexpr (CN > 0) fft_lines_ct<T, IPV, CN>(bufa, n1p, lsz, twz);
-    else fft_lines_ip<T, IPV>(bufa, p.pz, n1p, lsz, twz);
-    C2<T> z1[UPV], z2[UPV];
-#pragma unroll
-    for (int i = 0; i < UPV; ++i) {
-      const int e = threadIdx.x + i * FT;
-      if (e < n1p * n2h) {
-        const int r = fn2h.div(e), kz = e - r * n2h;
-        z1[i] = bufa[swz(r, kz, lsz)];
-        z2[i] = bufa[swz(r, kz == 0 ? 0 : n2 - kz, lsz)];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < UPV; ++i) {
-      const int e = threadIdx.x + i * FT;
-      if (e < n1p * n2h) {
-        const int r = fn2h.div(e), kz = e - r * n2h;
-        bufa[swz(kz, 2 * r, lsy)] = C2<T>{(z1[i].x + z2[i].x) * T(0.5), (z1[i].y - z2[i].y) * T(0.5)};
-        if (2 * r + 1 < n1)
-          bufa[swz(kz, 2 * r + 1, lsy)] = C2<T>{(z1[i].y + z2[i].y) * T(0.5), (z2[i].x - z1[i].x) * T(0.5)};
-      }
-    }
-    __syncthreads();
-    if constexpr (CN > 0) fft_lines_ct<T, IPV, CN>(bufa, n2h, lsy, twy);
-    else fft_lines_ip<T, IPV>(bufa, p.py, n2h, lsy, twy);
-    fin = bufa;
+  if constexpr (ip) {
+    __syncthreads();  // twiddles
+    // z: rows (2r, 2r+1) as re/im, read from memory by the first stage
+    fft_lines_io<T, IPV, CN, false, false, true>(
+        bufa, p.pz, n2, n1p, lsz, twz,
+        [&](int r, int z) {
+          return C2<T>{(T)src[2 * r * n2 + z], 2 * r + 1 < n1 ? (T)src[(2 * r + 1) * n2 + z] : T(0)};
+        },
+        [](int, int, int, int, C2<T>) {});
+    // y, with the unpacking A(k) = (Z(k) + conj Z(-k)) / 2 (even rows), B(k) =
+    // (Z(k) - conj Z(-k)) / (2i) (odd rows) in its first stage's reads; the last
+    // stage stores a wave's outputs contiguously
+    fft_lines_io<T, IPV, CN, true, true, false>(
+        bufa, p.py, n1, n2h, lsy, twy,
+        [&](int kz, int y) {
+          const C2<T> z1 = bufa[swz(y >> 1, kz, lsz)], z2 = bufa[swz(y >> 1, kz == 0 ? 0 : n2 - kz, lsz)];
+          return (y & 1) ? C2<T>{(z1.y + z2.y) * T(0.5), (z2.x - z1.x) * T(0.5)}
+                         : C2<T>{(z1.x + z2.x) * T(0.5), (z1.y - z2.y) * T(0.5)};
+        },
+        [&](int, int, int kz, int y, C2<T> v) { dst[y * n2h + kz] = v; });
   } else {
+    // pack rows (2r, 2r+1) as re/im; LB loads per thread are issued before the
+    // first LDS store so the plane is fetched in one or two memory round trips
+    constexpr int LB = 8;
+    const int tot = n1p * n2;
+    for (int e0 = threadIdx.x; e0 < tot; e0 += LB * blockDim.x) {
+      X re[LB], im[LB];
+#pragma unroll
+      for (int b = 0; b < LB; ++b) {
+        const int e = e0 + b * (int)blockDim.x;
+        const int r = fn2.div(e), z = e - r * n2;
+        const bool ok = e < tot, ok1 = ok && 2 * r + 1 < n1;
+        re[b] = src[ok ? (long)(2 * r) * n2 + z : 0];
+        im[b] = ok1 ? src[(long)(2 * r + 1) * n2 + z] : X(0);
+      }
+#pragma unroll
+      for (int b = 0; b < LB; ++b) {
+        const int e = e0 + b * (int)blockDim.x;
+        const int r = fn2.div(e), z = e - r * n2;
+        if (e < tot) bufa[swz(r, z, lsz)] = C2<T>{(T)re[b], (T)im[b]};
+      }
+    }
+    __syncthreads();
+    // unpack, written transposed: y-line kz holds A and B of every row pair
     C2<T>* res = fft_lines<T>(bufa, bufb, p.pz, n1p, lsz, twz);
     C2<T>* h = (res == bufa) ? bufb : bufa;
     for (int e = threadIdx.x; e < n1p * n2h; e += blockDim.x) {
@@ -395,12 +449,11 @@ __global__ __launch_bounds__(FT) void pass_a(const X* __restrict__ x, C2<T>* __r
     }
     __syncthreads();
     C2<T>* other = (h == bufa) ? bufb : bufa;
-    fin = fft_lines<T>(h, other, p.py, n2h, lsy, twy);
-  }
-  C2<T>* dst = t + (mu * n0 + ix) * (long)n1 * n2h;
-  for (int e = threadIdx.x; e < n1 * n2h; e += blockDim.x) {
-    const int y = fn2h.div(e), kz = e - y * n2h;
-    dst[e] = fin[swz(kz, y, lsy)];
+    C2<T>* fin = fft_lines<T>(h, other, p.py, n2h, lsy, twy);
+    for (int e = threadIdx.x; e < n1 * n2h; e += blockDim.x) {
+      const int y = fn2h.div(e), kz = e - y * n2h;
+      dst[e] = fin[swz(kz, y, lsy)];
+    }
   }
 }
 
@@ -421,7 +474,7 @@ __global__ void weight_kernel(const double* __restrict__ coulG, int n1, int n2, 
 // t: (k, n0, n1, n2h) complex -> out (k, n0, n1, n2h, 2) weighted by wt, or
 // (DIG) its int8 digit planes (FftDigits).
 template <class T, int IPV, bool DIG, int CN = 0>  // IPV = 0: ping-pong stages; CN as in pass_a
-__global__ __launch_bounds__(FT) void pass_b(const C2<T>* __restrict__ t, const T* __restrict__ wt,
+__global__ __launch_bounds__(FT, min_waves(sizeof(T), IPV, CN)) void pass_b(const C2<T>* __restrict__ t, const T* __restrict__ wt,
                                              T* __restrict__ out, FftParams p) {
   constexpr bool ip = IPV > 0;
   static_assert(CN == 0 || ip, "compile-time sizes use the in-place stages");
@@ -435,33 +488,43 @@ __global__ __launch_bounds__(FT) void pass_b(const C2<T>* __restrict__ t, const 
   const long mu = blockIdx.y;
   const int iy = blockIdx.x;
   const C2<T>* src = t + mu * (long)n0 * n1 * n2h;
-  // loads in flight per thread: 8 for run-time sizes; the compile-time sizes
-  // unroll the loads of every batch into registers, and 3 keeps those kernels
-  // at about 50 VGPRs, eight waves per SIMD (64^3 FP32 with digits: 1.64 ->
-  // 1.34 ms against 8 at 112 VGPRs)
-  constexpr int LB = CN > 0 ? 3 : 8;
   const int tot = n0 * n2h;
   const FDiv fn2h(n2h);
-  for (int e0 = threadIdx.x; e0 < tot; e0 += LB * blockDim.x) {
-    C2<T> v[LB];
+  C2<T>* fin = nullptr;
+  // x-lines kz.  In-place budget: the first stage reads memory, the last one's
+  // outputs go to 'sink'
+  if constexpr (!ip) {
+    constexpr int LB = 8;
+    for (int e0 = threadIdx.x; e0 < tot; e0 += LB * blockDim.x) {
+      C2<T> v[LB];
 #pragma unroll
-    for (int b = 0; b < LB; ++b) {
-      const int e = e0 + b * (int)blockDim.x;
-      const int ix = fn2h.div(e), kz = e - ix * n2h;
-      v[b] = src[e < tot ? ((long)ix * n1 + iy) * n2h + kz : 0];
-    }
+      for (int b = 0; b < LB; ++b) {
+        const int e = e0 + b * (int)blockDim.x;
+        const int ix = fn2h.div(e), kz = e - ix * n2h;
+        v[b] = src[e < tot ? ((long)ix * n1 + iy) * n2h + kz : 0];
+      }
 #pragma unroll
-    for (int b = 0; b < LB; ++b) {
-      const int e = e0 + b * (int)blockDim.x;
-      const int ix = fn2h.div(e), kz = e - ix * n2h;
-      if (e < tot) bufa[swz(kz, ix, lsx)] = v[b];  // x-line kz
+      for (int b = 0; b < LB; ++b) {
+        const int e = e0 + b * (int)blockDim.x;
+        const int ix = fn2h.div(e), kz = e - ix * n2h;
+        if (e < tot) bufa[swz(kz, ix, lsx)] = v[b];
+      }
     }
+    __syncthreads();
+    fin = fft_lines<T>(bufa, bufb, p.px, n2h, lsx, twx);
   }
-  __syncthreads();
-  C2<T>* fin = bufa;
-  if constexpr (CN > 0) fft_lines_ct<T, IPV, CN>(bufa, n2h, lsx, twx);
-  else if (ip) fft_lines_ip<T, IPV>(bufa, p.px, n2h, lsx, twx);
-  else fin = fft_lines<T>(bufa, bufb, p.px, n2h, lsx, twx);
+  auto transform = [&](auto sink) {
+    if constexpr (ip) {
+      __syncthreads();  // twiddles
+      fft_lines_io<T, IPV, CN, true, false, false>(
+          bufa, p.px, n0, n2h, lsx, twx, [&](int kz, int ix) { return src[((long)ix * n1 + iy) * n2h + kz]; }, sink);
+    } else {
+      for (int e = threadIdx.x; e < tot; e += blockDim.x) {
+        const int kx = fn2h.div(e), kz = e - kx * n2h;
+        sink(0, 0, kz, kx, fin[swz(kz, kx, lsx)]);
+      }
+    }
+  };
   if constexpr (DIG) {
     // the line's weighted values a = v.x f, b = v.y f (rounded to T as the
     // stored spectrum would be); exponent: max |value| < 2^ex; then each value
@@ -471,18 +534,16 @@ __global__ __launch_bounds__(FT) void pass_b(const C2<T>* __restrict__ t, const 
     // can lose bits, where every digit is 0 anyway (|x| 128^5 < 1).
     __shared__ double red[FT / 64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    // (the weighted values go back into the thread's own LDS slots for the
-    // digit pass)
+    // (the weighted values go back into LDS, in the place that their own thread
+    // reads last or that nothing reads again, for the digit pass)
     double mx = 0.0;
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-      const int kx = fn2h.div(e), kz = e - kx * n2h;
+    C2<T>* keep = ip ? bufa : fin;
+    transform([&](int, int, int kz, int kx, C2<T> v) {
       const T f = wt[((long)kx * n1 + iy) * n2h + kz];
-      C2<T>& slot = fin[swz(kz, kx, lsx)];
-      const C2<T> v = slot;
       const T a = v.x * f, b = v.y * f;
-      slot = C2<T>{a, b};
+      keep[swz(kz, kx, lsx)] = C2<T>{a, b};
       mx = fmax(mx, fmax(fabs((double)a), fabs((double)b)));
-    }
+    });
     for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
     if (lane == 0) red[wv] = mx;
     __syncthreads();
@@ -492,53 +553,51 @@ __global__ __launch_bounds__(FT) void pass_b(const C2<T>* __restrict__ t, const 
     if (mx > 0.0) frexp(mx, &ex);
     if (threadIdx.x == 0) p.dig_e[mu * n1 + iy] = ex;
     signed char* row = p.dig_s + mu * p.dig_row + (long)iy * p.dig_lp;
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-      const int kx = fn2h.div(e), kz = e - kx * n2h;
-      const C2<T> v = fin[swz(kz, kx, lsx)];
-      T xa = ldexp(v.x, -ex), xb = ldexp(v.y, -ex);
+    // two values a thread: 4-byte stores (an odd last one leaves two zero bytes
+    // of the padding, a multiple of 64)
+    for (int e0 = 2 * threadIdx.x; e0 < tot; e0 += 2 * blockDim.x) {
+      T v[4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int e = e0 + h < tot ? e0 + h : e0;
+        const int kx = fn2h.div(e), kz = e - kx * n2h;
+        const C2<T> c = keep[swz(kz, kx, lsx)];
+        v[2 * h] = ldexp(c.x, -ex);
+        v[2 * h + 1] = ldexp(c.y, -ex);
+      }
+      if (e0 + 1 >= tot) v[2] = v[3] = T(0);
 #pragma unroll
       for (int q = 0; q < OZ_DIGITS; ++q) {
-        xa *= T(128);
-        const T da = trunc(xa);
-        xa -= da;
-        xb *= T(128);
-        const T db = trunc(xb);
-        xb -= db;
-        *reinterpret_cast<unsigned short*>(row + q * p.dig_plane + 2 * e) =
-            (unsigned short)(((unsigned)(int)da & 0xffu) | (((unsigned)(int)db & 0xffu) << 8));
+        unsigned w = 0;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          v[h] *= T(128);
+          const T d = trunc(v[h]);
+          v[h] -= d;
+          w |= ((unsigned)(int)d & 0xffu) << (8 * h);
+        }
+        *reinterpret_cast<unsigned*>(row + q * p.dig_plane + 2 * e0) = w;
       }
     }
-    for (int c = 2 * tot + threadIdx.x; c < p.dig_lp; c += blockDim.x)
+    for (int c = 4 * ((tot + 1) / 2) + threadIdx.x; c < p.dig_lp; c += blockDim.x)
 #pragma unroll
       for (int q = 0; q < OZ_DIGITS; ++q) row[q * p.dig_plane + c] = 0;
     return;
   }
-  typedef T v2 __attribute__((ext_vector_type(2)));
   T* dst = out + mu * (long)n0 * n1 * n2h * 2;
-  for (int e = threadIdx.x; e < n0 * n2h; e += blockDim.x) {
-    const int kx = fn2h.div(e), kz = e - kx * n2h;
+  transform([&](int, int, int kz, int kx, C2<T> v) {
     const long h = ((long)kx * n1 + iy) * n2h + kz;
     const T f = wt[h];
-    const C2<T> v = fin[swz(kz, kx, lsx)];
-    if (p.vec_out) {
-      *reinterpret_cast<v2*>(dst + 2 * h) = v2{v.x * f, v.y * f};
-    } else {
-      dst[2 * h] = v.x * f;
-      dst[2 * h + 1] = v.y * f;
-    }
-  }
+    // One store of element alignment.  No branch here: outputs of one butterfly
+    // in different blocks would have their sums of products contracted
+    // differently (other last bits than where they go to LDS).
+    *reinterpret_cast<C2<T>*>(dst + 2 * h) = C2<T>{v.x * f, v.y * f};
+  });
 }
 
 bool make_plan(int n, Plan1D& pl) {
-  pl.n = n;
-  pl.nst = 0;
-  int m = n;
-  while (m % 8 == 0 && pl.nst < MAXR) { pl.rad[pl.nst++] = 8; m /= 8; }
-  while (m % 4 == 0 && pl.nst < MAXR) { pl.rad[pl.nst++] = 4; m /= 4; }
-  while (m % 2 == 0 && pl.nst < MAXR) { pl.rad[pl.nst++] = 2; m /= 2; }
-  while (m % 3 == 0 && pl.nst < MAXR) { pl.rad[pl.nst++] = 3; m /= 3; }
-  while (m % 5 == 0 && pl.nst < MAXR) { pl.rad[pl.nst++] = 5; m /= 5; }
-  return m == 1;
+  pl = plan_of(n);
+  return pl.n == n;
 }
 
 // e^{-2 pi i j / n}, j < n, from sincospi (about 1 ulp in double).
@@ -628,15 +687,18 @@ int run(const X* x, int k, const int n[3], const double* coulG, void* out, void*
     p.dig_row = dig->g2p;
     p.dig_plane = (long)k * dig->g2p;
     p.dig_lp = dig->lp;
-    if (dig->lp < 2L * n[0] * (n[2] / 2 + 1) || dig->lp % 2 || dig->g2p != (long)n[1] * dig->lp) return THC_ERR_ARG;
+    if (dig->lp < 2L * n[0] * (n[2] / 2 + 1) || dig->lp % 4 || (dig->lp < 4 * ((n[0] * (n[2] / 2 + 1) + 1) / 2)) || dig->g2p != (long)n[1] * dig->lp) return THC_ERR_ARG;
   }
   p.k = k; p.n0 = n[0]; p.n1 = n[1]; p.n2 = n[2]; p.n2h = n[2] / 2 + 1;
   p.lsz = line_stride(n[2]); p.lsy = line_stride(n[1]); p.lsx = line_stride(n[0]);
   if (!make_plan(n[2], p.pz) || !make_plan(n[1], p.py) || !make_plan(n[0], p.px)) return THC_ERR_UNSUPPORTED;
-  // in-place stages (one LDS buffer) when every stage and the unpack keep to
-  // their per-thread register budgets
+  // in-place stages (one LDS buffer) when every stage keeps to its per-thread
+  // register budget.  The run-time plans have kernels of 8 and 12 values too: the
+  // registers of the radix the budget is largest for are taken whatever the
+  // grid (FP64 95, 128 and 179 VGPRs for 8, 12 and 16; 50^3, 480 vectors: 0.66 ms
+  // with 12, 1.03 with 16)
   const int n1p = (n[1] + 1) / 2, n2h = n[2] / 2 + 1;
-  auto fa = [&](int v) { return fits_ip(p.pz, n1p, v) && fits_ip(p.py, n2h, v) && ((long)n1p * n2h + FT - 1) / FT <= UPV; };
+  auto fa = [&](int v) { return fits_ip(p.pz, n1p, v) && fits_ip(p.py, n2h, v); };
   const int ipa = fa(16) ? 16 : (fa(24) ? 24 : 0);
   const int ipb = fits_ip(p.px, n2h, 16) ? 16 : (fits_ip(p.px, n2h, 24) ? 24 : 0);
   const size_t la = lds_a<T>(n[1], n[2], ipa > 0), lb = lds_b<T>(n[0], n[2], ipb > 0);
@@ -658,20 +720,23 @@ int run(const X* x, int k, const int n[3], const double* coulG, void* out, void*
   THC_HIP(hipGetLastError());
   p.twz = dz; p.twy = dy; p.twx = dx;
   T* o = reinterpret_cast<T*>(out);
-  p.vec_out = (reinterpret_cast<uintptr_t>(out) % (2 * sizeof(T))) == 0;
   if (pass_ev) THC_HIP(hipEventRecord(pass_ev[0], s));
   const int cube = (n[0] == n[1] && n[1] == n[2]) ? n[0] : 0;
   const dim3 ga(n[0], k), gb(n[1], k);
   int st = THC_OK;
   if (!launch_a_ct<T, X>((CtEdges*)nullptr, ipa, cube, ga, la, x, tmid, p, s, st)) {
-    if (ipa == 16) st = launch_a<T, 16, X>(ga, la, x, tmid, p, s);
+    if (fa(8)) st = launch_a<T, 8, X>(ga, la, x, tmid, p, s);
+    else if (fa(12)) st = launch_a<T, 12, X>(ga, la, x, tmid, p, s);
+    else if (ipa == 16) st = launch_a<T, 16, X>(ga, la, x, tmid, p, s);
     else if (ipa == 24) st = launch_a<T, 24, X>(ga, la, x, tmid, p, s);
     else st = launch_a<T, 0, X>(ga, la, x, tmid, p, s);
   }
   THC_TRY(st);
   if (pass_ev) THC_HIP(hipEventRecord(pass_ev[1], s));
   if (!launch_b_ct<T>((CtEdges*)nullptr, ipb, cube, gb, lb, tmid, wt, o, p, s, st)) {
-    if (ipb == 16) st = launch_b<T, 16>(gb, lb, tmid, wt, o, p, s);
+    if (fits_ip(p.px, n2h, 8)) st = launch_b<T, 8>(gb, lb, tmid, wt, o, p, s);
+    else if (fits_ip(p.px, n2h, 12)) st = launch_b<T, 12>(gb, lb, tmid, wt, o, p, s);
+    else if (ipb == 16) st = launch_b<T, 16>(gb, lb, tmid, wt, o, p, s);
     else if (ipb == 24) st = launch_b<T, 24>(gb, lb, tmid, wt, o, p, s);
     else st = launch_b<T, 0>(gb, lb, tmid, wt, o, p, s);
   }
