@@ -950,16 +950,19 @@ int gemm_set_tuning(const int* entries, int n) {
 int gemm_f64(const GemmArgs& g, hipStream_t s) { return gemm_dispatch<double>(g, s); }
 int gemm_f32(const GemmArgs& g, hipStream_t s) { return gemm_dispatch<float>(g, s); }
 
-static void syrk_plan(long m, long k, long& ntiles, int& nsplit, long& kchunk) {
+static void syrk_plan(long m, long k, int prec, long& ntiles, int& nsplit, long& kchunk) {
   const long nb = (m + SY_BM - 1) / SY_BM;
   ntiles = nb * (nb + 1) / 2;
   // Splits: the count up to 2048 workgroups that fills the last round of the 512
   // resident ones best (57 splits of the 36 tiles at m = 1024 left four
   // workgroups to a fifth round), with 1024 or more k per split where 512
   // workgroups allow it: each one writes a 128 KB partial.
-  long want = 1;
+  // FP32 keeps 2048 workgroups: a split is an FP32 sum, the splits are added in
+  // FP64, and four times longer splits cost accuracy (V of a 48^3 cell 1.1e-7 ->
+  // 1.4e-7 of the 64-bit result).
+  long want = prec == 0 ? 1 : (2048 + ntiles - 1) / ntiles;
   double best = 0.0;
-  for (long w = 1; w * ntiles <= 2048; ++w) {
+  for (long w = 1; prec == 0 && w * ntiles <= 2048; ++w) {
     if (w * ntiles > 512 && k / w < 1024) break;
     const long rounds = (w * ntiles + 511) / 512;
     const double fill = (double)(w * ntiles) / (512.0 * rounds);
@@ -976,7 +979,7 @@ static void syrk_plan(long m, long k, long& ntiles, int& nsplit, long& kchunk) {
 size_t syrk_work_bytes(long m, long k, int prec) {
   long ntiles, kchunk;
   int nsplit;
-  syrk_plan(m, k, ntiles, nsplit, kchunk);
+  syrk_plan(m, k, prec, ntiles, nsplit, kchunk);
   return (size_t)nsplit * ntiles * SY_BM * SY_BN * (prec == 0 ? 8 : 4);
 }
 
@@ -985,7 +988,7 @@ int syrk_splitk(const void* a, long m, long k, long lda, int prec, double* v, lo
   if (m <= 0) return THC_OK;
   long ntiles, kchunk;
   int nsplit;
-  syrk_plan(m, k, ntiles, nsplit, kchunk);
+  syrk_plan(m, k, prec, ntiles, nsplit, kchunk);
   KArgs p = {};
   p.m = m; p.n = m; p.k = k;
   p.a = a; p.lda = lda; p.a_rows = nullptr;
