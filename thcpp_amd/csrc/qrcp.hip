@@ -651,10 +651,11 @@ __global__ __launch_bounds__(64 * QW) void qr_apply(const double* __restrict__ p
   }
 }
 
-// ---- one pivot a step, for complex half-rotated orbitals -----------------------
+// ---- one pivot a step: complex half-rotated orbitals, and few pivots of few points
 // Pivot step j; partial maxima are read from (pv_in, pi_in) and written to
-// (pv_out, pi_out), which the host alternates between steps.  G and L are
-// complex: L[2q] holds the real, L[2q + 1] the imaginary parts of column q.
+// (pv_out, pi_out), which the host alternates between steps.  CPLX: G and L are
+// complex, L[2q] holds the real, L[2q + 1] the imaginary parts of column q.
+template <bool CPLX>
 __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, const double* __restrict__ occ, long n,
                                               int m, int mo, int j, int nparts, double* __restrict__ d,
                                               double* __restrict__ L, const double* pv_in, const int* pi_in,
@@ -701,31 +702,47 @@ __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, co
   }
   double* prow = sh;
   double* orow = sh + m;
-  double* lp = orow + mo;
+  double* lp = orow + (occ ? mo : 0);
+  constexpr int LW = CPLX ? 2 : 1;  // doubles per entry of L
   for (int q = threadIdx.x; q < m; q += QB) prow[q] = phi[p * m + q];
-  for (int q = threadIdx.x; q < mo; q += QB) orow[q] = occ[p * mo + q];
-  for (int q = threadIdx.x; q < 2 * j; q += QB) lp[q] = L[(long)q * n + p];
+  if (occ)
+    for (int q = threadIdx.x; q < mo; q += QB) orow[q] = occ[p * mo + q];
+  for (int q = threadIdx.x; q < LW * j; q += QB) lp[q] = L[(long)q * n + p];
   __syncthreads();
   const double rs = 1.0 / sqrt(pval);
   const long a = (long)blockIdx.x * QB + threadIdx.x;
   double v = -DBL_MAX;
   int vi = INT_MAX;
   if (a < n) {
-    double da = d[a];
-    double qr, qi, o_r, o_i;
-    cdot_row(phi + a * m, prow, m, qr, qi);
-    cdot_row(occ + a * mo, orow, mo, o_r, o_i);
-    const double gr = o_r * qr + o_i * qi, gi = o_r * qi - o_i * qr;  // conj(Qocc) Q
-    double ar = 0.0, ai = 0.0;
-    for (int q = 0; q < j; ++q) {
-      const double xr = L[(long)(2 * q) * n + a], xi = L[(long)(2 * q + 1) * n + a];
-      const double yr = lp[2 * q], yi = lp[2 * q + 1];
-      ar = fma(xr, yr, fma(xi, yi, ar));
-      ai = fma(xi, yr, fma(-xr, yi, ai));
+    double da = d[a], lr, li = 0.0;
+    if constexpr (CPLX) {
+      double qr, qi, o_r, o_i;
+      cdot_row(phi + a * m, prow, m, qr, qi);
+      cdot_row(occ + a * mo, orow, mo, o_r, o_i);
+      const double gr = o_r * qr + o_i * qi, gi = o_r * qi - o_i * qr;  // conj(Qocc) Q
+      double ar = 0.0, ai = 0.0;
+      for (int q = 0; q < j; ++q) {
+        const double xr = L[(long)(2 * q) * n + a], xi = L[(long)(2 * q + 1) * n + a];
+        const double yr = lp[2 * q], yi = lp[2 * q + 1];
+        ar = fma(xr, yr, fma(xi, yi, ar));
+        ai = fma(xi, yr, fma(-xr, yi, ai));
+      }
+      lr = (gr - ar) * rs;
+      li = (gi - ai) * rs;
+      L[(long)(2 * j) * n + a] = lr;
+      L[(long)(2 * j + 1) * n + a] = li;
+    } else {
+      const double g = dot_row(phi + a * m, prow, m), h = occ ? dot_row(occ + a * mo, orow, mo) : g;
+      double s0 = 0.0, s1 = 0.0;
+      int q = 0;
+      for (; q + 2 <= j; q += 2) {
+        s0 = fma(L[(long)q * n + a], lp[q], s0);
+        s1 = fma(L[(long)(q + 1) * n + a], lp[q + 1], s1);
+      }
+      if (q < j) s0 = fma(L[(long)q * n + a], lp[q], s0);
+      lr = (g * h - (s0 + s1)) * rs;
+      L[(long)j * n + a] = lr;
     }
-    const double lr = (gr - ar) * rs, li = (gi - ai) * rs;
-    L[(long)(2 * j) * n + a] = lr;
-    L[(long)(2 * j + 1) * n + a] = li;
     if (a == p || da == RETIRED) da = RETIRED;
     else da -= lr * lr + li * li;
     d[a] = da;
@@ -812,13 +829,18 @@ int qrcp_points(const double* phi, const double* occ, long n, int m, int mo, int
   hipLaunchKernelGGL(qr_init, dim3((unsigned)nparts), dim3(QB), 0, s, phi, occ, n, m, mo, d, pv[0], pi[0]);
   THC_HIP(hipGetLastError());
   int h_fail = 0;
-  if (mode == 2) {
+  // Few pivots of few real points: a step is 8 us there and a round of shared
+  // pivots 75, of which six or seven are taken whatever k (27^3 points, k = 54:
+  // 0.44 ms in steps, 0.47 in rounds; 32^3 points, k = 50: 0.44 and 0.53; but
+  // 32^3 points, k = 67: 0.58 and 0.41; 48^3 points, k = 40: 0.67 and 0.33).
+  if (mode == 2 || (mode == 0 && k < 64 && n <= 40000)) {
+    const auto step = mode == 2 ? qr_step<true> : qr_step<false>;
     if (lds > 64 * 1024)
-      THC_HIP(hipFuncSetAttribute((const void*)qr_step, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      THC_HIP(hipFuncSetAttribute((const void*)step, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     THC_HIP(hipMemsetAsync(fail, 0, sizeof(int), s));
     for (int j = 0; j < k; ++j) {
       const int in = j & 1;
-      hipLaunchKernelGGL(qr_step, dim3((unsigned)nparts), dim3(QB), lds, s, phi, occ, n, m, mo, j, (int)nparts, d, L,
+      hipLaunchKernelGGL(step, dim3((unsigned)nparts), dim3(QB), lds, s, phi, occ, n, m, mo, j, (int)nparts, d, L,
                          pv[in], pi[in], pv[in ^ 1], pi[in ^ 1], piv, rd, fail);
     }
     THC_HIP(hipGetLastError());
