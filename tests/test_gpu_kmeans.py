@@ -283,3 +283,25 @@ def test_kmeans_empty_cluster_later(ctx, n, k, seed):
         assert out["status"] == L.THC_ERR_EMPTY_CLUSTER
         assert out["iters"] == 2
         assert out["diffs"][0] == ref["diffs"][0]
+
+
+@pytest.mark.parametrize("n,k", [(4000, 1), (9000, 300), (30000, 1500)])
+@pytest.mark.parametrize("stop", [0, 1, 2, 5])
+def test_kmeans_stops_beside_next_iteration(ctx, n, k, stop):
+    """A threshold that stops the loop while the next iteration is on its way: the points, map, centroids and
+    differences are those of the iteration that it stopped at."""
+    rng = np.random.default_rng(k + stop)
+    grid = rng.uniform(0, 9, size=(n, 3))
+    rho = rng.uniform(0.1, 2.0, size=n)
+    run = KO.kmeans(grid, rho, k, 6, -1.0, 7)["diffs"]
+    thr = float(np.nextafter(run[: stop + 1].min(), np.inf))
+    ref = KO.kmeans(grid, rho, k, 20, thr, 7, keep_maps=True)
+    assert ref["status"] in (0, 2) and ref["iters"] <= stop + 1  # 2: two centroids on one point
+    out = ctx.kmeans(grid, rho, k, 20, thr, 7, want_map=True, want_centroids=True)
+    assert out["status"] == (L.THC_WARN_DUPLICATE_INDICES if ref["status"] else L.THC_OK) and out["converged"]
+    assert out["iters"] == ref["iters"]
+    np.testing.assert_array_equal(out["interp_idx"].cpu().numpy(), ref["interp_idx"])
+    np.testing.assert_array_equal(out["diffs"], ref["diffs"])
+    np.testing.assert_array_equal(out["pcts"], ref["pcts"])
+    np.testing.assert_array_equal(out["grid_map"].cpu().numpy(), ref["maps"][-1])
+    np.testing.assert_array_equal(out["centroids"].cpu().numpy(), ref["centroids"])

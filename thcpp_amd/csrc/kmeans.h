@@ -16,7 +16,7 @@ enum { MODE_LATEST = 0, MODE_FINAL = 1, MODE_ZEROS = 2 };
 
 // Device-side loop state (one per run).
 struct State {
-  int done;        // loop ended: diff < threshold, or an error
+  int ended;       // iteration the loop ended at (diff < threshold, or an error), INT_MAX before
   int final_buf;   // centroid buffer with the converged centroids (MODE_FINAL)
   int error;       // 1: a cluster weight < 1e-8 in an iteration the loop ran; 2: bad cluster key
   int bad;         // first iteration with a cluster weight < 1e-8 (later ones do nothing), else INT_MAX

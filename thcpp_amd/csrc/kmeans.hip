@@ -247,7 +247,7 @@ __device__ __forceinline__ void init_run_b(const double* grid, const int* idx, i
   const int j = bid * 256 + threadIdx.x;
   for (int i = j; i < nchg; i += nblk * 256) chg[i] = 0;
   if (j == 0) {
-    st->done = 0;
+    st->ended = INT_MAX;
     st->final_buf = 0;
     st->error = 0;
     st->bad = INT_MAX;
@@ -445,8 +445,8 @@ __device__ __forceinline__ void assign_b(const double* sx, const double* sy, con
                                               const int* perm, long n, const double* boxes, const double* wboxes,
                                               const double* cen, int k, int* map_new, const int* map_old,
                                               int* cnt, int* bucket, int cap, int* chg, const State* st, int it,
-                                              int bid) {
-  if (st && (st->done || st->bad < it)) return;
+                                              int seen, int bid) {
+  if (st && (st->ended <= seen || st->bad < it)) return;
   __shared__ int cidx[256 * CPT];
   __shared__ double ccx[CAND_CAP], ccy[CAND_CAP], ccz[CAND_CAP];
   __shared__ int lcnt[CAND_CAP], lbase[CAND_CAP];
@@ -618,8 +618,9 @@ template <int CPT>
 __global__ __launch_bounds__(256) void assign(const double* sx, const double* sy, const double* sz,
                                               const int* perm, long n, const double* boxes, const double* wboxes,
                                               const double* cen, int k, int* map_new, const int* map_old, int* cnt,
-                                              int* bucket, int cap, int* chg, const State* st, int it) {
-  assign_b<CPT>(sx, sy, sz, perm, n, boxes, wboxes, cen, k, map_new, map_old, cnt, bucket, cap, chg, st, it,
+                                              int* bucket, int cap, int* chg, const State* st, int it,
+                                              int seen) {
+  assign_b<CPT>(sx, sy, sz, perm, n, boxes, wboxes, cen, k, map_new, map_old, cnt, bucket, cap, chg, st, it, seen,
                 (int)blockIdx.x);
 }
 
@@ -680,7 +681,7 @@ __device__ inline void sums_rank(SumsLds& S, int wb, int we, int& pos, int& tota
 
 __device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int cap, const int* map, const int* perm,
                                                      long n, const double* rho, const double* grid, double* cen_out,
-                                                     State* st, int it, int c) {
+                                                     State* st, int it, int seen, int c) {
   __shared__ SumsLds S;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int* mem = bucket + (long)c * cap;
@@ -688,7 +689,7 @@ __device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int
 #pragma unroll
   for (int u = 0; u < SB_R; ++u) i[u] = tid + 256 * u < cap ? mem[tid + 256 * u] : 0;  // before the count is known
   const int m = cnt[c];
-  if (st->done || st->bad < it) return;
+  if (st->ended <= seen || st->bad < it) return;
   const bool listed = m <= cap;
   int lo = INT_MAX, hi = INT_MAX;  // hi negated: both are minima
   double v[SB_R][4];
@@ -798,8 +799,8 @@ __device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int
 }
 __global__ __launch_bounds__(256) void centroid_sums(int* cnt, const int* bucket, int cap, const int* map,
                                                      const int* perm, long n, const double* rho, const double* grid,
-                                                     double* cen_out, State* st, int it) {
-  centroid_sums_b(cnt, bucket, cap, map, perm, n, rho, grid, cen_out, st, it, (int)blockIdx.x);
+                                                     double* cen_out, State* st, int it, int seen) {
+  centroid_sums_b(cnt, bucket, cap, map, perm, n, rho, grid, cen_out, st, it, seen, (int)blockIdx.x);
 }
 
 // normed_difference(new, cur) with the reference's sequential sum, % changed,
@@ -810,7 +811,7 @@ __device__ __forceinline__ void diff_control_b(const double* nxt, const double* 
                                                      double threshold, int it, int max_it, int nxt_buf,
                                                      State* st, int* chg, double* diffs, double* pcts,
                                                      bool defer) {
-  if (!defer && st->done) return;
+  if (!defer && st->ended < it) return;
   extern __shared__ __attribute__((aligned(16))) double terms[];
   __shared__ double red[4][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -820,7 +821,7 @@ __device__ __forceinline__ void diff_control_b(const double* nxt, const double* 
     if (bad == it && tid == 0) {
       st->error = 1;
       st->iters = it + 1;
-      if (!defer) st->done = 1;
+      if (!defer) st->ended = it;
     }
     return;
   }
@@ -854,7 +855,7 @@ __device__ __forceinline__ void diff_control_b(const double* nxt, const double* 
     if (!defer || it == max_it - 1) st->iters = it + 1;
     if (!defer || it == max_it - 1 || bad == it + 1) st->last_diff = diff;
     if (diff < threshold) {
-      st->done = 1;
+      st->ended = it;
       st->mode = MODE_FINAL;
       st->final_buf = nxt_buf;
     } else if (it == max_it - 1) {
@@ -1152,7 +1153,10 @@ __host__ __device__ inline long chg_at(const Layout& L, int it) { return (long)(
 // the stop test) runs on the second stream beside iteration it + 1, which does
 // not need its result: if iteration it stops the loop, iteration it + 1
 // (already started) only writes buffers the final state does not use, and
-// iteration it + 2 waits for it and returns at once.  Hence three centroid
+// iteration it + 2 waits for it and returns at once.  Iteration it + 1 runs to
+// its end even if the stop comes while it runs: its workgroups go only by
+// controls that had ended before they started ('seen'), so the waves of one
+// never part at a flag that changes under them.  Hence three centroid
 // buffers (iteration it reads it % 3, writes (it+1) % 3, and diff_control(it)
 // still reads both while iteration it + 1 writes (it+2) % 3).  With sa == s
 // the same code runs in order on one stream.
@@ -1167,16 +1171,17 @@ static int enqueue_kmeans(const Layout& L, const Bufs& b, const double* grid, co
   const size_t dyn = (size_t)3 * L.k * sizeof(double);
   for (int it = 0; it < L.max_it; ++it) {
     const int cur = cen_buf(L, it), nxt = cen_buf(L, it + 1), par = it & 1;
+    const int seen = it - (two ? 2 : 1);  // the latest loop control this iteration starts after
     int* mnew = b.map[par];
     const int* mold = it == 0 ? nullptr : b.map[par ^ 1];
     if (!L.defer && two && it >= 2) THC_HIP(hipStreamWaitEvent(s, kev[1 + par], 0));  // diff_control(it - 2)
     with_cpt(L.k, [&](auto cpt) {
       hipLaunchKernelGGL(assign<cpt.value>, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes,
                          b.wboxes, b.cen + cur * cs, L.k, mnew, mold, b.cnt, b.bucket, L.cap, b.chg + chg_at(L, it),
-                         b.st, it);
+                         b.st, it, seen);
     });
     hipLaunchKernelGGL(centroid_sums, dim3(L.k), dim3(256), 0, s, b.cnt, b.bucket, L.cap, mnew, b.perm, L.n, rho, grid,
-                       b.cen + nxt * cs, b.st, it);
+                       b.cen + nxt * cs, b.st, it, seen);
     if (L.defer) continue;
     if (two) {
       THC_HIP(hipEventRecord(kev[0], s));
@@ -1312,7 +1317,7 @@ __global__ __launch_bounds__(256) void assign_m(const Job* jobs, const int* off,
   const int par = it & 1;
   assign_b<CPT>(q.b.sx, q.b.sy, q.b.sz, q.b.perm, q.L.n, q.b.boxes, q.b.wboxes, job_cen(q, it), q.L.k, q.b.map[par],
            it == 0 ? nullptr : q.b.map[par ^ 1], q.b.cnt, q.b.bucket, q.L.cap, q.b.chg + chg_at(q.L, it), q.b.st, it,
-           bid);
+           it - 1, bid);
 }
 
 __global__ __launch_bounds__(256) void centroid_sums_m(const Job* jobs, const int* off, int nj, int it) {
@@ -1320,7 +1325,7 @@ __global__ __launch_bounds__(256) void centroid_sums_m(const Job* jobs, const in
   (void)nblk;
   if (it >= q.L.max_it) return;
   centroid_sums_b(q.b.cnt, q.b.bucket, q.L.cap, q.b.map[it & 1], q.b.perm, q.L.n, q.rho, q.grid, job_cen(q, it + 1),
-                  q.b.st, it, bid);
+                  q.b.st, it, it - 1, bid);
 }
 
 // loop control of iteration it0 + blockIdx.y
@@ -1627,7 +1632,7 @@ int kmeans_classify(thc_ctx* ctx, const double* grid, long n, const double* cent
   with_cpt(k, [&](auto cpt) {
     hipLaunchKernelGGL(assign<cpt.value>, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes,
                        b.wboxes, centroids, k, grid_map, (const int*)nullptr, (int*)nullptr, (int*)nullptr, 0,
-                       (int*)nullptr, (const State*)nullptr, 0);
+                       (int*)nullptr, (const State*)nullptr, 0, -1);
   });
   THC_HIP(hipGetLastError());
   THC_HIP(hipStreamSynchronize(s));
@@ -1653,7 +1658,7 @@ int kmeans_update(thc_ctx* ctx, const double* rho, const double* grid, long n, c
   hipLaunchKernelGGL(check_keys, dim3(256), dim3(256), 0, s, grid_map, n, k, st);
   hipLaunchKernelGGL(bucket_map, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, grid_map, n, k, cnt, bucket, cap);
   hipLaunchKernelGGL(centroid_sums, dim3(k), dim3(256), 0, s, cnt, bucket, cap, grid_map, (const int*)nullptr, n, rho,
-                     grid, centroids, st, 0);
+                     grid, centroids, st, 0, -1);
   THC_HIP(hipGetLastError());
   State hst;
   THC_HIP(hipMemcpyAsync(&hst, st, sizeof(State), hipMemcpyDeviceToHost, s));
