@@ -135,3 +135,27 @@ def test_batched_kmeans_uneven_loops(ctx, batch):
         assert o["iters"] == (1 if d["threshold"] > 0 else d["max_it"])
         assert torch.equal(o["interp_idx"], one["interp_idx"])
         assert torch.equal(o["V"], one["V"])
+
+
+def test_batched_kmeans_converged_before_empty_cluster(ctx):
+    """Loops that their threshold ends after the first iteration, where the second would have emptied a cluster:
+    the oracle's points, in a batch and one by one."""
+    systems, refs = [], []
+    for n, edges, k, seed in [(40, (5, 4, 2), 12, 132), (40, (5, 4, 2), 12, 1857), (60, (5, 4, 3), 25, 1710)]:
+        rng = np.random.default_rng(seed)
+        grid = rng.integers(0, 5, size=(n, 3)).astype(float)
+        rho = 10.0 ** rng.uniform(-12, 1, size=n)
+        thr = 2 * KO.kmeans(grid, rho, k, 8, -1.0, seed)["diffs"][0]
+        refs.append(KO.kmeans(grid, rho, k, 8, thr, seed))
+        assert refs[-1]["status"] == 0 and refs[-1]["iters"] == 1
+        systems.append({"grid": grid, "rho": rho, "aoR": rng.standard_normal((n, k)), "fft_grid": edges,
+                        "coulG": synthetic.coulomb_kernel(5.0, edges), "thc_cfac": 1, "max_it": 8, "threshold": thr,
+                        "seed": seed})
+    st, outs = ctx.factorize_batched(systems, precision=L.PREC_FP64, max_streams=2)
+    assert st == L.THC_OK
+    for d, o, ref in zip(systems, outs, refs):
+        one = ctx.factorize(d["grid"], d["rho"], d["aoR"], 1, 8, d["fft_grid"], d["coulG"], threshold=d["threshold"],
+                            seed=d["seed"])
+        for r in (o, one):
+            assert r["iters"] == 1
+            np.testing.assert_array_equal(r["interp_idx"].cpu().numpy(), ref["interp_idx"])

@@ -305,3 +305,41 @@ def test_kmeans_stops_beside_next_iteration(ctx, n, k, stop):
     np.testing.assert_array_equal(out["pcts"], ref["pcts"])
     np.testing.assert_array_equal(out["grid_map"].cpu().numpy(), ref["maps"][-1])
     np.testing.assert_array_equal(out["centroids"].cpu().numpy(), ref["centroids"])
+
+
+@pytest.mark.parametrize("n,k,seed", [(40, 12, 132), (40, 12, 1857), (60, 25, 1710)])
+def test_kmeans_converged_before_empty_cluster(ctx, n, k, seed):
+    """The runs of test_kmeans_empty_cluster_later with a threshold that ends them after the first iteration: the
+    weight that vanishes in the second, which has been started by then, is none of their business."""
+    rng = np.random.default_rng(seed)
+    grid = rng.integers(0, 5, size=(n, 3)).astype(float)
+    rho = 10.0 ** rng.uniform(-12, 1, size=n)
+    thr = 2 * KO.kmeans(grid, rho, k, 8, -1.0, seed)["diffs"][0]
+    _check_converged_first(ctx, grid, rho, k, thr, seed, None)
+
+
+def test_kmeans_converged_before_empty_cluster_many(ctx):
+    """The same with 1200 centroids, whose loop control ends well after the next iteration has started.  On a line
+    away from the rest, the middle one of three centroids has two heavy points and a light one; its neighbours move
+    towards the heavy ones and take them."""
+    rng = np.random.default_rng(12)
+    n, k = 6000, 1200
+    grid = rng.uniform(0, 9, size=(n, 3))
+    rho = rng.uniform(0.1, 2.0, size=n)
+    grid[:7, 1:] = 0.0
+    grid[:7, 0] = [-26.0, -23.5, -22.0, -20.0, -18.0, -16.5, -14.0]
+    rho[:7] = [1e-3, 1.0, 1.0, 1e-12, 1.0, 1.0, 1e-3]
+    init = np.concatenate([[0, 3, 6], np.arange(100, 100 + k - 3)]).astype(np.int32)
+    run = KO.kmeans(grid, rho, k, 8, -1.0, 0, init_idx=init)
+    assert run["status"] == 1 and run["iters"] == 2
+    _check_converged_first(ctx, grid, rho, k, 2 * run["diffs"][0], 0, init)
+
+
+def _check_converged_first(ctx, grid, rho, k, thr, seed, init):
+    ref = KO.kmeans(grid, rho, k, 8, thr, seed, init_idx=init)
+    assert ref["iters"] == 1 and ref["status"] in (0, 2)
+    out = ctx.kmeans(grid, rho, k, 8, thr, seed, init_idx=init, want_centroids=True)
+    assert out["status"] == (L.THC_WARN_DUPLICATE_INDICES if ref["status"] else L.THC_OK)
+    assert out["converged"] and out["iters"] == 1
+    np.testing.assert_array_equal(out["interp_idx"].cpu().numpy(), ref["interp_idx"])
+    np.testing.assert_array_equal(out["centroids"].cpu().numpy(), ref["centroids"])

@@ -19,7 +19,8 @@ struct State {
   int ended;       // iteration the loop ended at (diff < threshold, or an error), INT_MAX before
   int final_buf;   // centroid buffer with the converged centroids (MODE_FINAL)
   int error;       // 1: a cluster weight < 1e-8 in an iteration the loop ran; 2: bad cluster key
-  int bad;         // first iteration with a cluster weight < 1e-8 (later ones do nothing), else INT_MAX
+  int bad;         // first iteration with a cluster weight < 1e-8 (later ones do nothing), else INT_MAX; it may be
+                   // one that the loop had already ended before
   int iters;       // iterations executed
   int mode;        // which centroids map_to_grid uses (MODE_*)
   int dups;        // repeated indices after map_to_grid

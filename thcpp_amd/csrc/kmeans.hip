@@ -880,15 +880,18 @@ __global__ __launch_bounds__(1024) void diff_control_all(const double* cen, int 
 // ------------------------------------------------------------------ map_to_grid
 
 // Nearest grid point per centroid (lexicographic distance/index minimum over
-// the grid tiles the bounds cannot exclude).
+// the grid tiles the bounds cannot exclude).  beside: the loop control runs
+// after the loop, beside this kernel, and a vanished weight is known from the
+// sums alone; else it has ended, and only its verdict counts (the iteration
+// that a converged loop had started may have set 'bad').
 __device__ __forceinline__ void map_to_grid_b(const double* sx, const double* sy, const double* sz,
                                                    const int* perm, long n, const double* boxes, int ntiles,
                                                    const double* cen3, long cstride, int latest_buf,
-                                                   const State* st, int* out, int bid) {
+                                                   const State* st, bool beside, int* out, int bid) {
   const int c = bid;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int mode = st ? st->mode : MODE_LATEST;
-  if (mode == MODE_ZEROS || (st && st->bad != INT_MAX)) {
+  if (mode == MODE_ZEROS || (st && (beside ? st->bad != INT_MAX : st->error != 0))) {
     if (tid == 0) out[c] = 0;
     return;
   }
@@ -941,8 +944,8 @@ __device__ __forceinline__ void map_to_grid_b(const double* sx, const double* sy
 __global__ __launch_bounds__(256) void map_to_grid(const double* sx, const double* sy, const double* sz,
                                                    const int* perm, long n, const double* boxes, int ntiles,
                                                    const double* cen3, long cstride, int latest_buf,
-                                                   const State* st, int* out) {
-  map_to_grid_b(sx, sy, sz, perm, n, boxes, ntiles, cen3, cstride, latest_buf, st, out, (int)blockIdx.x);
+                                                   const State* st, bool beside, int* out) {
+  map_to_grid_b(sx, sy, sz, perm, n, boxes, ntiles, cen3, cstride, latest_buf, st, beside, out, (int)blockIdx.x);
 }
 
 // Sort the k indices ascending (bitonic in LDS) and count adjacent repeats; a
@@ -951,7 +954,7 @@ __device__ __forceinline__ void sort_indices_b(int* idx, int k, State* st) {
   __shared__ int s[MAXB];
   int p2 = 1;
   while (p2 < k) p2 <<= 1;
-  const bool none = st && (st->mode == MODE_ZEROS || st->bad != INT_MAX);
+  const bool none = st && (st->mode == MODE_ZEROS || st->error != 0);
   for (int i = threadIdx.x; i < p2; i += 1024) s[i] = i >= k ? INT_MAX : (none ? 0 : idx[i]);
   __syncthreads();
   for (int size = 2; size <= p2; size <<= 1) {
@@ -1205,7 +1208,7 @@ static int enqueue_kmeans(const Layout& L, const Bufs& b, const double* grid, co
   if (two && !L.defer) THC_HIP(hipStreamWaitEvent(s, kev[last], 0));
   const int latest = cen_buf(L, L.max_it);
   hipLaunchKernelGGL(map_to_grid, dim3(L.k), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes, L.ntiles,
-                     b.cen, cs, latest, b.st, interp_idx);
+                     b.cen, cs, latest, b.st, L.defer != 0, interp_idx);
   if (two && L.defer) THC_HIP(hipStreamWaitEvent(s, kev[last], 0));
   hipLaunchKernelGGL(sort_indices, dim3(1), dim3(1024), 0, s, interp_idx, L.k, b.st);
   if (map_out || cen_out)
@@ -1341,7 +1344,7 @@ __global__ __launch_bounds__(256) void map_to_grid_m(const Job* jobs, const int*
   KM_JOB(off)
   (void)nblk;
   map_to_grid_b(q.b.sx, q.b.sy, q.b.sz, q.b.perm, q.L.n, q.b.boxes, q.L.ntiles, q.b.cen, 3L * q.L.k,
-                cen_buf(q.L, q.L.max_it), q.b.st, q.interp_idx, bid);
+                cen_buf(q.L, q.L.max_it), q.b.st, q.L.defer != 0, q.interp_idx, bid);
 }
 
 __global__ __launch_bounds__(1024) void sort_indices_m(const Job* jobs) {
@@ -1686,7 +1689,7 @@ int kmeans_map_to_grid(thc_ctx* ctx, const double* grid, long n, const double* c
                      (int*)nullptr, (int*)nullptr, 0, b.st);
   enqueue_setup(L, b, grid, s);
   hipLaunchKernelGGL(map_to_grid, dim3(k), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes, L.ntiles,
-                     centroids, 0L, 0, (const State*)nullptr, interp_idx);
+                     centroids, 0L, 0, (const State*)nullptr, false, interp_idx);
   hipLaunchKernelGGL(sort_indices, dim3(1), dim3(1024), 0, s, interp_idx, k, b.st);
   THC_HIP(hipGetLastError());
   State hst;
