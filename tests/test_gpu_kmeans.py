@@ -343,3 +343,21 @@ def _check_converged_first(ctx, grid, rho, k, thr, seed, init):
     assert out["converged"] and out["iters"] == 1
     np.testing.assert_array_equal(out["interp_idx"].cpu().numpy(), ref["interp_idx"])
     np.testing.assert_array_equal(out["centroids"].cpu().numpy(), ref["centroids"])
+
+
+@pytest.mark.parametrize("k", [40, 1500])
+def test_kmeans_difference_not_a_number(ctx, k):
+    """A density that is not a number leaves no difference to compare: after the last iteration the reference maps
+    neither set of centroids and the points stay zero, whether the difference comes in the loop or after it."""
+    rng = np.random.default_rng(k)
+    n = 5000
+    grid = rng.uniform(0, 9, size=(n, 3))
+    rho = rng.uniform(0.1, 2.0, size=n)
+    rho[77] = np.nan
+    for thr in (-1.0, 1e-3):
+        ref = KO.kmeans(grid, rho, k, 1, thr, 1)
+        assert ref["iters"] == 1 and np.isnan(ref["diffs"]).all() and not ref["interp_idx"].any()
+        out = ctx.kmeans(grid, rho, k, 1, thr, 1)
+        assert out["iters"] == 1 and not out["converged"] and out["interp_zeroed"]
+        assert np.isnan(out["diffs"]).all()
+        assert not out["interp_idx"].cpu().numpy().any()

@@ -881,16 +881,18 @@ __global__ __launch_bounds__(1024) void diff_control_all(const double* cen, int 
 
 // Nearest grid point per centroid (lexicographic distance/index minimum over
 // the grid tiles the bounds cannot exclude).  beside: the loop control runs
-// after the loop, beside this kernel, and a vanished weight is known from the
-// sums alone; else it has ended, and only its verdict counts (the iteration
-// that a converged loop had started may have set 'bad').
+// after the loop, beside this kernel: a vanished weight is known from the sums
+// alone, and 'mode', which it may be writing, is not read (all of a workgroup's
+// waves take one way; sort_indices zeroes the points of MODE_ZEROS).  Else it
+// has ended, and only its verdict counts (the iteration that a converged loop
+// had started may have set 'bad').
 __device__ __forceinline__ void map_to_grid_b(const double* sx, const double* sy, const double* sz,
                                                    const int* perm, long n, const double* boxes, int ntiles,
                                                    const double* cen3, long cstride, int latest_buf,
                                                    const State* st, bool beside, int* out, int bid) {
   const int c = bid;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int mode = st ? st->mode : MODE_LATEST;
+  const int mode = st && !beside ? st->mode : MODE_LATEST;
   if (mode == MODE_ZEROS || (st && (beside ? st->bad != INT_MAX : st->error != 0))) {
     if (tid == 0) out[c] = 0;
     return;
