@@ -361,3 +361,57 @@ def test_kmeans_difference_not_a_number(ctx, k):
         assert out["iters"] == 1 and not out["converged"] and out["interp_zeroed"]
         assert np.isnan(out["diffs"]).all()
         assert not out["interp_idx"].cpu().numpy().any()
+
+
+def _windows_map(case):
+    """(n, k, map): cluster sizes and index ranges at the edges of the sums' 65536-point windows and 256-member runs."""
+    rng = np.random.default_rng(3)
+    if case == "dense":  # two windows full of one cluster, then a window of another
+        return 140000, 2, (np.arange(140000) >= 131072).astype(np.int32)
+    if case == "runs":  # 255, 256, 257, 512, 513 members in five windows, an empty window between, ends of windows
+        n = 6 * 65536 + 5
+        gmap = (1 + np.arange(n) % 9).astype(np.int32)
+        for w, m in ((0, 255), (1, 256), (2, 257), (4, 512), (5, 513)):
+            gmap[65536 * w + np.concatenate([[0, 65535], 1 + rng.choice(65534, m - 2, replace=False)])] = 0
+        gmap[3 * 65536:4 * 65536][gmap[3 * 65536:4 * 65536] == 0] = 1
+        return n, 10, gmap
+    if case == "shared":  # six clusters beyond their buckets (8 n / k members) share the list
+        n, k = 150000, 900
+        gmap = rng.integers(0, 6, n).astype(np.int32) * 150
+        gmap[:k] = np.arange(k)
+        return n, k, gmap
+    n = 513 * 65536 + 100  # "far": more windows than one partition takes
+    gmap = np.zeros(n, dtype=np.int32)
+    gmap[rng.integers(0, n, 3000)] = 1
+    gmap[[0, n - 1]] = 2
+    return n, 3, gmap
+
+
+@pytest.mark.parametrize("case", ["dense", "runs", "shared", "far"])
+def test_update_centroids_windows(ctx, case):
+    n, k, gmap = _windows_map(case)
+    rng = np.random.default_rng(n)
+    grid = rng.uniform(0, 7, size=(n, 3))
+    rho = rng.uniform(0.1, 2.0, size=n)
+    got, st = ctx.update_centroids(rho, grid, gmap, k)
+    ref, crit = KO.update_centroids(rho, grid, gmap, k)
+    assert st == L.THC_OK and crit == 0
+    np.testing.assert_array_equal(got.cpu().numpy(), ref)
+
+
+def test_kmeans_vacuum(ctx):
+    """A density that falls off into vacuum: the centroids follow it and the few left outside own far more points
+    than a bucket holds, more of them with every iteration."""
+    rng = np.random.default_rng(4)
+    n, k = 40000, 600
+    grid = rng.uniform(0, 24, size=(n, 3))
+    rho = np.exp(-1.0 * np.linalg.norm(grid - 12.0, axis=1))
+    ref = KO.kmeans(grid, rho, k, 16, -1.0, 2, keep_maps=True)
+    big = [(np.bincount(m, minlength=k) > 8 * -(-n // k)).sum() for m in ref["maps"]]
+    assert ref["status"] == 0 and big[0] == 0 and big[-1] > 3
+    for thr in (-1.0, 1e-300):
+        out = ctx.kmeans(grid, rho, k, 16, thr, 2, want_map=True, want_centroids=True)
+        np.testing.assert_array_equal(out["interp_idx"].cpu().numpy(), ref["interp_idx"])
+        np.testing.assert_array_equal(out["diffs"], ref["diffs"])
+        np.testing.assert_array_equal(out["grid_map"].cpu().numpy(), ref["maps"][-1])
+        np.testing.assert_array_equal(out["centroids"].cpu().numpy(), ref["centroids"])

@@ -241,10 +241,11 @@ __global__ __launch_bounds__(256) void sorted_tiles(const double* grid, const in
 }
 
 // Start of a run: the loop state, the starting centroids, empty buckets and
-// change counts.
-__device__ __forceinline__ void init_run_b(const double* grid, const int* idx, int k, double* cen, int* cnt, int* chg,
-                                                int nchg, State* st, int bid, int nblk) {
+// lists (ctr) and change counts.
+__device__ __forceinline__ void init_run_b(const double* grid, const int* idx, int k, double* cen, int* cnt, int* ctr,
+                                                int* chg, int nchg, State* st, int bid, int nblk) {
   const int j = bid * 256 + threadIdx.x;
+  if (ctr && j < 4) ctr[j] = 0;
   for (int i = j; i < nchg; i += nblk * 256) chg[i] = 0;
   if (j == 0) {
     st->ended = INT_MAX;
@@ -265,8 +266,8 @@ __device__ __forceinline__ void init_run_b(const double* grid, const int* idx, i
   cen[j * 3 + 2] = grid[i * 3 + 2];
 }
 __global__ __launch_bounds__(256) void init_run(const double* grid, const int* idx, int k, double* cen, int* cnt,
-                                                int* chg, int nchg, State* st) {
-  init_run_b(grid, idx, k, cen, cnt, chg, nchg, st, (int)blockIdx.x, (int)gridDim.x);
+                                                int* ctr, int* chg, int nchg, State* st) {
+  init_run_b(grid, idx, k, cen, cnt, ctr, chg, nchg, st, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ------------------------------------------------------------------ stable counting sort (Morton cells)
@@ -432,9 +433,26 @@ __global__ __launch_bounds__(256) void cs_scatter(const int* keys, long n, int n
 // the whole list for every wave it took 38 us.
 //
 // With buckets (cnt, bucket) the points of a cluster are also listed for
-// centroid_sums, cap of them at most, in any order: one device atomic per tile
-// and cluster that has points there.
+// centroid_sums in any order, one device atomic per tile and cluster that has
+// points there: cap of them in its bucket, any more in one list of (cluster,
+// point) for all clusters, over.  ctr: its length and that of centroid_sums'
+// partitions, each for even and odd iterations; an iteration clears those of
+// the next, which the one before it has used up.
 constexpr double SURE = 1.0 + 0x1p-49;
+
+// Point 'orig' as member number 'at' of its cluster, by every lane of a wave.
+__device__ __forceinline__ void list_member(bool live, int cluster, int at, int orig, int* bucket, int cap, int2* over,
+                                            int* nover) {
+  if (live && at < cap) bucket[(long)cluster * cap + at] = orig;
+  const unsigned long long more = __ballot(live && at >= cap);
+  if (more) {
+    const int lane = threadIdx.x & 63, first = __ffsll((long long)more) - 1;
+    int base = 0;
+    if (lane == first) base = atomicAdd(nover, __popcll(more));
+    base = __shfl(base, first);
+    if (live && at >= cap) over[base + __popcll(more & ((1ull << lane) - 1))] = make_int2(cluster, orig);
+  }
+}
 
 //
 // CPT: centroids a thread looks at (k <= 256 CPT); the smallest that holds k
@@ -444,8 +462,8 @@ template <int CPT>
 __device__ __forceinline__ void assign_b(const double* sx, const double* sy, const double* sz,
                                               const int* perm, long n, const double* boxes, const double* wboxes,
                                               const double* cen, int k, int* map_new, const int* map_old,
-                                              int* cnt, int* bucket, int cap, int* chg, const State* st, int it,
-                                              int seen, int bid) {
+                                              int* cnt, int* bucket, int cap, int2* over, int* ctr, int* chg,
+                                              const State* st, int it, int seen, int bid) {
   if (st && (st->ended <= seen || st->bad < it)) return;
   __shared__ int cidx[256 * CPT];
   __shared__ double ccx[CAND_CAP], ccy[CAND_CAP], ccz[CAND_CAP];
@@ -608,30 +626,28 @@ __device__ __forceinline__ void assign_b(const double* sx, const double* sy, con
     const int sum = redi[0] + redi[1] + redi[2] + redi[3];
     if (sum) atomicAdd(&chg[bid % CHG], sum);
   }
+  if (bid == 0 && tid < 2) ctr[2 * tid + ((it + 1) & 1)] = 0;
   __syncthreads();
-  if (live) {
-    const int at = bc < CAND_CAP ? lbase[bc] + rank : atomicAdd(&cnt[bj], 1);
-    if (at < cap) bucket[(long)bj * cap + at] = orig;
-  }
+  const int at = !live ? 0 : (bc < CAND_CAP ? lbase[bc] + rank : atomicAdd(&cnt[bj], 1));
+  list_member(live, bj, at, orig, bucket, cap, over, &ctr[it & 1]);
 }
 template <int CPT>
 __global__ __launch_bounds__(256) void assign(const double* sx, const double* sy, const double* sz,
                                               const int* perm, long n, const double* boxes, const double* wboxes,
                                               const double* cen, int k, int* map_new, const int* map_old, int* cnt,
-                                              int* bucket, int cap, int* chg, const State* st, int it,
-                                              int seen) {
-  assign_b<CPT>(sx, sy, sz, perm, n, boxes, wboxes, cen, k, map_new, map_old, cnt, bucket, cap, chg, st, it, seen,
-                (int)blockIdx.x);
+                                              int* bucket, int cap, int2* over, int* ctr, int* chg, const State* st,
+                                              int it, int seen) {
+  assign_b<CPT>(sx, sy, sz, perm, n, boxes, wboxes, cen, k, map_new, map_old, cnt, bucket, cap, over, ctr, chg, st, it,
+                seen, (int)blockIdx.x);
 }
 
 // Buckets of an assignment given in grid order.
-__global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k, int* cnt, int* bucket, int cap) {
+__global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k, int* cnt, int* bucket, int cap, int2* over,
+                                                  int* ctr) {
   const long i = blockIdx.x * 256L + threadIdx.x;
-  if (i >= n) return;
-  const int key = map[i];
-  if ((unsigned)key >= (unsigned)k) return;
-  const int at = atomicAdd(&cnt[key], 1);
-  if (at < cap) bucket[(long)key * cap + at] = (int)i;
+  const int key = i < n ? map[i] : -1;
+  const bool live = (unsigned)key < (unsigned)k;
+  list_member(live, key, live ? atomicAdd(&cnt[key], 1) : 0, (int)i, bucket, cap, over, ctr);
 }
 
 // Weighted centroid of one cluster per workgroup, its members' rho and rho * x
@@ -643,10 +659,11 @@ __global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k,
 // less on a 64^3 grid), a scan of the words' bit counts gives every member its
 // rank, the values go to LDS by rank, and lanes 0..3 run the four sequential
 // sums.  Up to SB_R members a thread stay in registers, their values on the
-// way while the bits are counted; larger clusters, and index ranges wider than
-// the window, take the general passes, and a cluster with more members than
-// its bucket holds reads them from the whole map (perm: the map's order, null:
-// grid order).
+// way while the bits are counted.  Larger clusters, and index ranges wider than
+// the window, are partitioned by window first (in 'seg', of which every such
+// cluster takes as many entries as it has members), so that each member is set
+// as a bit once, whatever the range; wave 0 then adds a run of members while
+// the other waves look up the next run by rank.
 //
 // Bound by latency: two dependent loads and the chain of adds (about 9 ns
 // each).  N = 262144, K = 1024: 13 us, where the stable counting sort and the
@@ -654,32 +671,105 @@ __global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k,
 constexpr int SB_W = 2048;  // words of the window
 constexpr int SB_M = 512;   // members summed at a time
 constexpr int SB_R = 4;     // members a thread of the register path
+constexpr int SB_H = SB_M / 2;  // members of a run of the partitioned path
+constexpr int SB_BINS = 512;    // windows partitioned at a time
+static_assert(SB_W * 32 == 1 << 16, "window of an index: its bits from 16 on");
 
 struct SumsLds {
-  unsigned bm[SB_W];
-  unsigned short pre[SB_W];                            // members before a word (register path)
-  int list[SB_M];                                      // members in order (general passes)
+  __attribute__((aligned(16))) unsigned bm[SB_W];
+  unsigned short pre[SB_W];                            // members before a word
+  int bin[SB_BINS];                                    // members by window, then where each window's end in 'seg'
   __attribute__((aligned(16))) double buf[4][SB_M + 2];  // [w, x, y, z][member], rows on different banks
   int red[4], red2[4];
+  int at;
 };
 
-// Members before this thread's words wb .. we - 1 of the window, and in all.
-__device__ inline void sums_rank(SumsLds& S, int wb, int we, int& pos, int& total) {
+// v summed over the threads before this one, and over all.
+__device__ inline void sums_scan(SumsLds& S, int v, int& before, int& total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int have = 0;
-  for (int w = wb; w < we; ++w) have += __popc(S.bm[w]);
-  const int upto = wave_scan(have);
+  const int upto = wave_scan(v);
   if (lane == 63) S.red[wave] = upto;
   __syncthreads();
-  pos = upto - have;
+  before = upto - v;
   total = 0;
   for (int w = 0; w < 4; ++w) {
-    if (w < wave) pos += S.red[w];
+    if (w < wave) before += S.red[w];
     total += S.red[w];
   }
 }
 
-__device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int cap, const int* map, const int* perm,
+// pre of this thread's words wb .. we - 1 of the window; a barrier inside, none
+// at the end.
+__device__ inline void sums_rank(SumsLds& S, int wb, int we) {
+  int have = 0, pos, total;
+  for (int w = wb; w < we; ++w) have += __popc(S.bm[w]);
+  sums_scan(S, have, pos, total);
+  for (int w = wb; w < we; ++w) {
+    S.pre[w] = (unsigned short)pos;
+    pos += __popc(S.bm[w]);
+  }
+}
+
+// Member of rank r of the window, as an offset into it.
+__device__ inline int sums_member(const SumsLds& S, int r) {
+  int w = 0;
+#pragma unroll
+  for (int step = SB_W / 2; step > 0; step >>= 1)
+    if (S.pre[w + step] <= r) w += step;  // the last word with at most r members before it
+  unsigned bits = S.bm[w], at = 0;
+  int left = r - S.pre[w];
+#pragma unroll
+  for (int half = 16; half > 0; half >>= 1) {
+    const int low = __popc(bits & ((1u << half) - 1));
+    if (left >= low) {
+      left -= low;
+      bits >>= half;
+      at += half;
+    }
+  }
+  return 32 * w + (int)at;
+}
+
+// acc + the members seg[0 .. len) of the window at w0 in ascending order.
+__device__ inline double sums_window(SumsLds& S, double acc, int w0, const int* seg, int len, const double* rho,
+                                     const double* grid) {
+  const int tid = threadIdx.x;
+  for (int w = tid; w < SB_W / 4; w += 256) reinterpret_cast<uint4*>(S.bm)[w] = make_uint4(0, 0, 0, 0);
+  __syncthreads();
+  for (int t = tid; t < len; t += 256 * 4) {
+    int e[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) e[u] = t + 256 * u < len ? seg[t + 256 * u] : -1;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (e[u] >= 0) atomicOr(&S.bm[(e[u] - w0) >> 5], 1u << (e[u] & 31));
+  }
+  __syncthreads();
+  sums_rank(S, tid * (SB_W / 256), (tid + 1) * (SB_W / 256));
+  __syncthreads();
+  auto values = [&](int run) {  // of the members of a run, by waves 1 to 3
+    const int h = (run & 1) * SB_H, end = min(len, (run + 1) * SB_H);
+#pragma unroll 2
+    for (int r = run * SB_H + tid - 64; r < end; r += 192) {
+      const long e = w0 + sums_member(S, r);
+      const double q = rho[e];
+      double* b = &S.buf[0][h + r - run * SB_H];
+      b[0] = q;
+      for (int d = 0; d < 3; ++d) b[(1 + d) * (SB_M + 2)] = q * grid[e * 3 + d];
+    }
+  };
+  const int runs = (len + SB_H - 1) / SB_H;
+  if (tid >= 64) values(0);
+  __syncthreads();
+  for (int run = 0; run < runs; ++run) {
+    if (tid < 4) acc = seq_sum(acc, &S.buf[tid][(run & 1) * SB_H], min(SB_H, len - run * SB_H));
+    if (tid >= 64 && run + 1 < runs) values(run + 1);
+    __syncthreads();
+  }
+  return acc;
+}
+
+__device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int cap, const int2* over, int* ctr, int* seg,
                                                      long n, const double* rho, const double* grid, double* cen_out,
                                                      State* st, int it, int seen, int c) {
   __shared__ SumsLds S;
@@ -704,20 +794,6 @@ __device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int
         for (int d = 0; d < 3; ++d) v[u][1 + d] = grid[i[u] * 3L + d];
       }
   }
-  // every member: f(grid index)
-  auto members = [&](auto f) {
-    if (listed) {
-      for (int t = tid; t < m; t += 256) f(mem[t]);
-    } else {
-      for (long p = tid; p < n; p += 256)
-        if (map[p] == c) f(perm ? perm[p] : (int)p);
-    }
-  };
-  if (!few)
-    members([&](int e) {
-      lo = min(lo, e);
-      hi = min(hi, -e);
-    });
   lo = wave_min(lo);
   hi = wave_min(hi);
   if (lane == 0) { S.red[wave] = lo; S.red2[wave] = hi; }
@@ -732,12 +808,7 @@ __device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int
     for (int u = 0; u < SB_R; ++u)
       if (tid + 256 * u < m) atomicOr(&S.bm[(i[u] - lo) >> 5], 1u << (i[u] & 31));
     __syncthreads();
-    int pos, total;
-    sums_rank(S, wb, wb + per, pos, total);
-    for (int w = wb; w < wb + per; ++w) {
-      S.pre[w] = (unsigned short)pos;
-      pos += __popc(S.bm[w]);
-    }
+    sums_rank(S, wb, wb + per);
     __syncthreads();
     for (int base = 0; base < m; base += SB_M) {
 #pragma unroll
@@ -754,39 +825,56 @@ __device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int
       if (tid < 4) acc = seq_sum(acc, S.buf[tid], min(SB_M, m - base));
       if (base + SB_M < m) __syncthreads();
     }
-  } else {
-    for (long w0 = lo; m > 0 && w0 <= hi; w0 += SB_W * 32L) {
-      const int nw = (int)min((long)SB_W, ((hi - w0) >> 5) + 1);
-      if (w0 > lo) {
-        for (int w = tid; w < nw; w += 256) S.bm[w] = 0;
-        __syncthreads();
+  } else if (m > 0) {
+    // every member: f(grid index), eight loads in flight
+    const int nb = min(m, cap), no = listed ? 0 : ctr[it & 1];
+    auto members = [&](auto f) {
+      for (int t = tid; t < nb; t += 256 * 8) {
+        int e[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) e[u] = t + 256 * u < nb ? mem[t + 256 * u] : -1;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (e[u] >= 0) f(e[u]);
       }
+      for (int t = tid; t < no; t += 256 * 8) {
+        int2 e[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) e[u] = t + 256 * u < no ? over[t + 256 * u] : make_int2(-1, 0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (e[u].x == c) f(e[u].y);
+      }
+    };
+    if (tid == 0) S.at = atomicAdd(&ctr[2 + (it & 1)], m);
+    __syncthreads();
+    int base = S.at;
+    for (long r0 = 0; r0 < n; r0 += SB_BINS * (SB_W * 32L)) {
+      for (int q = tid; q < SB_BINS; q += 256) S.bin[q] = 0;
+      __syncthreads();
       members([&](int e) {
-        const long o = e - w0;
-        if (o >= 0 && o < SB_W * 32L) atomicOr(&S.bm[o >> 5], 1u << (o & 31));
+        const long q = (e - r0) >> 16;
+        if (e >= r0 && q < SB_BINS) atomicAdd(&S.bin[q], 1);
       });
       __syncthreads();
-      const int per = (nw + 255) / 256, wb = min(nw, tid * per), we = min(nw, wb + per);
-      int pos, total;
-      sums_rank(S, wb, we, pos, total);
-      for (int base = 0; base < total; base += SB_M) {
-        int q = pos - base;
-        for (int w = wb; w < we; ++w)
-          for (unsigned bits = S.bm[w]; bits; bits &= bits - 1, ++q)
-            if (q >= 0 && q < SB_M) S.list[q] = (int)(w0 + 32 * w) + __ffs(bits) - 1;
-        __syncthreads();
-        const int len = min(SB_M, total - base);
-        for (int t = tid; t < len; t += 256) {
-          const long e = S.list[t];
-          const double r = rho[e];
-          S.buf[0][t] = r;
-          for (int d = 0; d < 3; ++d) S.buf[1 + d][t] = r * grid[e * 3 + d];
-        }
-        __syncthreads();
-        if (tid < 4) acc = seq_sum(acc, S.buf[tid], len);
-        __syncthreads();
+      const int h0 = S.bin[2 * tid], h1 = S.bin[2 * tid + 1];
+      int before, total;
+      sums_scan(S, h0 + h1, before, total);
+      S.bin[2 * tid] = base + before;
+      S.bin[2 * tid + 1] = base + before + h0;
+      __syncthreads();
+      members([&](int e) {
+        const long q = (e - r0) >> 16;
+        if (e >= r0 && q < SB_BINS) seg[atomicAdd(&S.bin[q], 1)] = e;
+      });
+      __syncthreads();
+      const int windows = (int)min((long)SB_BINS, (n - r0 + SB_W * 32 - 1) / (SB_W * 32));
+      for (int q = 0; q < windows; ++q) {
+        const int end = S.bin[q];
+        if (end > base) acc = sums_window(S, acc, (int)r0 + q * (SB_W * 32), seg + base, end - base, rho, grid);
+        base = end;
       }
-      __syncthreads();  // an empty window: its counts are read before they are cleared
+      __syncthreads();
     }
   }
   if (tid >= 64) return;
@@ -797,10 +885,10 @@ __device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int
   }
   if (lane >= 1 && lane < 4) cen_out[c * 3 + lane - 1] = acc / w;
 }
-__global__ __launch_bounds__(256) void centroid_sums(int* cnt, const int* bucket, int cap, const int* map,
-                                                     const int* perm, long n, const double* rho, const double* grid,
+__global__ __launch_bounds__(256) void centroid_sums(int* cnt, const int* bucket, int cap, const int2* over, int* ctr,
+                                                     int* seg, long n, const double* rho, const double* grid,
                                                      double* cen_out, State* st, int it, int seen) {
-  centroid_sums_b(cnt, bucket, cap, map, perm, n, rho, grid, cen_out, st, it, seen, (int)blockIdx.x);
+  centroid_sums_b(cnt, bucket, cap, over, ctr, seg, n, rho, grid, cen_out, st, it, seen, (int)blockIdx.x);
 }
 
 // normed_difference(new, cur) with the reference's sequential sum, % changed,
@@ -1040,8 +1128,8 @@ static int bits_for(int nb) {
 }
 
 // Members a cluster's bucket holds: eight times the average (the largest
-// clusters of the 64^3 systems reach four times), a larger cluster is read
-// from the map.
+// clusters of filled 64^3 cells reach four times); those of larger clusters, as
+// vacuum around a molecule or slab gives, share one list.
 static int bucket_cap(long n, int k) { return (int)std::min<long>(n, std::max<long>(256, 8 * ((n + k - 1) / k))); }
 
 // A normed difference is never negative, so a negative threshold never stops
@@ -1073,7 +1161,8 @@ static Layout plan(long n, int k, int max_it, bool defer) {
 struct Bufs {
   double *part, *sx, *sy, *sz, *boxes, *wboxes, *cen, *diffs, *pcts;  // cen: L.ncen centroid buffers
   int *keys, *perm, *map[2], *tc, *total, *start, *idx0;     // map: in tile order
-  int *cnt, *bucket, *chg;
+  int *cnt, *bucket, *ctr, *seg, *chg;
+  int2* over;
   State* st;
 };
 
@@ -1090,6 +1179,7 @@ static size_t bytes_for(const Layout& L, bool full) {
     b += carve_bytes<double>(3L * L.k * L.ncen) + 2 * carve_bytes<double>(std::max(1, L.max_it));
     b += 2 * carve_bytes<int>(n) + carve_bytes<int>(L.k);
     b += carve_bytes<int>(L.k) + carve_bytes<int>((size_t)L.k * L.cap) + carve_bytes<int>((size_t)L.nchg * CHG);
+    b += carve_bytes<int>(4) + carve_bytes<int>(n) + carve_bytes<int2>(n);
   }
   return b;
 }
@@ -1121,7 +1211,11 @@ static bool carve(Arena& a, const Layout& L, Bufs& b, bool full) {
     b.cnt = a.take<int>(L.k);
     b.bucket = a.take<int>((size_t)L.k * L.cap);
     b.chg = a.take<int>((size_t)L.nchg * CHG);
-    ok = ok && b.cen && b.diffs && b.pcts && b.map[0] && b.map[1] && b.idx0 && b.cnt && b.bucket && b.chg;
+    b.ctr = a.take<int>(4);
+    b.seg = a.take<int>(n);
+    b.over = a.take<int2>(n);
+    ok = ok && b.cen && b.diffs && b.pcts && b.map[0] && b.map[1] && b.idx0 && b.cnt && b.bucket && b.chg && b.ctr &&
+         b.seg && b.over;
   }
   return ok;
 }
@@ -1170,7 +1264,7 @@ static int enqueue_kmeans(const Layout& L, const Bufs& b, const double* grid, co
                           const hipEvent_t kev[3]) {
   const long cs = 3L * L.k;
   const bool two = sa != s;
-  hipLaunchKernelGGL(init_run, dim3(ceil_div(L.k, 256)), dim3(256), 0, s, grid, b.idx0, L.k, b.cen, b.cnt, b.chg,
+  hipLaunchKernelGGL(init_run, dim3(ceil_div(L.k, 256)), dim3(256), 0, s, grid, b.idx0, L.k, b.cen, b.cnt, b.ctr, b.chg,
                      L.nchg * CHG, b.st);
   enqueue_setup(L, b, grid, s);
   const size_t dyn = (size_t)3 * L.k * sizeof(double);
@@ -1182,11 +1276,11 @@ static int enqueue_kmeans(const Layout& L, const Bufs& b, const double* grid, co
     if (!L.defer && two && it >= 2) THC_HIP(hipStreamWaitEvent(s, kev[1 + par], 0));  // diff_control(it - 2)
     with_cpt(L.k, [&](auto cpt) {
       hipLaunchKernelGGL(assign<cpt.value>, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes,
-                         b.wboxes, b.cen + cur * cs, L.k, mnew, mold, b.cnt, b.bucket, L.cap, b.chg + chg_at(L, it),
-                         b.st, it, seen);
+                         b.wboxes, b.cen + cur * cs, L.k, mnew, mold, b.cnt, b.bucket, L.cap, b.over, b.ctr,
+                         b.chg + chg_at(L, it), b.st, it, seen);
     });
-    hipLaunchKernelGGL(centroid_sums, dim3(L.k), dim3(256), 0, s, b.cnt, b.bucket, L.cap, mnew, b.perm, L.n, rho, grid,
-                       b.cen + nxt * cs, b.st, it, seen);
+    hipLaunchKernelGGL(centroid_sums, dim3(L.k), dim3(256), 0, s, b.cnt, b.bucket, L.cap, b.over, b.ctr, b.seg,
+                       L.n, rho, grid, b.cen + nxt * cs, b.st, it, seen);
     if (L.defer) continue;
     if (two) {
       THC_HIP(hipEventRecord(kev[0], s));
@@ -1272,7 +1366,7 @@ __device__ inline int job_of(const int* off, int nj, int b) {
 
 __global__ __launch_bounds__(256) void init_run_m(const Job* jobs, const int* off, int nj) {
   KM_JOB(off)
-  init_run_b(q.grid, q.b.idx0, q.L.k, q.b.cen, q.b.cnt, q.b.chg, q.L.nchg * CHG, q.b.st, bid, nblk);
+  init_run_b(q.grid, q.b.idx0, q.L.k, q.b.cen, q.b.cnt, q.b.ctr, q.b.chg, q.L.nchg * CHG, q.b.st, bid, nblk);
 }
 
 __global__ __launch_bounds__(256) void bbox_partial_m(const Job* jobs, const int* off, int nj) {
@@ -1321,15 +1415,15 @@ __global__ __launch_bounds__(256) void assign_m(const Job* jobs, const int* off,
   if (it >= q.L.max_it) return;
   const int par = it & 1;
   assign_b<CPT>(q.b.sx, q.b.sy, q.b.sz, q.b.perm, q.L.n, q.b.boxes, q.b.wboxes, job_cen(q, it), q.L.k, q.b.map[par],
-           it == 0 ? nullptr : q.b.map[par ^ 1], q.b.cnt, q.b.bucket, q.L.cap, q.b.chg + chg_at(q.L, it), q.b.st, it,
-           it - 1, bid);
+           it == 0 ? nullptr : q.b.map[par ^ 1], q.b.cnt, q.b.bucket, q.L.cap, q.b.over, q.b.ctr,
+           q.b.chg + chg_at(q.L, it), q.b.st, it, it - 1, bid);
 }
 
 __global__ __launch_bounds__(256) void centroid_sums_m(const Job* jobs, const int* off, int nj, int it) {
   KM_JOB(off)
   (void)nblk;
   if (it >= q.L.max_it) return;
-  centroid_sums_b(q.b.cnt, q.b.bucket, q.L.cap, q.b.map[it & 1], q.b.perm, q.L.n, q.rho, q.grid, job_cen(q, it + 1),
+  centroid_sums_b(q.b.cnt, q.b.bucket, q.L.cap, q.b.over, q.b.ctr, q.b.seg, q.L.n, q.rho, q.grid, job_cen(q, it + 1),
                   q.b.st, it, it - 1, bid);
 }
 
@@ -1637,7 +1731,7 @@ int kmeans_classify(thc_ctx* ctx, const double* grid, long n, const double* cent
   with_cpt(k, [&](auto cpt) {
     hipLaunchKernelGGL(assign<cpt.value>, dim3(L.ntiles), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes,
                        b.wboxes, centroids, k, grid_map, (const int*)nullptr, (int*)nullptr, (int*)nullptr, 0,
-                       (int*)nullptr, (const State*)nullptr, 0, -1);
+                       (int2*)nullptr, (int*)nullptr, (int*)nullptr, (const State*)nullptr, 0, -1);
   });
   THC_HIP(hipGetLastError());
   THC_HIP(hipStreamSynchronize(s));
@@ -1651,19 +1745,24 @@ int kmeans_update(thc_ctx* ctx, const double* rho, const double* grid, long n, c
   if (k > MAXB) return THC_ERR_UNSUPPORTED;
   THC_HIP(hipSetDevice(ctx->device));
   const int cap = bucket_cap(n, k);
-  THC_TRY(ctx->ws.reserve(carve_bytes<State>(1) + carve_bytes<int>(k) + carve_bytes<int>((size_t)k * cap)));
+  THC_TRY(ctx->ws.reserve(carve_bytes<State>(1) + carve_bytes<int>(k) + carve_bytes<int>((size_t)k * cap) +
+                          carve_bytes<int>(4) + carve_bytes<int>(n) + carve_bytes<int2>(n)));
   ctx->ws.reset();
   State* st = ctx->ws.take<State>(1);
   int* cnt = ctx->ws.take<int>(k);
   int* bucket = ctx->ws.take<int>((size_t)k * cap);
-  if (!st || !cnt || !bucket) return THC_ERR_NO_MEMORY;
+  int* ctr = ctx->ws.take<int>(4);
+  int* seg = ctx->ws.take<int>(n);
+  int2* over = ctx->ws.take<int2>(n);
+  if (!st || !cnt || !bucket || !ctr || !seg || !over) return THC_ERR_NO_MEMORY;
   hipStream_t s = ctx->stream;
   hipLaunchKernelGGL(init_run, dim3(ceil_div(k, 256)), dim3(256), 0, s, grid, (const int*)nullptr, k, (double*)nullptr,
-                     cnt, (int*)nullptr, 0, st);
+                     cnt, ctr, (int*)nullptr, 0, st);
   hipLaunchKernelGGL(check_keys, dim3(256), dim3(256), 0, s, grid_map, n, k, st);
-  hipLaunchKernelGGL(bucket_map, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, grid_map, n, k, cnt, bucket, cap);
-  hipLaunchKernelGGL(centroid_sums, dim3(k), dim3(256), 0, s, cnt, bucket, cap, grid_map, (const int*)nullptr, n, rho,
-                     grid, centroids, st, 0, -1);
+  hipLaunchKernelGGL(bucket_map, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, grid_map, n, k, cnt, bucket, cap,
+                     over, ctr);
+  hipLaunchKernelGGL(centroid_sums, dim3(k), dim3(256), 0, s, cnt, bucket, cap, over, ctr, seg, n, rho, grid, centroids, st,
+                     0, -1);
   THC_HIP(hipGetLastError());
   State hst;
   THC_HIP(hipMemcpyAsync(&hst, st, sizeof(State), hipMemcpyDeviceToHost, s));
@@ -1688,7 +1787,7 @@ int kmeans_map_to_grid(thc_ctx* ctx, const double* grid, long n, const double* c
   if (!carve(ctx->ws, L, b, false)) return THC_ERR_NO_MEMORY;
   hipStream_t s = ctx->stream;
   hipLaunchKernelGGL(init_run, dim3(1), dim3(256), 0, s, grid, (const int*)nullptr, 0, (double*)nullptr,
-                     (int*)nullptr, (int*)nullptr, 0, b.st);
+                     (int*)nullptr, (int*)nullptr, (int*)nullptr, 0, b.st);
   enqueue_setup(L, b, grid, s);
   hipLaunchKernelGGL(map_to_grid, dim3(k), dim3(256), 0, s, b.sx, b.sy, b.sz, b.perm, L.n, b.boxes, L.ntiles,
                      centroids, 0L, 0, (const State*)nullptr, false, interp_idx);
