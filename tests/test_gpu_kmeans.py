@@ -415,3 +415,22 @@ def test_kmeans_vacuum(ctx):
         np.testing.assert_array_equal(out["diffs"], ref["diffs"])
         np.testing.assert_array_equal(out["grid_map"].cpu().numpy(), ref["maps"][-1])
         np.testing.assert_array_equal(out["centroids"].cpu().numpy(), ref["centroids"])
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (255, 2), (1023, 4), (1024, 1024), (1025, 7), (5000, 4096)])
+def test_update_centroids_tile_edges(ctx, n, k):
+    """Point counts either side of the 1024-point tiles that fill the buckets, every key count; a key outside
+    [0, k) in the first and last place of a tile is refused."""
+    rng = np.random.default_rng(n + k)
+    grid = rng.uniform(0, 7, size=(n, 3))
+    rho = rng.uniform(0.1, 2.0, size=n)
+    gmap = rng.permutation(np.arange(n) % k).astype(np.int32)
+    got, st = ctx.update_centroids(rho, grid, gmap, k)
+    ref, crit = KO.update_centroids(rho, grid, gmap, k)
+    assert st == L.THC_OK and crit == 0
+    np.testing.assert_array_equal(got.cpu().numpy(), ref)
+    for at in sorted({0, min(n, 1024) - 1, n - 1}):
+        for key in (-1, k, 2 ** 31 - 1):
+            bad = gmap.copy()
+            bad[at] = key
+            assert ctx.update_centroids(rho, grid, bad, k)[1] == L.THC_ERR_ARG
