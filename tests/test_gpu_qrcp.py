@@ -120,3 +120,27 @@ def test_qrcp_no_finite_residual(ctx):
     for fill in (0.0, np.nan):
         st, _, _ = ctx.qrcp_points(np.full((700, 4), fill), 3)
         assert st == L.THC_ERR_NOT_POSDEF
+
+
+@pytest.mark.parametrize("m,copies,alone,k,half,cplx", [(10, 1100, 0, 40, False, False), (14, 400, 45, 64, False, False),
+                                                        (14, 300, 70, 72, False, False), (12, 350, 60, 64, True, False),
+                                                        (9, 300, 40, 64, False, True)])
+def test_qrcp_equal_points_in_rounds(ctx, m, copies, alone, k, half, cplx):
+    """More equal points than a round takes candidates, as symmetry gives, in runs long enough for rounds: the first
+    copy of a point is the pivot; with points of their own between them the run changes between rounds and steps."""
+    rng = np.random.default_rng(k + copies)
+    base = 90 if alone else 45
+    a = _orbitals(base, m, k) * rng.uniform(0.3, 1.0, (base, 1))
+    if cplx:
+        a = a * np.exp(2j * np.pi * rng.random(a.shape))
+    reps = np.where(np.arange(base) % 90 < alone, 1, copies)[rng.permutation(base)]
+    occ = np.ascontiguousarray(a[:, : m - 2]) if half else None
+    big, bocc = np.repeat(a, reps, axis=0), None if occ is None else np.repeat(occ, reps, axis=0)
+    assert k >= 64 or len(big) > 40000
+    first = np.concatenate([[0], np.cumsum(reps)[:-1]])
+    print("qrcp equal points: m=%d n=%d k=%d" % (m, len(big), k), flush=True)
+    ref_idx, ref_rd, _ = QO.qrcp_points(a, k, occ)
+    st, idx, rd = ctx.qrcp_points_complex(big, k) if cplx else ctx.qrcp_points(big, k, bocc)
+    assert st == L.THC_OK
+    np.testing.assert_array_equal(idx.cpu().numpy(), first[ref_idx])
+    np.testing.assert_allclose(rd, ref_rd, rtol=1e-7)

@@ -32,6 +32,11 @@
 // QC = 256 candidates: 128 give 37 rounds, 512 give 21 with a four times
 // larger block.
 //
+// Where more than QC points share the top bin -- symmetry-equivalent points of a
+// crystal, whose residuals are equal -- no set of candidates holds every point
+// that may be next.  The run then goes on one pivot a step (qr_step), and tries
+// a round again after 4, 8, ... 32 of them.
+//
 // Complex orbitals (ZT[(i k), a] = conj(phi_i(r_a)) phi_k(r_a), src/qrcp.cpp:
 // 33-48): with Q[a][b] = sum_k conj(phi_k(a)) phi_k(b) the Gram matrix is
 // conj(Q) o Q = |Q|^2, real, and the steps above apply with g_a = |Q[a][p]|^2.
@@ -128,10 +133,11 @@ constexpr int QR_MAX = 32;    // pivots of a round: two MFMA tiles of columns
 constexpr int QBINS = 1536;   // bins of the residual histogram: 128 an octave, 12 octaves below the reference
 constexpr int QBIN_SHIFT = 13;  // a residual's bin: the exponent and 7 mantissa bits of its high word
 
-enum { G_SQUARE = 0, G_PRODUCT = 1, G_MODULUS = 2 };  // G = P^2, P Pocc, |P|^2 (complex)
+// G = P^2, P Pocc, |P|^2 (complex), conj(Pocc) P (complex half-rotated: G itself is complex)
+enum { G_SQUARE = 0, G_PRODUCT = 1, G_MODULUS = 2, G_COMPLEX = 3 };
 
 struct QrState {
-  int j, fail, done;  // pivots chosen, step that found none (1-based), run ended: read back together
+  int j, done, stall;  // pivots chosen, run ended, no candidates to be had: read back together
   int base, r;      // pivots chosen before this round, chosen in it
   int ncand, cut;   // candidates, the lowest bin (counted downwards) that is among them
   int refkey;       // bin key no residual is above
@@ -167,15 +173,20 @@ __device__ inline void qr_top(const double* pv, const int* pi, int nparts, doubl
     if (wins(sv[q], si[q], v, vi)) { v = sv[q]; vi = si[q]; }
 }
 
-// Start: the reference residual, an empty histogram.
-__global__ __launch_bounds__(QB) void qr_begin(const double* pv, const int* pi, int nparts, QrState* st, int* hist) {
+// Start of the rounds with j of k pivots chosen: the reference residual, an
+// empty histogram.
+__global__ __launch_bounds__(QB) void qr_begin(const double* pv, const int* pi, int nparts, int j, int k, int* fail,
+                                               QrState* st, int* hist) {
   __shared__ double sv[QB / 64];
   __shared__ int si[QB / 64];
   double v;
   int vi;
   qr_top(pv, pi, nparts, v, vi, sv, si);
   if (threadIdx.x == 0) {
-    st->j = st->base = st->r = st->ncand = st->fail = st->done = 0;
+    st->j = j;
+    st->base = st->r = st->ncand = st->stall = 0;
+    if (j == 0) *fail = 0;
+    st->done = *fail || j >= k;
     st->cut = -1;
     st->refkey = v > 0.0 ? qr_key(v) : 0;
   }
@@ -202,17 +213,14 @@ __global__ __launch_bounds__(QB) void qr_hist(const double* __restrict__ d, long
 }
 
 // Candidates: the points of the most bins from the top that hold at most QC
-// of them.  If the top bin alone holds more (or nothing is in range), the
-// first maximum is the only candidate.
-__global__ __launch_bounds__(QB) void qr_pick(const double* __restrict__ d, long n, int nparts, const double* pv,
-                                              const int* pi, const int* __restrict__ hist, QrState* st, int* cand) {
-  if (st->done) return;
+// of them.  None if the top bin alone holds more (or nothing is in range).
+__global__ __launch_bounds__(QB) void qr_pick(const double* __restrict__ d, long n, const int* __restrict__ hist,
+                                              QrState* st, int* cand) {
+  if (st->done || st->stall) return;
   constexpr int PER = QBINS / QB;
   static_assert(PER * QB == QBINS, "bins split evenly over the threads");
   __shared__ int part[QB];
   __shared__ int cut;
-  __shared__ double sv[QB / 64];
-  __shared__ int si[QB / 64];
   const int t = threadIdx.x;
   const int refkey = st->refkey;
   int c[PER], sum = 0;
@@ -237,20 +245,8 @@ __global__ __launch_bounds__(QB) void qr_pick(const double* __restrict__ d, long
     if (run > 0 && run <= QC) atomicMax(&cut, t * PER + q);
   }
   __syncthreads();
-  if (cut < 0) {
-    if (blockIdx.x == 0) {
-      double v;
-      int vi;
-      qr_top(pv, pi, nparts, v, vi, sv, si);
-      if (t == 0) {
-        st->cut = -1;
-        st->ncand = vi >= 0 && vi < n ? 1 : 0;
-        cand[0] = vi;
-      }
-    }
-    return;
-  }
   if (blockIdx.x == 0 && t == 0) st->cut = cut;
+  if (cut < 0) return;
   const long a = (long)blockIdx.x * QB + t;
   const double v = a < n ? d[a] : 0.0;
   if (v > 0.0 && qr_bin(v, refkey) <= cut) cand[atomicAdd(&st->ncand, 1)] = (int)a;
@@ -260,7 +256,7 @@ __global__ __launch_bounds__(QB) void qr_pick(const double* __restrict__ d, long
 // and slots without a candidate.
 __global__ __launch_bounds__(QC) void qr_gather(const double* __restrict__ L, long ln, const QrState* st,
                                                 const int* __restrict__ cand, double* __restrict__ LT) {
-  if (st->done) return;
+  if (st->done || st->ncand == 0) return;
   const int t = threadIdx.x, j = st->j, j4 = (j + 3) & ~3;
   const bool ok = t < st->ncand;
   const double* src = L + (ok ? cand[t] : 0);
@@ -381,14 +377,16 @@ __device__ inline double qr_wave_max(double v) {
 
 // Pivot steps on the candidates, until the largest residual falls out of
 // their bins.  The first pivot of a round is the first maximum over all points
-// in any case: the candidates hold every point of the top bin.  One wave, four
+// in any case: the candidates hold every point of the top bin; without
+// candidates the round ends here (stall).  One wave, four
 // candidates a lane (lane l owns l, l + 64, ...), so a step is a chain without
 // barriers: the maximum over the lanes, one row of S, r multiply-adds.  The
 // other waves read S once, so that its rows are in this XCD's L2 by then.
 __global__ __launch_bounds__(1024) void qr_run(const double* __restrict__ S, const double* __restrict__ d,
                                              const int* __restrict__ cand, int k, QrState* st, int* __restrict__ hist,
-                                             int* __restrict__ piv, double* __restrict__ rdiag) {
-  if (st->done) return;
+                                             int* __restrict__ piv, double* __restrict__ rdiag,
+                                             int* __restrict__ fail_out) {
+  if (st->done || st->stall) return;
   constexpr int PL = QC / 64;
   __shared__ double lh[QR_MAX][QC];
   const int lane = threadIdx.x & 63;
@@ -398,6 +396,10 @@ __global__ __launch_bounds__(1024) void qr_run(const double* __restrict__ S, con
     const int lines = (nc + 15) / 16;  // 128-byte lines of a row's first nc entries
     for (int q = threadIdx.x - 64; q < nc * lines; q += 1024 - 64) sum += S[(long)(q / lines) * QC + q % lines * 16];
     asm volatile("" ::"v"(sum));
+    return;
+  }
+  if (cut < 0) {
+    if (lane == 0) st->stall = 1;
     return;
   }
   int me[PL];
@@ -427,7 +429,7 @@ __global__ __launch_bounds__(1024) void qr_run(const double* __restrict__ S, con
     v = top;
     vi = __builtin_amdgcn_readlane(vi, win);
     vs = __builtin_amdgcn_readlane(vs, win);
-    if (r > 0 && (cut < 0 || !(v > 0.0) || qr_bin(v, refkey) > cut)) break;
+    if (r > 0 && (!(v > 0.0) || qr_bin(v, refkey) > cut)) break;
     if (j + r == 0) d0 = v;
     // residual exhausted (K beyond the numerical rank): below 1e-13 of the first
     // pivot the squared residuals are rounding noise of the Gram downdate
@@ -471,7 +473,7 @@ __global__ __launch_bounds__(1024) void qr_run(const double* __restrict__ S, con
     st->j = j + r;
     st->ncand = 0;
     st->refkey = newkey;
-    st->fail = fail;
+    if (fail) *fail_out = fail;  // the step that found no pivot, 1-based
     st->done = fail || j + r >= k;
   }
 }
@@ -481,7 +483,7 @@ __global__ __launch_bounds__(1024) void qr_run(const double* __restrict__ S, con
 // the 40^3, K = 512 run took 3.05 ms, with this kernel 2.80.
 __global__ __launch_bounds__(256) void qr_compact(const QrState* st, const double* __restrict__ LT,
                                                   double* __restrict__ LP) {
-  if (st->done) return;
+  if (st->done || st->stall) return;
   const int s = threadIdx.x & (QR_MAX - 1), j4 = (st->base + 3) & ~3;
   const bool ok = s < st->r;
   const double* src = LT + (ok ? st->slot[s] : 0);
@@ -505,7 +507,7 @@ __global__ __launch_bounds__(64 * QW) void qr_apply(const double* __restrict__ p
                                                     long n, int m, int mo, double* __restrict__ d,
                                                     double* __restrict__ L, long ln, const double* __restrict__ LP,
                                                     const QrState* __restrict__ st, double* pv, int* pi, int* hist) {
-  if (st->done) return;
+  if (st->done || st->stall) return;
   __shared__ double tile[QW][32][QR_MAX + 1];
   __shared__ int h[QBINS];
   __shared__ double sv[QW];
@@ -651,14 +653,15 @@ __global__ __launch_bounds__(64 * QW) void qr_apply(const double* __restrict__ p
   }
 }
 
-// ---- one pivot a step: complex half-rotated orbitals, and few pivots of few points
+// ---- one pivot a step: complex half-rotated orbitals, few pivots, more equal points than candidates
 // Pivot step j; partial maxima are read from (pv_in, pi_in) and written to
-// (pv_out, pi_out), which the host alternates between steps.  CPLX: G and L are
-// complex, L[2q] holds the real, L[2q + 1] the imaginary parts of column q.
-template <bool CPLX>
+// (pv_out, pi_out), which the host alternates between steps.  G_COMPLEX: L is
+// complex too, row 2q (ln doubles apart) holds the real, row 2q + 1 the
+// imaginary parts of column q.
+template <int G>
 __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, const double* __restrict__ occ, long n,
                                               int m, int mo, int j, int nparts, double* __restrict__ d,
-                                              double* __restrict__ L, const double* pv_in, const int* pi_in,
+                                              double* __restrict__ L, long ln, const double* pv_in, const int* pi_in,
                                               double* pv_out, int* pi_out, int* piv, double* rdiag, int* fail) {
   extern __shared__ double sh[];  // pivot rows: phi (m), occ (mo), then L[q][p], 2j values
   __shared__ double gv;
@@ -703,11 +706,11 @@ __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, co
   double* prow = sh;
   double* orow = sh + m;
   double* lp = orow + (occ ? mo : 0);
-  constexpr int LW = CPLX ? 2 : 1;  // doubles per entry of L
+  constexpr int LW = G == G_COMPLEX ? 2 : 1;  // doubles per entry of L
   for (int q = threadIdx.x; q < m; q += QB) prow[q] = phi[p * m + q];
   if (occ)
     for (int q = threadIdx.x; q < mo; q += QB) orow[q] = occ[p * mo + q];
-  for (int q = threadIdx.x; q < LW * j; q += QB) lp[q] = L[(long)q * n + p];
+  for (int q = threadIdx.x; q < LW * j; q += QB) lp[q] = L[q * ln + p];
   __syncthreads();
   const double rs = 1.0 / sqrt(pval);
   const long a = (long)blockIdx.x * QB + threadIdx.x;
@@ -715,33 +718,36 @@ __global__ __launch_bounds__(QB) void qr_step(const double* __restrict__ phi, co
   int vi = INT_MAX;
   if (a < n) {
     double da = d[a], lr, li = 0.0;
-    if constexpr (CPLX) {
+    if constexpr (G == G_COMPLEX) {
       double qr, qi, o_r, o_i;
       cdot_row(phi + a * m, prow, m, qr, qi);
       cdot_row(occ + a * mo, orow, mo, o_r, o_i);
       const double gr = o_r * qr + o_i * qi, gi = o_r * qi - o_i * qr;  // conj(Qocc) Q
       double ar = 0.0, ai = 0.0;
       for (int q = 0; q < j; ++q) {
-        const double xr = L[(long)(2 * q) * n + a], xi = L[(long)(2 * q + 1) * n + a];
+        const double xr = L[2 * q * ln + a], xi = L[(2 * q + 1) * ln + a];
         const double yr = lp[2 * q], yi = lp[2 * q + 1];
         ar = fma(xr, yr, fma(xi, yi, ar));
         ai = fma(xi, yr, fma(-xr, yi, ai));
       }
       lr = (gr - ar) * rs;
       li = (gi - ai) * rs;
-      L[(long)(2 * j) * n + a] = lr;
-      L[(long)(2 * j + 1) * n + a] = li;
+      L[2 * j * ln + a] = lr;
+      L[(2 * j + 1) * ln + a] = li;
     } else {
-      const double g = dot_row(phi + a * m, prow, m), h = occ ? dot_row(occ + a * mo, orow, mo) : g;
+      double g, h = 0.0;
+      if constexpr (G == G_MODULUS) cdot_row(phi + a * m, prow, m, g, h);
+      else g = dot_row(phi + a * m, prow, m);
+      if constexpr (G == G_PRODUCT) h = dot_row(occ + a * mo, orow, mo);
       double s0 = 0.0, s1 = 0.0;
       int q = 0;
       for (; q + 2 <= j; q += 2) {
-        s0 = fma(L[(long)q * n + a], lp[q], s0);
-        s1 = fma(L[(long)(q + 1) * n + a], lp[q + 1], s1);
+        s0 = fma(L[q * ln + a], lp[q], s0);
+        s1 = fma(L[(q + 1) * ln + a], lp[q + 1], s1);
       }
-      if (q < j) s0 = fma(L[(long)q * n + a], lp[q], s0);
-      lr = (g * h - (s0 + s1)) * rs;
-      L[(long)j * n + a] = lr;
+      if (q < j) s0 = fma(L[q * ln + a], lp[q], s0);
+      lr = (qr_combine<G>(g, h) - (s0 + s1)) * rs;
+      L[j * ln + a] = lr;
     }
     if (a == p || da == RETIRED) da = RETIRED;
     else da -= lr * lr + li * li;
@@ -760,20 +766,46 @@ inline long qr_ln(long n) { return (n + QB - 1) / QB * QB; }
 size_t qrcp_work_bytes(long n, int k, bool cplx) {
   const long nparts = (n + QB - 1) / QB;
   return carve_bytes<double>((size_t)n) + carve_bytes<double>((size_t)qr_ln(n) * k * (cplx ? 2 : 1)) +
-         2 * carve_bytes<double>(nparts) + 2 * carve_bytes<int>(nparts) + carve_bytes<int>(k) +
-         carve_bytes<double>(k) + carve_bytes<int>(1) + carve_bytes<double>((size_t)(k + 4) * QC) +
-         carve_bytes<double>((size_t)(k + 4) * QR_MAX) + carve_bytes<double>((size_t)QC * QC) + carve_bytes<int>(QC) + carve_bytes<int>(QBINS) +
-         carve_bytes<QrState>(1);
+         2 * carve_bytes<double>(nparts) + 2 * carve_bytes<int>(nparts) +
+         carve_bytes<char>(sizeof(double) * k + sizeof(int) * ((size_t)k + 1)) + carve_bytes<double>((size_t)(k + 4) * QC) +
+         carve_bytes<double>((size_t)(k + 4) * QR_MAX) + carve_bytes<double>((size_t)QC * QC) + carve_bytes<int>(QC) +
+         carve_bytes<int>(QBINS) + carve_bytes<QrState>(1);
 }
 
 namespace {
 
-// Rounds of pivots (real G) until k are chosen; pv, pi hold the first maxima.
+// The orbitals, d, L and the maxima of a run; pv, pi [cur] are the latest.
+struct QrRun {
+  const double *phi, *occ;
+  long n;
+  int m, mo, k;
+  double *d, *L, *pv[2];
+  int* pi[2];
+  double* rd;  // rd, piv and fail lie together: one copy back
+  int *piv, *fail;
+  int nparts;
+  long ln;
+  size_t lds;  // of a step, at most
+};
+
+// Pivot steps j .. j + count - 1; an even count leaves the latest maxima in [0].
 template <int G>
-int qr_rounds(const double* phi, const double* occ, long n, int m, int mo, int k, double* d, double* L, double* pv,
-              int* pi, int* piv, double* rd, int* fail, Arena& ws, hipStream_t s) {
-  const int nparts = (int)((n + QB - 1) / QB);
-  const long ln = qr_ln(n);
+int qr_steps(const QrRun& q, int j, int count, hipStream_t s) {
+  if (q.lds > 64 * 1024)
+    THC_HIP(hipFuncSetAttribute((const void*)qr_step<G>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)q.lds));
+  for (int i = 0; i < count; ++i) {
+    const int in = i & 1;
+    hipLaunchKernelGGL(qr_step<G>, dim3((unsigned)q.nparts), dim3(QB), q.lds, s, q.phi, q.occ, q.n, q.m, q.mo, j + i,
+                       q.nparts, q.d, q.L, q.ln, q.pv[in], q.pi[in], q.pv[in ^ 1], q.pi[in ^ 1], q.piv, q.rd, q.fail);
+  }
+  THC_HIP(hipGetLastError());
+  return THC_OK;
+}
+
+// Rounds of pivots (real G) until k are chosen.
+template <int G>
+int qr_rounds(const QrRun& q, Arena& ws, hipStream_t s) {
+  const int k = q.k;
   double* LT = ws.take<double>((size_t)(k + 4) * QC);
   double* LP = ws.take<double>((size_t)(k + 4) * QR_MAX);
   double* S = ws.take<double>((size_t)QC * QC);
@@ -781,31 +813,52 @@ int qr_rounds(const double* phi, const double* occ, long n, int m, int mo, int k
   int* hist = ws.take<int>(QBINS);
   QrState* st = ws.take<QrState>(1);
   if (!LT || !LP || !S || !cand || !hist || !st) return THC_ERR_NO_MEMORY;
-  hipLaunchKernelGGL(qr_begin, dim3(1), dim3(QB), 0, s, pv, pi, nparts, st, hist);
-  hipLaunchKernelGGL(qr_hist, dim3(nparts), dim3(QB), 0, s, d, n, st, hist);
-  // Every round chooses a pivot or ends the run.  The host looks after up to
-  // eight rounds, fewer where the pivots left should take fewer (16 a round);
-  // rounds past the end return at once.
-  int h[3] = {0, 0, 0};  // j, fail, done
-  for (int rounds = 0; rounds <= k + 8 && !h[2];) {
-    const int batch = std::max(1, std::min(8, (k - h[0] + 15) / 16));
-    for (int q = 0; q < batch; ++q) {
-      hipLaunchKernelGGL(qr_pick, dim3(nparts), dim3(QB), 0, s, d, n, nparts, pv, pi, hist, st, cand);
-      hipLaunchKernelGGL(qr_gather, dim3(256), dim3(QC), 0, s, L, ln, st, cand, LT);
-      hipLaunchKernelGGL(qr_gram<G>, dim3((QC / 16) * (QC / 16)), dim3(256), 0, s, phi, occ, m, mo, st, cand, LT, S);
-      hipLaunchKernelGGL(qr_run, dim3(1), dim3(1024), 0, s, S, d, cand, k, st, hist, piv, rd);
+  auto begin = [&](int j) {
+    hipLaunchKernelGGL(qr_begin, dim3(1), dim3(QB), 0, s, q.pv[0], q.pi[0], q.nparts, j, k, q.fail, st, hist);
+    hipLaunchKernelGGL(qr_hist, dim3(q.nparts), dim3(QB), 0, s, q.d, q.n, st, hist);
+  };
+  begin(0);
+  // Every round chooses a pivot, ends the run or stalls.  The host looks after
+  // up to eight rounds, fewer where the pivots left should take fewer (16 a
+  // round) or a round stalled lately; rounds past an end or a stall return at
+  // once.
+  int h[3] = {0, 0, 0};  // j, done, stall
+  int steps = 4, most = 8;
+  while (!h[1]) {
+    const int batch = std::min(most, (k - h[0] + 15) / 16);
+    for (int b = 0; b < batch; ++b) {
+      hipLaunchKernelGGL(qr_pick, dim3(q.nparts), dim3(QB), 0, s, q.d, q.n, hist, st, cand);
+      hipLaunchKernelGGL(qr_gather, dim3(256), dim3(QC), 0, s, q.L, q.ln, st, cand, LT);
+      hipLaunchKernelGGL(qr_gram<G>, dim3((QC / 16) * (QC / 16)), dim3(256), 0, s, q.phi, q.occ, q.m, q.mo, st, cand, LT,
+                         S);
+      hipLaunchKernelGGL(qr_run, dim3(1), dim3(1024), 0, s, S, q.d, cand, k, st, hist, q.piv, q.rd, q.fail);
       hipLaunchKernelGGL(qr_compact, dim3(64), dim3(256), 0, s, st, LT, LP);
-      hipLaunchKernelGGL(qr_apply<G>, dim3(nparts), dim3(64 * QW), 0, s, phi, occ, n, m, mo, d, L, ln, LP, st, pv, pi,
-                         hist);
+      hipLaunchKernelGGL(qr_apply<G>, dim3(q.nparts), dim3(64 * QW), 0, s, q.phi, q.occ, q.n, q.m, q.mo, q.d, q.L, q.ln,
+                         LP, st, q.pv[0], q.pi[0], hist);
     }
-    rounds += batch;
     THC_HIP(hipGetLastError());
+    const int before = h[0];
     THC_HIP(hipMemcpyAsync(h, &st->j, sizeof(h), hipMemcpyDeviceToHost, s));
     THC_HIP(hipStreamSynchronize(s));
+    most = std::min(8, 2 * most);
+    if (h[0] > before) steps = std::max(4, steps / 2);
+    if (h[1] || !h[2]) continue;
+    const int count = std::min(steps, k - h[0]);
+    THC_TRY(qr_steps<G>(q, h[0], count, s));
+    h[0] += count;
+    begin(h[0]);
+    steps = std::min(32, 2 * steps);
+    most = 1;
   }
-  h[1] = h[2] ? h[1] : k + 1;
-  *fail = h[1];
   return THC_OK;
+}
+
+template <int G>
+int qr_run_all(const QrRun& q, bool by_steps, Arena& ws, hipStream_t s) {
+  if constexpr (G != G_COMPLEX)
+    if (!by_steps) return qr_rounds<G>(q, ws, s);
+  THC_HIP(hipMemsetAsync(q.fail, 0, sizeof(int), s));
+  return qr_steps<G>(q, 0, q.k, s);
 }
 
 }  // namespace
@@ -815,48 +868,45 @@ int qrcp_points(const double* phi, const double* occ, long n, int m, int mo, int
   const long nparts = (n + QB - 1) / QB;
   if (nparts > 0x7fffffffL) return THC_ERR_ARG;
   if (cplx && (m % 2 || (occ && mo % 2))) return THC_ERR_ARG;
-  const int mode = !cplx ? 0 : (occ ? 2 : 1);
-  double* d = ws.take<double>((size_t)n);
-  double* L = ws.take<double>((size_t)qr_ln(n) * k * (mode == 2 ? 2 : 1));
-  double* pv[2] = {ws.take<double>(nparts), ws.take<double>(nparts)};
-  int* pi[2] = {ws.take<int>(nparts), ws.take<int>(nparts)};
-  int* piv = ws.take<int>(k);
-  double* rd = ws.take<double>(k);
-  int* fail = ws.take<int>(1);
-  if (!d || !L || !pv[0] || !pv[1] || !pi[0] || !pi[1] || !piv || !rd || !fail) return THC_ERR_NO_MEMORY;
-  const size_t lds = sizeof(double) * ((size_t)m + (occ ? mo : 0) + (size_t)k * (mode == 2 ? 2 : 1));
-  if (lds > 160 * 1024) return THC_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(qr_init, dim3((unsigned)nparts), dim3(QB), 0, s, phi, occ, n, m, mo, d, pv[0], pi[0]);
+  const int g = cplx ? (occ ? G_COMPLEX : G_MODULUS) : (occ ? G_PRODUCT : G_SQUARE);
+  const int lw = g == G_COMPLEX ? 2 : 1;
+  QrRun q = {phi, occ, n, m, occ ? mo : 0, k};
+  q.nparts = (int)nparts;
+  q.ln = qr_ln(n);
+  q.d = ws.take<double>((size_t)n);
+  q.L = ws.take<double>((size_t)q.ln * k * lw);
+  for (int i = 0; i < 2; ++i) {
+    q.pv[i] = ws.take<double>(nparts);
+    q.pi[i] = ws.take<int>(nparts);
+  }
+  const size_t back = sizeof(double) * k + sizeof(int) * ((size_t)k + 1);
+  char* result = ws.take<char>(back);
+  q.rd = reinterpret_cast<double*>(result);
+  q.piv = reinterpret_cast<int*>(q.rd + k);
+  q.fail = q.piv + k;
+  if (!q.d || !q.L || !q.pv[0] || !q.pv[1] || !q.pi[0] || !q.pi[1] || !result) return THC_ERR_NO_MEMORY;
+  q.lds = sizeof(double) * ((size_t)m + q.mo + (size_t)k * lw);
+  if (q.lds > 160 * 1024) return THC_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(qr_init, dim3((unsigned)nparts), dim3(QB), 0, s, phi, occ, n, m, mo, q.d, q.pv[0], q.pi[0]);
   THC_HIP(hipGetLastError());
-  int h_fail = 0;
   // Few pivots of few real points: a step is 8 us there and a round of shared
   // pivots 75, of which six or seven are taken whatever k (27^3 points, k = 54:
   // 0.44 ms in steps, 0.47 in rounds; 32^3 points, k = 50: 0.44 and 0.53; but
   // 32^3 points, k = 67: 0.58 and 0.41; 48^3 points, k = 40: 0.67 and 0.33).
-  if (mode == 2 || (mode == 0 && k < 64 && n <= 40000)) {
-    const auto step = mode == 2 ? qr_step<true> : qr_step<false>;
-    if (lds > 64 * 1024)
-      THC_HIP(hipFuncSetAttribute((const void*)step, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    THC_HIP(hipMemsetAsync(fail, 0, sizeof(int), s));
-    for (int j = 0; j < k; ++j) {
-      const int in = j & 1;
-      hipLaunchKernelGGL(step, dim3((unsigned)nparts), dim3(QB), lds, s, phi, occ, n, m, mo, j, (int)nparts, d, L,
-                         pv[in], pi[in], pv[in ^ 1], pi[in ^ 1], piv, rd, fail);
-    }
-    THC_HIP(hipGetLastError());
-    THC_HIP(hipMemcpyAsync(&h_fail, fail, sizeof(int), hipMemcpyDeviceToHost, s));
-  } else if (mode == 1) {
-    THC_TRY(qr_rounds<G_MODULUS>(phi, nullptr, n, m, 0, k, d, L, pv[0], pi[0], piv, rd, &h_fail, ws, s));
-  } else if (occ) {
-    THC_TRY(qr_rounds<G_PRODUCT>(phi, occ, n, m, mo, k, d, L, pv[0], pi[0], piv, rd, &h_fail, ws, s));
-  } else {
-    THC_TRY(qr_rounds<G_SQUARE>(phi, nullptr, n, m, 0, k, d, L, pv[0], pi[0], piv, rd, &h_fail, ws, s));
+  const bool by_steps = !cplx && k < 64 && n <= 40000;
+  switch (g) {
+    case G_COMPLEX: THC_TRY(qr_run_all<G_COMPLEX>(q, true, ws, s)); break;
+    case G_MODULUS: THC_TRY(qr_run_all<G_MODULUS>(q, by_steps, ws, s)); break;
+    case G_PRODUCT: THC_TRY(qr_run_all<G_PRODUCT>(q, by_steps, ws, s)); break;
+    default: THC_TRY(qr_run_all<G_SQUARE>(q, by_steps, ws, s));
   }
-  std::vector<int> h(k);
-  THC_HIP(hipMemcpyAsync(h.data(), piv, sizeof(int) * k, hipMemcpyDeviceToHost, s));
-  if (rdiag_out) THC_HIP(hipMemcpyAsync(rdiag_out, rd, sizeof(double) * k, hipMemcpyDeviceToHost, s));
+  std::vector<double> host((back + sizeof(double) - 1) / sizeof(double));
+  THC_HIP(hipMemcpyAsync(host.data(), result, back, hipMemcpyDeviceToHost, s));
   THC_HIP(hipStreamSynchronize(s));
-  if (h_fail) return THC_ERR_NOT_POSDEF;
+  const int* hp = reinterpret_cast<const int*>(host.data() + k);
+  if (rdiag_out) std::copy(host.begin(), host.begin() + k, rdiag_out);
+  if (hp[k]) return THC_ERR_NOT_POSDEF;
+  std::vector<int> h(hp, hp + k);
   // the reference keeps the first K pivots in ascending grid order
   std::sort(h.begin(), h.end());
   THC_HIP(hipMemcpyAsync(piv_out, h.data(), sizeof(int) * k, hipMemcpyHostToDevice, s));
