@@ -144,3 +144,16 @@ def test_qrcp_equal_points_in_rounds(ctx, m, copies, alone, k, half, cplx):
     assert st == L.THC_OK
     np.testing.assert_array_equal(idx.cpu().numpy(), first[ref_idx])
     np.testing.assert_allclose(rd, ref_rd, rtol=1e-7)
+
+
+@pytest.mark.parametrize("n,m,k,cplx", [(40001, 4, 4, False), (40001, 4, 5, False), (120001, 4, 1, False),
+                                        (120001, 4, 2, False), (3000, 5, 8, True), (3000, 5, 9, True), (41000, 3, 4, True)])
+def test_qrcp_few_pivots(ctx, n, m, k, cplx):
+    """Either side of the point and pivot counts up to which a run goes one pivot a step."""
+    print("qrcp few pivots n=%d m=%d k=%d" % (n, m, k), flush=True)
+    a = (_complex_orbitals if cplx else _orbitals)(n, m, n + k)
+    st, idx, rd = (ctx.qrcp_points_complex if cplx else ctx.qrcp_points)(a, k)
+    assert st == L.THC_OK
+    ref_idx, ref_rd, _ = QO.qrcp_points(a, k)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ref_idx)
+    np.testing.assert_allclose(rd, ref_rd, rtol=1e-7)

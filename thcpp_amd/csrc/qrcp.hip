@@ -889,11 +889,16 @@ int qrcp_points(const double* phi, const double* occ, long n, int m, int mo, int
   if (q.lds > 160 * 1024) return THC_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(qr_init, dim3((unsigned)nparts), dim3(QB), 0, s, phi, occ, n, m, mo, q.d, q.pv[0], q.pi[0]);
   THC_HIP(hipGetLastError());
-  // Few pivots of few real points: a step is 8 us there and a round of shared
-  // pivots 75, of which six or seven are taken whatever k (27^3 points, k = 54:
-  // 0.44 ms in steps, 0.47 in rounds; 32^3 points, k = 50: 0.44 and 0.53; but
-  // 32^3 points, k = 67: 0.58 and 0.41; 48^3 points, k = 40: 0.67 and 0.33).
-  const bool by_steps = !cplx && k < 64 && n <= 40000;
+  // Few pivots: a step is 8 us on a small grid and a round of shared pivots 75,
+  // of which six or seven are taken whatever k (27^3 points, k = 54: 0.44 ms in
+  // steps, 0.47 in rounds; 32^3 points, k = 50: 0.44 and 0.53; but 32^3 points,
+  // k = 67: 0.58 and 0.41; 48^3 points, k = 40: 0.67 and 0.33).  Steps of complex
+  // orbitals cost more (24^3 points, M = 16: k = 8 0.14 both, k = 16 0.20 and
+  // 0.16).  Up to four pivots take less than what surrounds one round (48^3
+  // points, k = 2: 0.09 and 0.15; k = 4: 0.12 and 0.16; 64^3 points, M = 100,
+  // k = 1: 0.23 and 0.28, k = 2: 0.28 both).
+  const bool by_steps =
+      k == 1 || (k <= 4 && n <= 120000) || (n <= 40000 && k < (g == G_MODULUS ? 9 : 64));
   switch (g) {
     case G_COMPLEX: THC_TRY(qr_run_all<G_COMPLEX>(q, true, ws, s)); break;
     case G_MODULUS: THC_TRY(qr_run_all<G_MODULUS>(q, by_steps, ws, s)); break;
