@@ -360,3 +360,23 @@ def test_mixed_digits_of_short_lines(ctx, grid):
     ref = ctx.isdf(a, idx, grid, cg, precision=L.PREC_FP64, want_luv=False)["V"].cpu().numpy()
     got = ctx.isdf(a, idx, grid, cg, precision=L.PREC_MIXED, want_luv=False)["V"].cpu().numpy()
     assert rel(got, ref) < 1e-6
+
+
+@pytest.mark.parametrize("grid", [(1, 64, 64), (64, 1, 64), (64, 64, 1), (128, 128, 1), (1, 1, 128), (1, 128, 1), (128, 1, 1)])
+def test_fft_edges_of_one(ctx, grid):
+    """Transforms of a single point are a stage of their own in the kernels that read and store memory directly:
+    within the bound of test_fft_stage_classes, and their digits (V of the mixed path) within that of
+    test_mixed_digits_of_short_lines."""
+    from thcpp_amd import synthetic
+    rng = np.random.default_rng(sum(grid))
+    n = int(np.prod(grid))
+    x = rng.standard_normal((5, n))
+    cg = rng.random(n) + 0.5
+    got = ctx.fft_vectors(x, grid, cg).cpu().numpy()
+    assert rel(got, _half_spectrum_ref(x, grid, cg)) < 4e-15
+    a = rng.standard_normal((n, 6))
+    idx = np.sort(rng.choice(n, 6, replace=False)).astype(np.int32)
+    cg = synthetic.coulomb_kernel(5.0, grid)
+    ref = ctx.isdf(a, idx, grid, cg, precision=L.PREC_FP64, want_luv=False)["V"].cpu().numpy()
+    got = ctx.isdf(a, idx, grid, cg, precision=L.PREC_MIXED, want_luv=False)["V"].cpu().numpy()
+    assert rel(got, ref) < 1e-6

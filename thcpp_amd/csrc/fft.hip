@@ -88,7 +88,8 @@ struct Plan1D {
 constexpr unsigned fdiv_magic(int d) { return d > 1 ? 0xFFFFFFFFu / (unsigned)d + 1u : 0u; }
 
 // The plan of a length: radix 8, then 4, 2, 3, 5 (pl.n = 0 where it has another
-// factor).
+// factor); one stage of radix 1 for a single point, which is loaded and stored
+// like any other.
 constexpr Plan1D plan_of(int n) {
   Plan1D pl{};
   int m = n, ns = 1;
@@ -103,6 +104,10 @@ constexpr Plan1D plan_of(int n) {
       ns *= rs[i];
       m /= rs[i];
     }
+  if (n == 1) {
+    pl.nst = pl.rad[0] = pl.ns[0] = pl.tstep[0] = 1;
+    pl.mns[0] = fdiv_magic(1);
+  }
   pl.n = m == 1 ? n : 0;
   return pl;
 }
@@ -233,6 +238,7 @@ __device__ C2<T>* fft_lines(C2<T>* a, C2<T>* b, const Plan1D& pl, int nlines, in
   int ns = 1;
   for (int s = 0; s < pl.nst; ++s) {
     const int r = pl.rad[s];
+    if (r == 1) continue;  // one point: its own transform
     if (r == 8) stage<T, 8>(a, b, pl.n, ns, nlines, ls, tw);
     else if (r == 4) stage<T, 4>(a, b, pl.n, ns, nlines, ls, tw);
     else if (r == 2) stage<T, 2>(a, b, pl.n, ns, nlines, ls, tw);
@@ -291,14 +297,20 @@ __device__ __forceinline__ void stage_io(int n, int ns, FDiv fns, int tstep, int
 }
 
 // Stage s of a plan, f(radix, values), radix an integral constant: of the
-// run-time plan, or (N > 0) of the plan of length N with s = S.
-template <int N, int S, class F>
+// run-time plan (radix 1 only if it is the plan's ONLY stage), or (N > 0) of the
+// plan of length N with s = S.
+template <int N, int S, bool ONLY, class F>
 __device__ __forceinline__ void with_radix(const Plan1D& pl, int s, F f) {
   if constexpr (N > 0) {
     constexpr Plan1D cp = plan_of(N);
     f(std::integral_constant<int, cp.rad[S]>{}, cp.ns[S], FDiv(cp.ns[S]), cp.tstep[S]);
   } else {
     const FDiv fns(pl.ns[s], pl.mns[s]);
+    if constexpr (ONLY)
+      if (pl.rad[s] == 1) {
+        f(std::integral_constant<int, 1>{}, 1, fns, 1);
+        return;
+      }
     switch (pl.rad[s]) {
       case 8: f(std::integral_constant<int, 8>{}, pl.ns[s], fns, pl.tstep[s]); break;
       case 4: f(std::integral_constant<int, 4>{}, pl.ns[s], fns, pl.tstep[s]); break;
@@ -322,8 +334,8 @@ __device__ __forceinline__ void fft_lines_io(C2<T>* buf, const Plan1D& pl, int n
   auto wr = [&](int, int, int line, int pos, C2<T> y) { buf[swz(line, pos, ls)] = y; };
   auto one = [&](auto first_stage, auto last_stage, auto st, int s) {
     constexpr bool F = decltype(first_stage)::value, L = decltype(last_stage)::value && !TOBUF;
-    with_radix<N, decltype(st)::value>(pl, s, [&](auto r, int ns, FDiv fns, int tstep) {
-      constexpr int R = decltype(r)::value, NB = IPV / R > 0 ? IPV / R : 1;
+    with_radix<N, decltype(st)::value, F && decltype(last_stage)::value>(pl, s, [&](auto r, int ns, FDiv fns, int tstep) {
+      constexpr int R = decltype(r)::value, NB = R > 1 && IPV / R > 0 ? IPV / R : 1;  // at most FT lines of one point
       constexpr bool LF = !F || LF1;
       const FDiv fw = LF ? fl : FDiv(n / R);
       if constexpr (F && L) stage_io<T, R, NB, LF, false>(n, ns, fns, tstep, nlines, fw, tw, first, last);
@@ -354,7 +366,6 @@ __device__ __forceinline__ void fft_lines_io(C2<T>* buf, const Plan1D& pl, int n
 
 // Whether every stage of a plan over nlines lines keeps to ipv values per thread.
 bool fits_ip(const Plan1D& pl, int nlines, int ipv) {
-  if (pl.nst == 0) return false;  // one point: no stage to load or store through
   for (int s = 0; s < pl.nst; ++s) {
     const int r = pl.rad[s];
     const long per = ((long)nlines * (pl.n / r) + FT - 1) / FT;
