@@ -29,9 +29,10 @@ HOST_HEADERS = ["h5io.h", "json.h", "thcpp.h"]
 HOST_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-I/opt/rocm/include", "-D__HIP_PLATFORM_AMD__",
               "-I" + os.path.join(ROOT, "include")]
 
-HIP_SOURCES = ["kmeans.hip", "gemm.hip", "linalg.hip", "fft.hip", "ozaki.hip", "qrcp.hip", "api.hip"]
+HIP_SOURCES = ["fft_f32.hip", "fft.hip", "gemm.hip", "kmeans.hip", "linalg.hip", "ozaki.hip", "qrcp.hip", "api.hip"]
 CXX_SOURCES = ["seed.cpp"]
 HEADERS = ["common.h", "kmeans.h"]
+INCLUDED = {"fft_f32.hip": ["fft.hip"]}  # sources that a source includes
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
@@ -45,7 +46,8 @@ def _stale(src: str, obj: str) -> bool:
     if not os.path.exists(obj):
         return True
     t = os.path.getmtime(obj)
-    deps = [src] + [os.path.join(CSRC, h) for h in HEADERS] + [os.path.join(ROOT, "include", "thcpp_amd.h")]
+    local = HEADERS + INCLUDED.get(os.path.basename(src), [])
+    deps = [src] + [os.path.join(CSRC, h) for h in local] + [os.path.join(ROOT, "include", "thcpp_amd.h")]
     return any(os.path.getmtime(d) > t for d in deps)
 
 

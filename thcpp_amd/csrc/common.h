@@ -238,6 +238,9 @@ size_t fft_work_bytes(int k, const int n[3], int prec);
 // passes and after the second
 int fft_coulomb(const void* x, int x_f32, int k, const int n[3], const double* coulG, void* out, int prec,
                 void* work, hipStream_t s, hipEvent_t* pass_ev = nullptr, const FftDigits* dig = nullptr);
+// Its FP32 part (fft_f32.hip).
+int fft_coulomb_f32(const void* x, int x_f32, int k, const int n[3], const double* coulG, void* out, void* work,
+                    hipStream_t s, hipEvent_t* pass_ev, const FftDigits* dig);
 inline long half_spectrum_len(const int n[3]) { return 2L * n[0] * n[1] * (n[2] / 2 + 1); }
 
 }  // namespace thc

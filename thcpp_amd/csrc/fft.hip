@@ -759,6 +759,16 @@ int run(const X* x, int k, const int n[3], const double* coulG, void* out, void*
 
 }  // namespace
 
+#ifdef THC_FFT_F32  // fft_f32.hip
+
+int fft_coulomb_f32(const void* x, int x_f32, int k, const int n[3], const double* coulG, void* out, void* work,
+                    hipStream_t s, hipEvent_t* pass_ev, const FftDigits* dig) {
+  if (x_f32) return run<float>(reinterpret_cast<const float*>(x), k, n, coulG, out, work, s, pass_ev, dig);
+  return run<float>(reinterpret_cast<const double*>(x), k, n, coulG, out, work, s, pass_ev, dig);
+}
+
+#else
+
 size_t fft_work_bytes(int k, const int n[3], int prec) {
   const size_t es = prec == 0 ? sizeof(double) : sizeof(float);
   const size_t tb = align_up(es * 2 * MAXN, 256);
@@ -776,8 +786,9 @@ int fft_coulomb(const void* x, int x_f32, int k, const int n[3], const double* c
     if (dig) return THC_ERR_ARG;
     return run<double>(reinterpret_cast<const double*>(x), k, n, coulG, out, work, s, pass_ev, nullptr);
   }
-  if (x_f32) return run<float>(reinterpret_cast<const float*>(x), k, n, coulG, out, work, s, pass_ev, dig);
-  return run<float>(reinterpret_cast<const double*>(x), k, n, coulG, out, work, s, pass_ev, dig);
+  return fft_coulomb_f32(x, x_f32, k, n, coulG, out, work, s, pass_ev, dig);
 }
+
+#endif
 
 }  // namespace thc

@@ -1654,7 +1654,7 @@ int kmeans_run_many(thc_ctx* ctx, int nj, const KmSpec* spec, int* status, thc_k
     Job& J = hj[t];
     J.L = lay[j];
     if (!carve(ctx->kmws, J.L, J.b, true)) return THC_ERR_NO_MEMORY;
-    J.b.idx0 = didx + ipos;  // read by init_centroids only
+    J.b.idx0 = didx + ipos;  // read by init_run only
     std::copy(init[j].begin(), init[j].end(), hidx + ipos);
     ipos += spec[j].k;
     J.grid = spec[j].grid;
