@@ -375,6 +375,16 @@ def _windows_map(case):
             gmap[65536 * w + np.concatenate([[0, 65535], 1 + rng.choice(65534, m - 2, replace=False)])] = 0
         gmap[3 * 65536:4 * 65536][gmap[3 * 65536:4 * 65536] == 0] = 1
         return n, 10, gmap
+    if case == "near":  # up to 1024 members in one to nine windows of the register path, some empty, ends on both sides
+        n = 10 * 65536
+        gmap = np.full(n, 7, dtype=np.int32)
+        for c, lo, hi, m in ((0, 64, 64 + 8 * 65536 - 1, 1024), (1, 96, 96 + 8 * 65536, 1024), (2, 65535, 65536, 2),
+                             (3, 65537, 3 * 65536, 700), (4, 40, 40 + 65535, 1023), (5, 41, 41 + 65536, 1023)):
+            inner = np.setdiff1d(np.concatenate([lo + 1 + np.arange(640), hi - 1 - np.arange(640)]),
+                                 np.flatnonzero(gmap != 7)) if hi - lo > 2000 else np.empty(0, dtype=np.int64)
+            gmap[np.concatenate([[lo, hi], rng.permutation(inner)[:m - 2]])] = c
+        gmap[200000] = 6
+        return n, 8, gmap
     if case == "shared":  # six clusters beyond their buckets (8 n / k members) share the list
         n, k = 150000, 900
         gmap = rng.integers(0, 6, n).astype(np.int32) * 150
@@ -387,7 +397,7 @@ def _windows_map(case):
     return n, 3, gmap
 
 
-@pytest.mark.parametrize("case", ["dense", "runs", "shared", "far"])
+@pytest.mark.parametrize("case", ["dense", "runs", "near", "shared", "far"])
 def test_update_centroids_windows(ctx, case):
     n, k, gmap = _windows_map(case)
     rng = np.random.default_rng(n)

@@ -683,8 +683,9 @@ __global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k,
 // less on a 64^3 grid), a scan of the words' bit counts gives every member its
 // rank, the values go to LDS by rank, and lanes 0..3 run the four sequential
 // sums.  Up to SB_R members a thread stay in registers, their values on the
-// way while the bits are counted.  Larger clusters, and index ranges wider than
-// the window, are partitioned by window first (in 'seg', of which every such
+// way while the bits are counted, for up to SB_NEAR windows one after the other
+// (a cluster of 256 points on a 96^3 grid may take two).  Larger clusters, and
+// wider index ranges, are partitioned by window first (in 'seg', of which every such
 // cluster takes as many entries as it has members), so that each member is set
 // as a bit once, whatever the range; wave 0 then adds a run of members while
 // the other waves look up the next run by rank.
@@ -695,6 +696,7 @@ __global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k,
 constexpr int SB_W = 2048;  // words of the window
 constexpr int SB_M = 512;   // members summed at a time
 constexpr int SB_R = 4;     // members a thread of the register path
+constexpr int SB_NEAR = 8;  // windows of the register path
 constexpr int SB_H = SB_M / 2;  // members of a run of the partitioned path
 constexpr int SB_BINS = 512;    // windows partitioned at a time
 static_assert(SB_W * 32 == 1 << 16, "window of an index: its bits from 16 on");
@@ -722,9 +724,9 @@ __device__ inline void sums_scan(SumsLds& S, int v, int& before, int& total) {
   }
 }
 
-// pre of this thread's words wb .. we - 1 of the window; a barrier inside, none
-// at the end.
-__device__ inline void sums_rank(SumsLds& S, int wb, int we) {
+// pre of this thread's words wb .. we - 1 of the window; the window's members.
+// A barrier inside, none at the end.
+__device__ inline int sums_rank(SumsLds& S, int wb, int we) {
   int have = 0, pos, total;
   for (int w = wb; w < we; ++w) have += __popc(S.bm[w]);
   sums_scan(S, have, pos, total);
@@ -732,6 +734,7 @@ __device__ inline void sums_rank(SumsLds& S, int wb, int we) {
     S.pre[w] = (unsigned short)pos;
     pos += __popc(S.bm[w]);
   }
+  return total;
 }
 
 // Member of rank r of the window, as an offset into it.
@@ -826,28 +829,40 @@ __device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int
   lo = min(min(S.red[0], S.red[1]), min(S.red[2], S.red[3])) & ~31;
   hi = -min(min(S.red2[0], S.red2[1]), min(S.red2[2], S.red2[3]));
   double acc = 0.0;  // lane q < 4 of wave 0 owns accumulator q
-  if (few && m > 0 && hi - lo < SB_W * 32) {
-    const int per = ((hi - lo) >> 13) + 1, wb = tid * per;  // words a thread, all inside the window
+  if (few && m > 0 && hi - lo < SB_NEAR * (SB_W * 32)) {
+    for (long w0 = lo; w0 <= hi; w0 += SB_W * 32) {
+      if (w0 > lo) {
+        __syncthreads();
+        for (int w = tid; w < SB_W; w += 256) S.bm[w] = 0;
+        __syncthreads();
+      }
+      const int last = (int)min((long)SB_W * 32 - 1, hi - w0);
+      const int per = (last >> 13) + 1, wb = tid * per;  // words a thread, all inside the window
 #pragma unroll
-    for (int u = 0; u < SB_R; ++u)
-      if (tid + 256 * u < m) atomicOr(&S.bm[(i[u] - lo) >> 5], 1u << (i[u] & 31));
-    __syncthreads();
-    sums_rank(S, wb, wb + per);
-    __syncthreads();
-    for (int base = 0; base < m; base += SB_M) {
+      for (int u = 0; u < SB_R; ++u) {
+        const unsigned at = (unsigned)(i[u] - w0);
+        if (tid + 256 * u < m && at < SB_W * 32) atomicOr(&S.bm[at >> 5], 1u << (i[u] & 31));
+      }
+      __syncthreads();
+      const int here = sums_rank(S, wb, wb + per);
+      __syncthreads();
+      for (int base = 0; base < here; base += SB_M) {
 #pragma unroll
-      for (int u = 0; u < SB_R; ++u)
-        if (tid + 256 * u < m) {
-          const int w = (i[u] - lo) >> 5;
-          const int r = S.pre[w] + __popc(S.bm[w] & ((1u << (i[u] & 31)) - 1)) - base;
-          if (r >= 0 && r < SB_M) {
-            S.buf[0][r] = v[u][0];
-            for (int d = 0; d < 3; ++d) S.buf[1 + d][r] = v[u][0] * v[u][1 + d];
+        for (int u = 0; u < SB_R; ++u) {
+          const unsigned at = (unsigned)(i[u] - w0);
+          if (tid + 256 * u < m && at < SB_W * 32) {
+            const int w = at >> 5;
+            const int r = S.pre[w] + __popc(S.bm[w] & ((1u << (i[u] & 31)) - 1)) - base;
+            if (r >= 0 && r < SB_M) {
+              S.buf[0][r] = v[u][0];
+              for (int d = 0; d < 3; ++d) S.buf[1 + d][r] = v[u][0] * v[u][1 + d];
+            }
           }
         }
-      __syncthreads();
-      if (tid < 4) acc = seq_sum(acc, S.buf[tid], min(SB_M, m - base));
-      if (base + SB_M < m) __syncthreads();
+        __syncthreads();
+        if (tid < 4) acc = seq_sum(acc, S.buf[tid], min(SB_M, here - base));
+        if (base + SB_M < here) __syncthreads();
+      }
     }
   } else if (m > 0) {
     // every member: f(grid index), eight loads in flight
