@@ -11,9 +11,8 @@ system: ZC^T (N x N_mu x M, rows of Phi gathered, square epilogue) and the
 FP64 solve (N_mu x N x N_mu).  Shapes are grouped by (ceil log2 m, n, k) and
 kind; each group gets the configuration with the least summed time.
 
-A GEMM alone is not the whole story (the ZC^T GEMM of a large grid keeps one
-workgroup per CU so that the Cholesky of CC^T on the second stream finds free
-CUs), so each candidate entry is then validated end to end, largest measured
+A GEMM alone is not the whole story (the Cholesky of CC^T on the second stream
+runs beside the ZC^T GEMM), so each candidate entry is then validated end to end, largest measured
 gain first: the workloads with shapes in its bucket are timed (mixed and FP64
 factorisations, or the batched call) with the entries kept so far, with and
 without it, and it is kept only if they got faster.
