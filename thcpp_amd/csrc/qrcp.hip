@@ -496,8 +496,10 @@ __global__ __launch_bounds__(256) void qr_compact(const QrState* st, const doubl
 // acc[s][a] = sum_q L[q][p_s] L[q][a] by MFMA (A: the pivots' entries from LP,
 // B: 32 points a wave, two interleaved 16-point fragments from one 16-byte
 // load), G the same way from the orbitals, then the triangular solve with one
-// lane a point.  Loads of QU steps are in flight while the previous QU are
-// multiplied.  Bound by the read of L, 8 j N bytes a round, and by latency: two
+// lane a point.  Even and odd steps of four are summed apart: with one chain
+// |R_jj| was 2.5e-14 from the exact values on 40^3, K = 512, with two 2.1e-14 (one
+// kernel per pivot: 2.0e-14).  Loads of QU steps are in
+// flight while the previous QU are multiplied.  Bound by the read of L, 8 j N bytes a round, and by latency: two
 // waves a SIMD at N = 64000, 3.4 TB/s.
 constexpr int QU = 8;
 constexpr int QW = QB / 32;  // waves of a workgroup: 32 points each, QB together
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(64 * QW) void qr_apply(const double* __restrict__ p
   const int r = st->r, j = st->base;
   const bool two = r > 16;
   const long a0 = (long)blockIdx.x * QB + 32 * w;
-  qd4 acc[2][2] = {}, p1[2][2] = {}, p2[2][2] = {};
+  qd4 acc[2][2] = {}, odd[2][2] = {}, p1[2][2] = {}, p2[2][2] = {};
   {
     // rows are ln >= the workgroups' points apart, so every load is inside L
     const double2* lb = reinterpret_cast<const double2*>(L + (long)l4 * ln + a0 + 2 * l16);
@@ -536,11 +538,12 @@ __global__ __launch_bounds__(64 * QW) void qr_apply(const double* __restrict__ p
         }
       };
       auto mul = [&](int buf, int u) {
-        acc[0][0] = qr_mfma(u0[buf][u], b[buf][u].x, acc[0][0]);
-        acc[0][1] = qr_mfma(u0[buf][u], b[buf][u].y, acc[0][1]);
+        auto& s = u & 1 ? odd : acc;
+        s[0][0] = qr_mfma(u0[buf][u], b[buf][u].x, s[0][0]);
+        s[0][1] = qr_mfma(u0[buf][u], b[buf][u].y, s[0][1]);
         if (both.value) {
-          acc[1][0] = qr_mfma(u1[buf][u], b[buf][u].x, acc[1][0]);
-          acc[1][1] = qr_mfma(u1[buf][u], b[buf][u].y, acc[1][1]);
+          s[1][0] = qr_mfma(u1[buf][u], b[buf][u].x, s[1][0]);
+          s[1][1] = qr_mfma(u1[buf][u], b[buf][u].y, s[1][1]);
         }
       };
       load(0, 0);
@@ -572,39 +575,51 @@ __global__ __launch_bounds__(64 * QW) void qr_apply(const double* __restrict__ p
       acc[1][1] = qr_mfma(v1, x.y, acc[1][1]);
     }
   }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      acc[i][f] += odd[i][f];
+      odd[i][f] = qd4{};
+    }
   {
     const long ra = min(a0 + 2 * l16, n - 1), rb = min(a0 + 2 * l16 + 1, n - 1);
     const long q0 = st->piv[min(l16, r - 1)], q1 = st->piv[min(16 + l16, r - 1)];
-    for (int k0 = 0; k0 < m; k0 += 4) {
-      const int k = k0 + l4;
-      const bool ok = k < m;
-      const double x = ok ? phi[ra * m + k] : 0.0, y = ok ? phi[rb * m + k] : 0.0;
-      const double u = ok ? phi[q0 * m + k] : 0.0, v = ok ? phi[q1 * m + k] : 0.0;
-      p1[0][0] = qr_mfma(u, x, p1[0][0]);
-      p1[0][1] = qr_mfma(u, y, p1[0][1]);
+    qd4 odd2[2][2] = {};
+    auto four = [&](const double* __restrict__ rows, int width, int k, qd4(&s)[2][2], qd4(&si)[2][2]) {
+      const bool ok = k < width;
+      const double x = ok ? rows[ra * width + k] : 0.0, y = ok ? rows[rb * width + k] : 0.0;
+      const double u = ok ? rows[q0 * width + k] : 0.0, v = ok ? rows[q1 * width + k] : 0.0;
+      s[0][0] = qr_mfma(u, x, s[0][0]);
+      s[0][1] = qr_mfma(u, y, s[0][1]);
       if (two) {
-        p1[1][0] = qr_mfma(v, x, p1[1][0]);
-        p1[1][1] = qr_mfma(v, y, p1[1][1]);
+        s[1][0] = qr_mfma(v, x, s[1][0]);
+        s[1][1] = qr_mfma(v, y, s[1][1]);
       }
       if (G == G_MODULUS) {
-        const double u2 = ok ? qr_times_i(phi, q0, m, k) : 0.0;
-        const double v2 = ok ? qr_times_i(phi, q1, m, k) : 0.0;
-        p2[0][0] = qr_mfma(u2, x, p2[0][0]);
-        p2[0][1] = qr_mfma(u2, y, p2[0][1]);
-        p2[1][0] = qr_mfma(v2, x, p2[1][0]);
-        p2[1][1] = qr_mfma(v2, y, p2[1][1]);
+        const double u2 = ok ? qr_times_i(rows, q0, width, k) : 0.0;
+        const double v2 = ok ? qr_times_i(rows, q1, width, k) : 0.0;
+        si[0][0] = qr_mfma(u2, x, si[0][0]);
+        si[0][1] = qr_mfma(u2, y, si[0][1]);
+        si[1][0] = qr_mfma(v2, x, si[1][0]);
+        si[1][1] = qr_mfma(v2, y, si[1][1]);
       }
+    };
+    for (int k0 = l4; k0 < m + l4; k0 += 8) {
+      four(phi, m, k0, p1, p2);
+      four(phi, m, k0 + 4, odd, odd2);
     }
     if (G == G_PRODUCT)
-      for (int k0 = 0; k0 < mo; k0 += 4) {
-        const int k = k0 + l4;
-        const bool ok = k < mo;
-        const double x = ok ? occ[ra * mo + k] : 0.0, y = ok ? occ[rb * mo + k] : 0.0;
-        const double u = ok ? occ[q0 * mo + k] : 0.0, v = ok ? occ[q1 * mo + k] : 0.0;
-        p2[0][0] = qr_mfma(u, x, p2[0][0]);
-        p2[0][1] = qr_mfma(u, y, p2[0][1]);
-        p2[1][0] = qr_mfma(v, x, p2[1][0]);
-        p2[1][1] = qr_mfma(v, y, p2[1][1]);
+      for (int k0 = l4; k0 < mo + l4; k0 += 8) {
+        four(occ, mo, k0, p2, p2);
+        four(occ, mo, k0 + 4, odd2, odd2);
+      }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        p1[i][f] += odd[i][f];
+        p2[i][f] += odd2[i][f];
       }
   }
 #pragma unroll
