@@ -645,8 +645,8 @@ __global__ __launch_bounds__(256) void assign(const double* sx, const double* sy
 // st->error: a key outside [0, k).  The points of a cluster are counted in LDS
 // and take their places with one device atomic per tile and cluster: with one
 // per point, 4096 points to each of 64 addresses queued for 1.3 ms (64^3, K 64).
-__global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k, int* cnt, int* bucket, int cap, int2* over,
-                                                  int* ctr, State* st) {
+__global__ __launch_bounds__(256) void bucket_map(const int* map, long n, int k, int* cnt, int* bucket, int cap,
+                                                  int2* over, int* ctr, State* st) {
   __shared__ int h[MAXB];
   constexpr int PT = CS_TILE / 256;
   const long i0 = blockIdx.x * (long)CS_TILE + threadIdx.x;
@@ -796,8 +796,8 @@ __device__ inline double sums_window(SumsLds& S, double acc, int w0, const int* 
   return acc;
 }
 
-__device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int cap, const int2* over, int* ctr, int* seg,
-                                                     long n, const double* rho, const double* grid, double* cen_out,
+__device__ __forceinline__ void centroid_sums_b(int* cnt, const int* bucket, int cap, const int2* over, int* ctr,
+                                                     int* seg, long n, const double* rho, const double* grid, double* cen_out,
                                                      State* st, int it, int seen, int c) {
   __shared__ SumsLds S;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1794,8 +1794,8 @@ int kmeans_update(thc_ctx* ctx, const double* rho, const double* grid, long n, c
                      cnt, ctr, (int*)nullptr, 0, st);
   hipLaunchKernelGGL(bucket_map, dim3(ceil_div(n, CS_TILE)), dim3(256), 0, s, grid_map, n, k, cnt, bucket, cap, over,
                      ctr, st);
-  hipLaunchKernelGGL(centroid_sums, dim3(k), dim3(256), 0, s, cnt, bucket, cap, over, ctr, seg, n, rho, grid, centroids, st,
-                     0, -1);
+  hipLaunchKernelGGL(centroid_sums, dim3(k), dim3(256), 0, s, cnt, bucket, cap, over, ctr, seg, n, rho, grid, centroids,
+                     st, 0, -1);
   THC_HIP(hipGetLastError());
   State hst;
   THC_HIP(hipMemcpyAsync(&hst, st, sizeof(State), hipMemcpyDeviceToHost, s));

@@ -498,9 +498,9 @@ __global__ __launch_bounds__(256) void qr_compact(const QrState* st, const doubl
 // load), G the same way from the orbitals, then the triangular solve with one
 // lane a point.  Even and odd steps of four are summed apart: with one chain
 // |R_jj| was 2.5e-14 from the exact values on 40^3, K = 512, with two 2.1e-14 (one
-// kernel per pivot: 2.0e-14).  Loads of QU steps are in
-// flight while the previous QU are multiplied.  Bound by the read of L, 8 j N bytes a round, and by latency: two
-// waves a SIMD at N = 64000, 3.4 TB/s.
+// kernel per pivot: 2.0e-14).  Loads of QU steps are in flight while the previous
+// QU are multiplied.  Bound by the read of L, 8 j N bytes a round, and by
+// latency: two waves a SIMD at N = 64000, 3.4 TB/s.
 constexpr int QU = 8;
 constexpr int QW = QB / 32;  // waves of a workgroup: 32 points each, QB together
 
